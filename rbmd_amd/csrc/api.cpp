@@ -139,10 +139,11 @@ struct rbmd_ctx {
 };
 
 // producers of thermo partial rows (row widths kRowPair, kRowK, kRowBond, kRowKe, kRowShake)
-enum { SEG_PAIR, SEG_K, SEG_BOND, SEG_KE, SEG_SHAKE, NSEG };
-constexpr int kSegWidth[NSEG] = {kRowPair, kRowK, kRowBond, kRowKe, kRowShake};
-constexpr int kSegSlot0[NSEG] = {S_ELJ, S_VIR_K, S_VIR_BOND, S_KE, S_VIR_SHAKE};
-constexpr int kSegGroups[NSEG] = {64, 16, 16, 64, 16};  // 992 reduction threads in all
+enum { SEG_PAIR, SEG_K, SEG_BOND, SEG_SHAKE, SEG_KE, NSEG };
+constexpr int kSegWidth[NSEG] = {kRowPair, kRowK, kRowBond, kRowShake, kRowKe};
+constexpr int kSegSlot0[NSEG] = {S_ELJ, S_VIR_K, S_VIR_BOND, S_VIR_SHAKE, S_KE};
+// 928 reduction threads in all (64 x 8, 16 x 6, 16 x 14, 16 x 6); every thread strides the kinetic energy's rows
+constexpr int kSegGroups[NSEG] = {64, 16, 16, 16, 1};
 
 struct rbmd_sys {
   rbmd_ctx* ctx = nullptr;
@@ -176,6 +177,7 @@ struct rbmd_sys {
   // captured MD steps (rbmd_md_run_graph): [0] without, [1] with the thermo sums
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   bool graph_ok = false;           // cleared whenever captured pointers or sizes change
+  bool scale_pending = false;      // within an eager call: the last step's velocity scale runs with the next step's start
   bool rattle_pending = false;     // within an eager call: the last step's RATTLE runs with the next step's start
   double* kring = nullptr; // [2R][3P]
   double* stage[2] = {nullptr, nullptr};
@@ -272,6 +274,12 @@ void rbl_capacity(const rbmd_params& p, int n, double volume, int* rs_num, int* 
   // overwrites past rs_num silently, hazard Q7); pice_num keeps its formula
   *rs_num = (int)(2 * rsn + 32);
 }
+
+// the k-space tile choices a system's parameters name
+int k_lanes_lg_of(const rbmd_params& p) {
+  return p.kforce_lanes ? (p.kforce_lanes == 2 ? 1 : (p.kforce_lanes == 8 ? 3 : 2)) : 2;
+}
+int rho_kb_of(const rbmd_params& p) { return p.rho_kblock ? p.rho_kblock : 1; }
 
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
@@ -525,15 +533,20 @@ rbmd_status ensure_rho(rbmd_sys* s, int P) {
 // ExecutionNVT.cpp:195-235).  kvec: device pointer to this step's k vectors.
 // k-space and bonded forces on stream st (they read the unsorted positions
 // and charges only, and write their own force arrays and thermo rows)
+static KView step_kview(const rbmd_sys* s, const double* kvec) {
+  KView k = s->kv;
+  k.P = s->P;
+  k.kvec = kvec;
+  k.S_over_P = s->p.coulomb_type == RBMD_COULOMB_RBE ? s->S / (double)s->P : 1.0;
+  k.f32 = s->v.mixed;
+  k.ewald = s->p.coulomb_type == RBMD_COULOMB_EWALD;
+  return k;
+}
+
 static void launch_k_bonded(rbmd_sys* s, const double* kvec, int thermo, hipStream_t st) {
   rbmd_ctx* c = s->ctx;
   if (has_k(s)) {
-    KView k = s->kv;
-    k.P = s->P;
-    k.kvec = kvec;
-    k.S_over_P = s->p.coulomb_type == RBMD_COULOMB_RBE ? s->S / (double)s->P : 1.0;
-    k.f32 = s->v.mixed;
-    k.ewald = s->p.coulomb_type == RBMD_COULOMB_EWALD;
+    const KView k = step_kview(s, kvec);
     c->run("rho_partial", [&] { launch_rho_partial(s->v, k, st); });
     c->run("rho_reduce", [&] { launch_rho_reduce(s->v, k, st); });
     int nblk = 0;
@@ -894,6 +907,23 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   v.n_items = v.ncell + n / kChunk + 1;
   v.lds_bins = v.ncell <= 4096 ? 1 : 0;
   v.list_cut2 = v.cut2;
+  // the list predicate as one threshold: cut2 - d2 rounded falls as d2 grows
+  v.accept_d2 = v.cut2 - 0.0001;
+  while (!(v.cut2 - v.accept_d2 > 0.0001)) v.accept_d2 = std::nextafter(v.accept_d2, 0.0);
+  while (v.cut2 - std::nextafter(v.accept_d2, v.cut2) > 0.0001) v.accept_d2 = std::nextafter(v.accept_d2, v.cut2);
+  // The error of the stencil kernel's FP32 d^2 near the cutoff: pairs within it
+  // of a threshold are decided in FP64.  Coordinates from the box corner, less the image shift and the
+  // cell's centre, carry at most u (3 L + 5 w) (u = 2^-24, w the cell width,
+  // at least rc); for a pair within rc of an atom of the cell |a| <= 0.87 w
+  // and |c| <= 1.87 w, so |c|^2 - 2 c.a + |a|^2 rounds by at most 45 u w^2,
+  // and the coordinates move d^2 by at most 7 u rc (3 L + 5 w).  Twice that.
+  {
+    const double L = std::max(v.box[0], std::max(v.box[1], v.box[2]));
+    const double wd = std::max(v.dxdydz[0], std::max(v.dxdydz[1], v.dxdydz[2]));
+    const double band = std::ldexp(45.0 * wd * wd + 7.0 * v.cut * (3.0 * L + 5.0 * wd), -23);
+    v.test_band = std::nextafter((float)band, 3e38f);
+    for (int k = 0; k < 3; ++k) v.shift32[k] = (float)v.shift_len[k];
+  }
   s->g_ref = rbmd_sys::Geom{{v.dims[0], v.dims[1], v.dims[2]}, {v.dxdydz[0], v.dxdydz[1], v.dxdydz[2]},
                             v.ncell, v.n_items, v.lds_bins, v.cut2};
   s->g_skin = s->g_ref;
@@ -929,9 +959,13 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   // lanes per atom in the pair kernel: enough threads to fill 256 CUs for
   // small systems, fewer lanes (longer per-lane loops) for large ones
   v.lanes_lg = n <= 60000 ? 4 : (n <= 250000 ? 3 : 2);
+  v.compact = !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes && stencil_pays(v) ? 1 : 0;
+  v.st_cfg = stencil_choice(v);
   if (p->pair_lanes) v.lanes_lg = p->pair_lanes == 4 ? 2 : (p->pair_lanes == 8 ? 3 : 4);
-  v.k_lanes_lg = p->kforce_lanes ? (p->kforce_lanes == 2 ? 1 : (p->kforce_lanes == 8 ? 3 : 2)) : 2;
-  v.rho_kb = p->rho_kblock ? p->rho_kblock : 1;
+  if (v.compact) v.lanes_lg = 4;  // as the stencil kernel sums
+  v.k_lanes_lg = k_lanes_lg_of(*p);
+  v.rho_kb = rho_kb_of(*p);
+  if (v.compact) v.k_lanes_lg = 4;  // the latency counts: 16 wavefronts over the k range
   v.sp_max = 0;
   if (d->special_offsets && d->special_ids && d->special_weights)
     for (int i = 0; i < n; ++i) v.sp_max = std::max(v.sp_max, d->special_offsets[i + 1] - d->special_offsets[i]);
@@ -1008,6 +1042,27 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   A(s->dalloc(&v.misfit_list, n));
   A(s->dalloc(&v.misfit_count, 1));
   A(s->dalloc(&v.spos, n));
+  if (v.compact) {
+    A(s->dalloc(&v.spos32, n));
+    // stencil cells of every cell, x offset outermost, then y, then z: the
+    // wrapped cell and the image shift + 2 per axis (2 bits each)
+    std::vector<int> tab((size_t)v.ncell * 32, -1);
+    for (int c = 0; c < v.ncell; ++c)
+      for (int k = 0; k < 27; ++k) {
+        int at[3] = {c % v.dims[0] + k / 9 - 1, (c / v.dims[0]) % v.dims[1] + (k / 3) % 3 - 1,
+                     c / (v.dims[0] * v.dims[1]) + k % 3 - 1};
+        int code = 0;
+        for (int d = 0; d < 3; ++d) {
+          const int w = (at[d] + v.dims[d]) % v.dims[d];
+          code |= ((w - at[d]) / v.dims[d] + 2) << (2 * d);
+          at[d] = w;
+        }
+        tab[(size_t)c * 32 + k] = (at[0] + at[1] * v.dims[0] + at[2] * v.dims[0] * v.dims[1]) << 6 | code;
+      }
+    int* dt = nullptr;
+    A(s->upload(&dt, tab.data(), tab.size()));
+    v.stencil_tab = dt;
+  }
   A(s->dalloc(&v.stype, n));
   A(s->dalloc(&v.nbr_num, 9 * (size_t)n));
   A(s->dalloc(&v.vir_k, 6 * (size_t)n));
@@ -1155,9 +1210,10 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   // reduction rows: one segment per producer, sized for its largest launch
   {
     const int nblk = (n + kBlock - 1) / kBlock;
-    const int pair_rows = std::max(std::max(pair_blocks(v), force_cells_blocks(v)), v.rbl ? rbl_energy_blocks(v) : 0);
-    const int cap[NSEG] = {pair_rows, kforce_blocks(v), nblk, nblk,
-                           (std::max(s->nmol, 1) + kBlock - 1) / kBlock};
+    const int pair_rows = std::max(std::max(pair_blocks(v), force_cells_blocks(v)),
+                                   v.rbl ? rbl_energy_blocks(v) : 0);
+    const int cap[NSEG] = {pair_rows, kforce_blocks(v), nblk, (std::max(s->nmol, 1) + kBlock - 1) / kBlock,
+                           (n + kWave - 1) / kWave};
     size_t off = 0;
     for (int g = 0; g < NSEG; ++g) {
       s->seg_off[g] = off;
@@ -1778,7 +1834,9 @@ static void enqueue_step(rbmd_sys* s, const double* kv, bool from_ring, bool the
     }
     s->seg_used[SEG_SHAKE] = (s->nmol + kBlock - 1) / kBlock;
   } else {
-    c->run("first_half", [&] { launch_first_half(s->v, s->iv, st, scale, do_bin); });
+    const double* scale_end = s->scale_pending ? &s->nhc->factor_end : nullptr;
+    s->scale_pending = false;
+    c->run("first_half", [&] { launch_first_half(s->v, s->iv, st, scale_end, scale, do_bin); });
     if (shake) {
       c->run("shake", [&] { launch_shake(s->v, s->iv, st, s->seg_rows(SEG_SHAKE), s->shake_iter); });
       s->seg_used[SEG_SHAKE] = (s->nmol + kBlock - 1) / kBlock;
@@ -1795,28 +1853,47 @@ static void enqueue_step(rbmd_sys* s, const double* kv, bool from_ring, bool the
   // forces computed (kernel profiling keeps one stream, for its event timings).
   // Forking before the cell sort instead put the k-space kernels beside the
   // short cell kernels of the critical path and slowed the step.
-  const bool fork = !c->prof && (has_k(s) || has_bonded(s));
+  // Compact systems run one stream: a launch for the pair, structure-factor
+  // and bonded forces and one for the k-space force and the second half step
+  // (the same sums as the separate launches, which profiling and the steps with
+  // thermo sums keep).  Against lists and the side stream on every step: 600
+  // ions 84.5 -> 47.3 us a step, 2,000 76.5 -> 50, 4,000 77.1 -> 53.
+  const bool compact = s->v.compact != 0 && !c->prof && !thermo;
+  const bool fork = !c->prof && !compact && (has_k(s) || has_bonded(s));
   if (fork) {
     (void)hipEventRecord(s->ev_fork, st);
     (void)hipStreamWaitEvent(c->side, s->ev_fork, 0);
     launch_k_bonded(s, kv, thermo, c->side);
     (void)hipEventRecord(s->ev_join, c->side);
   }
-  gather_and_list(s);
-  if (fork) {
+  if (!compact) gather_and_list(s);
+  if (compact) {
+    const KView k = step_kview(s, kv);
+    s->v.nslab = 1;
+    s->locator_built = true;
+    s->nbr_built = false;  // the last step of the call builds the list
+    launch_compact_forces(s->v, s->iv, k, st, has_k(s), has_bonded(s));
+    if (has_k(s)) {
+      launch_rho_reduce(s->v, k, st);
+      launch_compact_finish(s->v, s->iv, k, st, has_bonded(s), s->seg_rows(SEG_KE), &s->seg_used[SEG_KE]);
+    }
+  } else if (fork) {
     launch_real(s, thermo, 0);
     (void)hipStreamWaitEvent(st, s->ev_join, 0);
   } else {
     compute_force(s, kv, thermo);
   }
-  c->run("second_half", [&] {
-    launch_second_half(s->v, s->iv, st, 1, has_k(s), has_bonded(s), s->seg_rows(SEG_KE), &s->seg_used[SEG_KE]);
-  });
+  if (!compact || !has_k(s))
+    c->run("second_half", [&] {
+      launch_second_half(s->v, s->iv, st, 1, has_k(s), has_bonded(s), s->seg_rows(SEG_KE), &s->seg_used[SEG_KE]);
+    });
   if (nh) {
     c->run("nhc", [&] {
       launch_nhc_rows(s->nhc, s->np, rows_desc(s, true), merge_end ? 6 : 2, st, thermo ? 0 : 1);
     });
-    if (tc == RBMD_TEMP_NOSE_HOOVER && !(shake && s->nfree == 0))
+    if (tc == RBMD_TEMP_NOSE_HOOVER && !shake && defer_rattle && merge_end)
+      s->scale_pending = true;  // the next step's first half applies it
+    else if (tc == RBMD_TEMP_NOSE_HOOVER && !(shake && s->nfree == 0))
       c->run("scale_v", [&] { launch_scale_v(s->v, st, &s->nhc->factor_end); });
     if (shake && s->nfree == 0 && defer_rattle && merge_end) {
       s->rattle_pending = true;
@@ -1835,8 +1912,12 @@ static void enqueue_step(rbmd_sys* s, const double* kv, bool from_ring, bool the
   }
 }
 
-// the RATTLE a step left to the next one, alone (a call that stops early)
+// the velocity scale or RATTLE a step left to the next one, alone (a call that stops early)
 static void flush_rattle(rbmd_sys* s) {
+  if (s->scale_pending) {
+    s->ctx->run("scale_v", [&] { launch_scale_v(s->v, s->ctx->stream, &s->nhc->factor_end); });
+    s->scale_pending = false;
+  }
   if (!s->rattle_pending) return;
   s->ctx->run("rattle", [&] { launch_rattle(s->v, s->iv, s->ctx->stream); });
   s->rattle_pending = false;
@@ -2052,7 +2133,7 @@ struct rbmd_pack {
 static const char* const kPackName[PK_COUNT] = {
     "pk_nhc",   "pk_kvec_slot", "pk_first_half", "pk_scan", "pk_scatter",     "pk_cell_sort",
     "pk_one",   "pk_shake",     "pk_nbr_build", "pk_pair",   "pk_rho_partial",
-    "pk_rho_reduce", "pk_kforce", "pk_bonded",   "pk_second_half", "pk_scale_v", "pk_rattle"};
+    "pk_rho_reduce", "pk_kforce", "pk_kforce", "pk_bonded",   "pk_second_half", "pk_scale_v", "pk_rattle"};
 
 // the thermo-row descriptor a system's own step reduces (rows per producer =
 // the grid of that producer's launch)
@@ -2061,7 +2142,7 @@ static RowsDesc pack_rows_desc(rbmd_sys* s, bool has_kk, bool has_bb, bool shk) 
   used[SEG_PAIR] = pair_blocks(s->v);
   used[SEG_K] = has_kk ? kforce_blocks(s->v) : 0;
   used[SEG_BOND] = has_bb ? (s->n + kBlock - 1) / kBlock : 0;
-  used[SEG_KE] = (s->n + kBlock - 1) / kBlock;
+  used[SEG_KE] = (s->n + kWave - 1) / kWave;
   used[SEG_SHAKE] = shk ? (s->nmol + kBlock - 1) / kBlock : 0;
   RowsDesc d;
   d.nseg = NSEG;
@@ -2100,9 +2181,8 @@ static void pack_enqueue_step(rbmd_pack* p, bool thermo) {
     (void)hipStreamWaitEvent(sk, p->ev_fork, 0);
   }
   if (p->has_k) {
-    ksp(PK_RHO, sk);
-    ksp(PK_RHO_RED, sk);
-    ksp(PK_KFORCE, sk);
+    for (int k : {PK_RHO, PK_RHO_RED, PK_KFORCE, PK_KFORCE_C})
+      if (p->nblk[k] > 0) ksp(k, sk);
   }
   if (p->has_b) integ(PK_BONDED, 0, 0, sk);
   if (fork) (void)hipEventRecord(p->ev_join, sk);
@@ -2150,7 +2230,7 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
         s->p.coulomb_type != s0->p.coulomb_type || has_bonded(s) != has_bonded(s0) || shake_on(s) != shake_on(s0) ||
         tc != s0->p.temp_ctrl)
       return fail(RBMD_ERR_ARG, "system %d differs from system 0 in force field, precision, constraints or thermostat", k);
-    if (s->v.k_lanes_lg != s0->v.k_lanes_lg || s->v.rho_kb != s0->v.rho_kb)
+    if (k_lanes_lg_of(s->p) != k_lanes_lg_of(s0->p) || rho_kb_of(s->p) != rho_kb_of(s0->p))
       return fail(RBMD_ERR_ARG, "system %d differs from system 0 in its k-space tile choices", k);
     for (int j = 0; j < k; ++j)
       if (systems[j] == s) return fail(RBMD_ERR_ARG, "system %d appears twice", k);
@@ -2172,8 +2252,8 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
   p->sig.has_k = p->has_k;
   p->sig.ewald = s0->p.coulomb_type == RBMD_COULOMB_EWALD;
   p->sig.has_b = p->has_b;
-  p->sig.k_lanes_lg = s0->v.k_lanes_lg;
-  p->sig.rho_kb = s0->v.rho_kb;
+  p->sig.k_lanes_lg = k_lanes_lg_of(s0->p);  // compact systems have their own tiles
+  p->sig.rho_kb = rho_kb_of(s0->p);
   p->sig.thermo = 1;
   auto dalloc = [&](void** q, size_t bytes) -> rbmd_status {
     hipError_t e = hipMalloc(q, std::max<size_t>(bytes, 4));
@@ -2215,7 +2295,7 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
     for (int q = 0; q < PK_COUNT; ++q) {
       bool on = true;
       if (q == PK_KSLOT) on = p->ring;
-      if (q == PK_RHO || q == PK_RHO_RED || q == PK_KFORCE) on = p->has_k;
+      if (q == PK_RHO || q == PK_RHO_RED || q == PK_KFORCE || q == PK_KFORCE_C) on = p->has_k;
       if (q == PK_BONDED) on = p->has_b;
       if (q == PK_SHAKE || q == PK_RATTLE) on = p->shake;
       blocks[q][k] = on ? pack_blocks(s->v, s->iv, s->P, q) : 0;

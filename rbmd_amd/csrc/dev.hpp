@@ -48,7 +48,9 @@ struct SysView {
   int nseg;         // VERLET: one list segment per (x, y) column of the 3x3x3 stencil (9); RBL: 1
   int seg_cap;      // slots per segment (multiple of the lane count)
   int lanes_lg;     // log2 of the lanes per atom in the pair kernel (2..4)
-  int k_lanes_lg;   // log2 of the lanes per atom in the k-space force kernel (1..3)
+  int compact;      // few atoms: steps without thermo sums take the stencil pair kernel, without a stored list
+  int st_cfg;       // compact: how the stencil pair kernel splits the work (stencil_choice)
+  int k_lanes_lg;   // log2 of the wavefronts splitting the k vectors of the k-space force (1..3; compact 4)
   int rho_kb;       // k vectors per workgroup in the structure-factor kernel (4, 8, 16)
   int sp_max;       // longest special list
   int n_items;      // capacity of the work-item list
@@ -64,6 +66,9 @@ struct SysView {
   // dxdydz[k] * dims[k]: one image shift along axis k as the cell code forms
   // it (kept beside dims and dxdydz whenever they change)
   double shift_len[3];
+  double accept_d2;  // largest d^2 the list predicate accepts: cut2 - d^2 > 1e-4 (as rounded) where d^2 <= accept_d2
+  // stencil pair kernel: the bound on its FP32 d^2's error, and the image shifts in FP32
+  float test_band, shift32[3];
   double volume, cut, cut2, rs, rs2, alpha, sqrt_alpha, qqr2e;
   // per atom, original order (SoA)
   double *x, *y, *z, *vx, *vy, *vz, *fx, *fy, *fz;
@@ -91,6 +96,7 @@ struct SysView {
   int *cursor;      // [ncell]
   int *point_ids;   // [n] sorted position -> atom id
   int *rank;        // [n] atom id -> sorted position
+  const int* stencil_tab;  // [ncell][32] compact: stencil cells 0..26 of every cell (cell << 6 | shift code)
   int *items;       // [n_items] packed (cell << 8 | chunk)
   int *n_items_dev; // [1]
   int *misfit;      // [n] sorted position flag
@@ -98,6 +104,7 @@ struct SysView {
   int *misfit_count;// [1]
   // sorted copies for the pair kernels
   double4* spos;    // [n] x,y,z,q in sorted order
+  float4* spos32;   // [n] x - lo, y - lo, z - lo in FP32 and the type's bits, in sorted order (stencil pair kernel)
   int* stype;       // [n]
   // neighbour lists, column-major [cap][n] of packed (j_sorted << 9 | shift code)
   int* nbr;         // layout nbr_index(slot, i, cap): one row per atom
@@ -162,7 +169,7 @@ struct RowSeg {
   int nrows, width, slot0, groups;
 };
 struct RowsDesc {
-  RowSeg seg[5];
+  RowSeg seg[5];  // the kinetic energy last
   int nseg;
 };
 
@@ -201,6 +208,8 @@ void launch_fill_double(double* p, double v, int n, hipStream_t st);
 // partials: [nblocks][kRowPair] block sums (may be null when thermo == 0)
 void launch_pair(const SysView& s, hipStream_t st, int thermo, int peratom, double* partials, int* nblocks);
 int pair_blocks(const SysView& s);
+bool stencil_pays(const SysView& s);  // the rule for compact systems
+int stencil_choice(const SysView& s);
 // RBL energies over a full rc stencil (no list) and the pair thermo rows
 // (energies + the mean-removed RBL virial); e_lj/e_coul per atom when peratom
 void launch_rbl_energy(const SysView& s, hipStream_t st, int peratom, double* rows, int* nblocks);
@@ -263,7 +272,9 @@ struct IntView {
   int spec_coul;
   const int *grp_off, *grp_ids;
 };
-void launch_first_half(const SysView& s, const IntView& iv, hipStream_t st, const double* scale, int do_bin);
+// scale_end: the velocity scale of the previous step's end, or null (applied before scale)
+void launch_first_half(const SysView& s, const IntView& iv, hipStream_t st, const double* scale_end,
+                       const double* scale, int do_bin);
 void launch_shake(const SysView& s, const IntView& iv, hipStream_t st, double* partials, int* max_iter);
 // launch_first_half + launch_shake in one launch, for systems whose every atom
 // is in a SHAKE triplet (bit for bit the two)
@@ -280,6 +291,13 @@ void launch_second_half(const SysView& s, const IntView& iv, hipStream_t st, int
 void launch_scale_v(const SysView& s, hipStream_t st, const double* scale);
 void launch_ke_rows(const SysView& s, const IntView& iv, hipStream_t st, double* rows);
 void launch_unconstrained_copy(const SysView& s, hipStream_t st, const int* free_ids, int nfree, int pos);
+
+// compact systems, steps without thermo sums, one launch: the stencil pair
+// forces, the structure factor (k, when has_k) and the bonded forces (has_b)
+void launch_compact_forces(const SysView& s, const IntView& iv, const KView& k, hipStream_t st, int has_k, int has_b);
+// and one more: the k-space force and the force assembly with the second kick
+void launch_compact_finish(const SysView& s, const IntView& iv, const KView& k, hipStream_t st, int has_b,
+                           double* rows_ke, int* n_ke);
 
 // NHC / thermostat scalar state on the device (one thread)
 struct NhcState {
@@ -354,6 +372,7 @@ enum PackKernel {
   PK_RHO,
   PK_RHO_RED,
   PK_KFORCE,
+  PK_KFORCE_C,  // compact systems
   PK_BONDED,
   PK_SECOND,
   PK_ATOMS,  // one thread per atom (velocity scale)

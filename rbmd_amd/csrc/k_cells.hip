@@ -329,7 +329,11 @@ __device__ __forceinline__ void cell_sort_body(const SysView& s, const int bid) 
     s.rank[me] = p;
     const double px = s.x[me], py = s.y[me], pz = s.z[me];
     s.spos[p] = make_double4(px, py, pz, s.q[me]);
-    s.stype[p] = s.type[me];
+    const int type = s.type[me];
+    s.stype[p] = type;
+    if (s.spos32)
+      s.spos32[p] = make_float4((float)(px - s.lo[0]), (float)(py - s.lo[1]), (float)(pz - s.lo[2]),
+                                __int_as_float(type));
     if (s.skin_on) {  // the build's positions, for the skin check and the gathers until the next build
       s.x0[me] = px;
       s.y0[me] = py;

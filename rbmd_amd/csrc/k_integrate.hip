@@ -12,15 +12,22 @@
 #include "dev.hpp"
 #include "pack.hpp"
 #include "reduce.hpp"
+#include "atoms.hpp"
 
 namespace rbmd {
 
 // NHC scale (optional), kick, drift, PBC of atom i; returns its cell when
 // do_bin (the binning of the drifted position), else -1
-__device__ __forceinline__ int first_half_atom(const SysView& s, const IntView& iv, const double* scale, int do_bin,
-                                               int i) {
+__device__ __forceinline__ int first_half_atom(const SysView& s, const IntView& iv, const double* scale_end,
+                                               const double* scale, int do_bin, int i) {
 #pragma clang fp contract(off)  // first_half_regs rounds the same way
   double vx = s.vx[i], vy = s.vy[i], vz = s.vz[i];
+  if (scale_end) {  // the previous step's k_scale_v
+    const double f = *scale_end;
+    vx = f * vx;
+    vy = f * vy;
+    vz = f * vz;
+  }
   if (scale) {
     double f = *scale;
     vx = f * vx;
@@ -68,63 +75,25 @@ __device__ __forceinline__ int first_half_atom(const SysView& s, const IntView& 
 }
 
 // NHC scale (optional), kick, drift, PBC, binning
-__device__ __forceinline__ void first_half_body(const SysView& s, const IntView& iv, const double* scale, int do_bin, const int bid) {
+__device__ __forceinline__ void first_half_body(const SysView& s, const IntView& iv, const double* scale_end,
+                                                const double* scale, int do_bin, const int bid) {
   extern __shared__ int lds_cells[];
   int i = bid * blockDim.x + threadIdx.x;
   int cell = -1;
-  if (i < s.n) cell = first_half_atom(s, iv, scale, do_bin, i);
+  if (i < s.n) cell = first_half_atom(s, iv, scale_end, scale, do_bin, i);
   if (do_bin) count_cells(s, cell, lds_cells);
 }
 
-__global__ __launch_bounds__(kBlock) void k_first_half(SysView s, IntView iv, const double* scale, int do_bin) {
-  first_half_body(s, iv, scale, do_bin, (int)blockIdx.x);
+__global__ __launch_bounds__(kBlock) void k_first_half(SysView s, IntView iv, const double* scale_end,
+                                                       const double* scale, int do_bin) {
+  first_half_body(s, iv, scale_end, scale, do_bin, (int)blockIdx.x);
 }
 
-void launch_first_half(const SysView& s, const IntView& iv, hipStream_t st, const double* scale, int do_bin) {
+void launch_first_half(const SysView& s, const IntView& iv, hipStream_t st, const double* scale_end,
+                       const double* scale, int do_bin) {
   size_t lds = (do_bin && s.lds_bins) ? (size_t)s.ncell * sizeof(int) : 0;
-  hipLaunchKernelGGL(k_first_half, dim3((s.n + kBlock - 1) / kBlock), dim3(kBlock), lds, st, s, iv, scale, do_bin);
-}
-
-struct D3 {
-  double x, y, z;
-};
-// The vector helpers, SHAKE and RATTLE compile with FMA contraction off: a
-// product and a sum written in separate helpers are then rounded separately
-// in every kernel that inlines them, so the fused and the separate launches
-// of these steps agree to the bit.
-__device__ __forceinline__ D3 sub(D3 a, D3 b) {
-#pragma clang fp contract(off)
-  return {a.x - b.x, a.y - b.y, a.z - b.z};
-}
-__device__ __forceinline__ D3 add(D3 a, D3 b) {
-#pragma clang fp contract(off)
-  return {a.x + b.x, a.y + b.y, a.z + b.z};
-}
-__device__ __forceinline__ D3 mul(double k, D3 a) {
-#pragma clang fp contract(off)
-  return {k * a.x, k * a.y, k * a.z};
-}
-__device__ __forceinline__ D3 divs(D3 a, double k) {
-#pragma clang fp contract(off)
-  return {a.x / k, a.y / k, a.z / k};
-}
-__device__ __forceinline__ double dotp(D3 a, D3 b) {
-#pragma clang fp contract(off)
-  return a.x * b.x + a.y * b.y + a.z * b.z;
-}
-__device__ __forceinline__ D3 mimg(const SysView& s, D3 a, D3 b) {
-#pragma clang fp contract(off)
-  D3 v = sub(a, b);
-  if (fabs(v.x) > s.box[0] * 0.5) v.x -= (v.x > 0 ? s.box[0] : -s.box[0]);
-  if (fabs(v.y) > s.box[1] * 0.5) v.y -= (v.y > 0 ? s.box[1] : -s.box[1]);
-  if (fabs(v.z) > s.box[2] * 0.5) v.z -= (v.z > 0 ? s.box[2] : -s.box[2]);
-  return v;
-}
-__device__ __forceinline__ D3 ld(const double* x, const double* y, const double* z, int i) { return {x[i], y[i], z[i]}; }
-__device__ __forceinline__ void st3(double* x, double* y, double* z, int i, D3 v) {
-  x[i] = v.x;
-  y[i] = v.y;
-  z[i] = v.z;
+  hipLaunchKernelGGL(k_first_half, dim3((s.n + kBlock - 1) / kBlock), dim3(kBlock), lds, st, s, iv, scale_end, scale,
+                     do_bin);
 }
 
 // SHAKE on (old x, old v, F) of one H-O-H triplet; writes x, v, image flags
@@ -520,122 +489,6 @@ void launch_rattle_first_half_shake(const SysView& s, const IntView& iv, hipStre
                        max_iter);
 }
 
-// bond + angle forces gathered per atom over its incident terms; the energy
-// and virial of a term are counted by its first atom.  With iv.spec_coul
-// (CVFF + RBL + special bonds) also the intramolecular Coulomb correction of
-// ComputeSpecialCoulGeneralWorklet (RunWorklet.cpp:2012-2084, added to the
-// force by ExecutionNVT::ComputeAllForce, ExecutionNVT.cpp:212-214): for the
-// other atoms j of i's molecule (molecules of 3 or more atoms),
-//   F_i += (1 - w_ij) (-332.06371 q_i q_j / r^3) r,  r = MinDistanceVec(x_i, x_j),
-// 332.06371 hard-coded as in the reference (hazard Q24), w_ij the last match of
-// j in i's special list (else 1); its virial +1/2 r (x) F (ComputePairVirial_fix)
-// goes into the bond virial slots (both enter the pressure once,
-// ExecutionMD.cpp:1323-1358).  The random-batch real space has no exclusions,
-// so this removes the intramolecular erfc Coulomb the pair term added.
-template <bool THERMO>
-__device__ __forceinline__ void bonded_body(const SysView& s, const IntView& iv, double* rows, const int bid) {
-  int i = bid * blockDim.x + threadIdx.x;
-  double f[3] = {0, 0, 0};
-  double eb = 0, ea = 0;
-  double vb[6] = {0, 0, 0, 0, 0, 0}, va[6] = {0, 0, 0, 0, 0, 0};
-  if (i < s.n && iv.spec_coul && iv.grp_off[i + 1] - iv.grp_off[i] >= 3) {
-    const D3 pi = ld(s.x, s.y, s.z, i);
-    const double qi = s.q[i];
-    for (int k = iv.grp_off[i]; k < iv.grp_off[i + 1]; ++k) {
-      const int j = iv.grp_ids[k];
-      if (j == i) continue;
-      const D3 r = mimg(s, pi, ld(s.x, s.y, s.z, j));
-      const double dis = sqrt(dotp(r, r));
-      const double fcomp = -332.06371 * qi * s.q[j] / (dis * dis * dis);
-      double w = 1.0;
-      if (s.sp_off)
-        for (int t = s.sp_off[i]; t < s.sp_off[i + 1]; ++t)
-          if (s.sp_ids[t] == j) w = s.sp_w[t];
-      const D3 cp = mul((1.0 - w) * fcomp, r);
-      f[0] += cp.x;
-      f[1] += cp.y;
-      f[2] += cp.z;
-      if (THERMO) {
-        vb[0] += 0.5 * (r.x * cp.x);
-        vb[1] += 0.5 * (r.y * cp.y);
-        vb[2] += 0.5 * (r.z * cp.z);
-        vb[3] += 0.5 * (r.x * cp.y);
-        vb[4] += 0.5 * (r.x * cp.z);
-        vb[5] += 0.5 * (r.y * cp.z);
-      }
-    }
-  }
-  if (i < s.n) {
-    for (int k = iv.inc_b_off[i]; k < iv.inc_b_off[i + 1]; ++k) {
-      int b = iv.inc_b[k];
-      int a0 = iv.bond_atoms[2 * b], a1 = iv.bond_atoms[2 * b + 1];
-      D3 r = mimg(s, ld(s.x, s.y, s.z, a0), ld(s.x, s.y, s.z, a1));
-      double d = sqrt(dotp(r, r));
-      double dr = d - iv.bond_r0[b];
-      double rk = iv.bond_k[b] * dr;
-      double fb = d > 0.01 ? -2.0 * rk / d : 0.0;
-      D3 fi = mul(fb, r);
-      double sg = (a0 == i) ? 1.0 : -1.0;
-      f[0] += sg * fi.x;
-      f[1] += sg * fi.y;
-      f[2] += sg * fi.z;
-      if (THERMO && a0 == i) {
-        eb += rk * dr;
-        vb[0] += r.x * fi.x;
-        vb[1] += r.y * fi.y;
-        vb[2] += r.z * fi.z;
-        vb[3] += r.x * fi.y;
-        vb[4] += r.x * fi.z;
-        vb[5] += r.y * fi.z;
-      }
-    }
-    for (int k = iv.inc_a_off[i]; k < iv.inc_a_off[i + 1]; ++k) {
-      int a = iv.inc_a[k];
-      int ai = iv.angle_all[3 * a], aj = iv.angle_all[3 * a + 1], ak = iv.angle_all[3 * a + 2];
-      D3 pj = ld(s.x, s.y, s.z, aj);
-      D3 rij = mimg(s, ld(s.x, s.y, s.z, ai), pj);
-      D3 rkj = mimg(s, ld(s.x, s.y, s.z, ak), pj);
-      double dij2 = dotp(rij, rij), dij = sqrt(dij2);
-      double dkj2 = dotp(rkj, rkj), dkj = sqrt(dkj2);
-      double c = dotp(rij, rkj);
-      c /= dij * dkj;
-      if (c > 1.0) c = 1.0;
-      if (c < -1.0) c = -1.0;
-      double sn = sqrt(1.0 - c * c);
-      if (sn < 0.001) sn = 0.001;
-      sn = 1.0 / sn;
-      double dth = acos(c) - (iv.angle_t0[a] * kPi) / 180;
-      double tk = iv.angle_k[a] * dth;
-      double aa = -2.0 * tk * sn;
-      double a11 = aa * c / dij2, a12 = -aa / (dij * dkj), a22 = aa * c / dkj2;
-      D3 fi = add(mul(a11, rij), mul(a12, rkj));
-      D3 fk = add(mul(a22, rkj), mul(a12, rij));
-      D3 mine = (i == ai) ? fi : ((i == ak) ? fk : mul(-1.0, add(fi, fk)));
-      f[0] += mine.x;
-      f[1] += mine.y;
-      f[2] += mine.z;
-      if (THERMO && i == ai) {
-        ea += tk * dth;
-        va[0] += rij.x * fi.x + rkj.x * fk.x;
-        va[1] += rij.y * fi.y + rkj.y * fk.y;
-        va[2] += rij.z * fi.z + rkj.z * fk.z;
-        va[3] += rij.x * fi.y + rkj.x * fk.y;
-        va[4] += rij.x * fi.z + rkj.x * fk.z;
-        va[5] += rij.y * fi.z + rkj.y * fk.z;
-      }
-    }
-    s.fbx[i] = f[0];
-    s.fby[i] = f[1];
-    s.fbz[i] = f[2];
-  }
-  if (THERMO) {
-    // slots S_VIR_BOND .. S_VIR_ANGLE + 5, S_EBOND, S_EANGLE
-    const double vals[kRowBond] = {vb[0], vb[1], vb[2], vb[3], vb[4], vb[5], va[0],
-                                   va[1], va[2], va[3], va[4], va[5], eb,    ea};
-    block_write_row<kRowBond>(vals, rows + (size_t)bid * kRowBond);
-  }
-}
-
 template <bool THERMO>
 __global__ __launch_bounds__(kBlock) void k_bonded(SysView s, IntView iv, double* rows) {
   bonded_body<THERMO>(s, iv, rows, (int)blockIdx.x);
@@ -650,61 +503,14 @@ void launch_bonded(const SysView& s, const IntView& iv, hipStream_t st, int ther
     hipLaunchKernelGGL(k_bonded<false>, dim3(grid), dim3(kBlock), 0, st, s, iv, rows);
 }
 
-// F = F_real[rank] (slab partials in order) + F_k + F_bonded; optional second kick;
-// kinetic energy row
-__device__ __forceinline__ void second_half_body(const SysView& s, const IntView& iv, int kick, int has_k, int has_b, double* rows, const int bid) {
-  int i = bid * blockDim.x + threadIdx.x;
-  double ke = 0.0;
-  if (i < s.n) {
-    int r = s.rank[i];
-    double fx = s.fnx[r], fy = s.fny[r], fz = s.fnz[r];
-    for (int k = 1; k < s.nslab; ++k) {
-      const size_t o = (size_t)k * s.n + r;
-      fx += s.fnx[o];
-      fy += s.fny[o];
-      fz += s.fnz[o];
-    }
-    if (has_k) {
-      fx = s.fkx[i] + fx;
-      fy = s.fky[i] + fy;
-      fz = s.fkz[i] + fz;
-    }
-    if (has_b) {
-      fx += s.fbx[i];
-      fy += s.fby[i];
-      fz += s.fbz[i];
-    }
-    s.fx[i] = fx;
-    s.fy[i] = fy;
-    s.fz[i] = fz;
-    double vx = s.vx[i], vy = s.vy[i], vz = s.vz[i];
-    double m = s.mass[i];
-    if (kick) {
-      s.ovx[i] = vx;
-      s.ovy[i] = vy;
-      s.ovz[i] = vz;
-      vx += 0.5 * fx / m * iv.dt * iv.fmt2v;
-      vy += 0.5 * fy / m * iv.dt * iv.fmt2v;
-      vz += 0.5 * fz / m * iv.dt * iv.fmt2v;
-      s.vx[i] = vx;
-      s.vy[i] = vy;
-      s.vz[i] = vz;
-    }
-    ke = m * (vx * vx + vy * vy + vz * vz) * iv.mvv2e;
-    if (!isfinite(fx + fy + fz)) atomicOr(s.status, 1);
-  }
-  const double vals[kRowKe] = {ke};
-  block_write_row<kRowKe>(vals, rows + (size_t)bid * kRowKe);
-}
-
 __global__ __launch_bounds__(kBlock) void k_second_half(SysView s, IntView iv, int kick, int has_k, int has_b, double* rows) {
-  second_half_body(s, iv, kick, has_k, has_b, rows, (int)blockIdx.x);
+  second_half_wave(s, iv, kick, has_k, has_b, rows, (int)(blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave));
 }
 
 void launch_second_half(const SysView& s, const IntView& iv, hipStream_t st, int kick, int has_k, int has_b,
                         double* rows, int* nblocks) {
   int grid = (s.n + kBlock - 1) / kBlock;
-  if (nblocks) *nblocks = grid;
+  if (nblocks) *nblocks = (s.n + kWave - 1) / kWave;
   hipLaunchKernelGGL(k_second_half, dim3(grid), dim3(kBlock), 0, st, s, iv, kick, has_k, has_b, rows);
 }
 
@@ -712,8 +518,9 @@ __global__ __launch_bounds__(kBlock) void k_ke_rows(SysView s, IntView iv, doubl
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   double ke = 0.0;
   if (i < s.n) ke = s.mass[i] * (s.vx[i] * s.vx[i] + s.vy[i] * s.vy[i] + s.vz[i] * s.vz[i]) * iv.mvv2e;
-  const double vals[kRowKe] = {ke};
-  block_write_row<kRowKe>(vals, rows + (size_t)blockIdx.x * kRowKe);
+  ke = wave_sum(ke);
+  const int wave = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+  if ((threadIdx.x & (kWave - 1)) == 0 && wave * kWave < s.n) rows[wave] = ke;
 }
 
 void launch_ke_rows(const SysView& s, const IntView& iv, hipStream_t st, double* rows) {
@@ -909,39 +716,53 @@ __device__ __forceinline__ void nhc_update(NhcState* state, const NhcParams& p, 
 // nseg: thermo row segments to reduce (rd.nseg, or 0 for no reduction)
 __device__ __forceinline__ void nhc_body(NhcState* state, const NhcParams& p, const RowsDesc& rd, const int nseg,
                                          int phase, const int ke_only, const int bid) {
-  // All producer segments at once: segment g owns threads [base, base +
+  // The kinetic energy first, on every phase that reduces: all threads stride
+  // its rows (segment SEG_KE is last), shuffle tree, wavefronts in order.
+  // Then the other segments at once: segment g owns threads [base, base +
   // groups * width); thread (group, k) strides rows group, group + groups, ...
   // of column k (consecutive threads read consecutive doubles), then thread k
   // of the segment adds the group partials in order.  Fixed order throughout.
   __shared__ double part[1024];
+  __shared__ double ke_part[16];
   __shared__ double sums[S_NSLOT];
   const int tid = threadIdx.x;
   if (tid < S_NSLOT) sums[tid] = 0.0;
-  int base = 0, mine = -1, mbase = 0;
-  for (int g = 0; g < nseg; ++g) {
-    const int span = rd.seg[g].groups * rd.seg[g].width;
-    if (tid >= base && tid < base + span) {
-      mine = g;
-      mbase = base;
+  if (nseg > 0) {  // the same for every thread
+    const RowSeg ke = rd.seg[nseg - 1];
+    double acc = 0.0;
+    for (int r = tid; r < ke.nrows; r += 1024) acc += ke.rows[r];
+    acc = wave_sum(acc);
+    if ((tid & (kWave - 1)) == 0) ke_part[tid / kWave] = acc;
+    int base = 0, mine = -1, mbase = 0;
+    for (int g = 0; g < (ke_only ? 0 : nseg - 1); ++g) {
+      const int span = rd.seg[g].groups * rd.seg[g].width;
+      if (tid >= base && tid < base + span) {
+        mine = g;
+        mbase = base;
+      }
+      base += span;
     }
-    base += span;
+    if (mine >= 0) {
+      const RowSeg sg = rd.seg[mine];
+      const int k = (tid - mbase) % sg.width, grp = (tid - mbase) / sg.width;
+      double a = 0.0;
+      for (int r = grp; r < sg.nrows; r += sg.groups) a += sg.rows[(size_t)r * sg.width + k];
+      part[tid] = a;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      double t = ke_part[0];
+      for (int u = 1; u < 16; ++u) t += ke_part[u];
+      sums[S_KE] = t;
+    }
+    if (mine >= 0 && tid - mbase < rd.seg[mine].width) {
+      const RowSeg sg = rd.seg[mine];
+      double a = 0.0;
+      for (int grp = 0; grp < sg.groups; ++grp) a += part[mbase + grp * sg.width + (tid - mbase)];
+      sums[sg.slot0 + (tid - mbase)] = a;
+    }
+    __syncthreads();
   }
-  if (mine >= 0) {
-    const RowSeg sg = rd.seg[mine];
-    const int k = (tid - mbase) % sg.width, grp = (tid - mbase) / sg.width;
-    const int nrows = (ke_only && sg.slot0 != S_KE) ? 0 : sg.nrows;  // skipped sums read as zero
-    double acc = 0.0;
-    for (int r = grp; r < nrows; r += sg.groups) acc += sg.rows[(size_t)r * sg.width + k];
-    part[tid] = acc;
-  }
-  __syncthreads();
-  if (mine >= 0 && tid - mbase < rd.seg[mine].width) {
-    const RowSeg sg = rd.seg[mine];
-    double acc = 0.0;
-    for (int grp = 0; grp < sg.groups; ++grp) acc += part[mbase + grp * sg.width + (tid - mbase)];
-    sums[sg.slot0 + (tid - mbase)] = acc;
-  }
-  __syncthreads();
   if (threadIdx.x != 0) return;
   nhc_update(state, p, sums, phase);
 }
@@ -966,7 +787,7 @@ __global__ __launch_bounds__(1024) void kp_nhc(PACK_PARAMS, int phase, int reduc
 
 __global__ __launch_bounds__(kBlock) void kp_first_half(PACK_PARAMS, int use_scale) {
   PACK_ENTRY(e, bid)
-  first_half_body(e.v, e.iv, use_scale ? &e.nhc->factor : nullptr, 1, bid);
+  first_half_body(e.v, e.iv, nullptr, use_scale ? &e.nhc->factor : nullptr, 1, bid);
 }
 
 // what 0: zero the SHAKE iteration counter; 1: copy the status word to out[k]
@@ -993,7 +814,7 @@ __global__ __launch_bounds__(kBlock) void kp_bonded(PACK_PARAMS) {
 
 __global__ __launch_bounds__(kBlock) void kp_second_half(PACK_PARAMS, int kick, int has_k, int has_b) {
   PACK_ENTRY(e, bid)
-  second_half_body(e.v, e.iv, kick, has_k, has_b, e.rows_ke, bid);
+  second_half_wave(e.v, e.iv, kick, has_k, has_b, e.rows_ke, bid * (kBlock / kWave) + (int)threadIdx.x / kWave);
 }
 
 __global__ __launch_bounds__(kBlock) void kp_scale_v(PACK_PARAMS) {
