@@ -193,6 +193,13 @@ struct rbmd_sys {
   KRec* krec = nullptr;  // [P] k records of the force pass
   double* rho = nullptr;
   int rho_part_cap = 0;  // doubles
+  // grid Ewald (coulomb EWALD): the step's plan and its buffers
+  bool ew_on = false;
+  EwView ew{};
+  double q2 = 0;  // sum of the squared charges
+  // workspace of the Ewald calls on other grids, kept and grown
+  void* ws = nullptr;
+  int64_t ws_bytes = 0;
   // cell geometry of the reference's per-step list (cells of width >= rc) and,
   // for a skin list, of the MD step's list (cells of width >= rc + skin)
   struct Geom {
@@ -545,7 +552,12 @@ static KView step_kview(const rbmd_sys* s, const double* kvec) {
 
 static void launch_k_bonded(rbmd_sys* s, const double* kvec, int thermo, hipStream_t st) {
   rbmd_ctx* c = s->ctx;
-  if (has_k(s)) {
+  if (has_k(s) && s->ew_on) {
+    int nblk = 0;
+    c->run("ewald_rho", [&] { launch_ewald_rho(s->v, s->ew, st); });
+    c->run("ewald_force", [&] { launch_ewald_force(s->v, s->ew, st, thermo, 0, s->seg_rows(SEG_K), &nblk); });
+    if (thermo) s->seg_used[SEG_K] = nblk;
+  } else if (has_k(s)) {
     const KView k = step_kview(s, kvec);
     c->run("rho_partial", [&] { launch_rho_partial(s->v, k, st); });
     c->run("rho_reduce", [&] { launch_rho_reduce(s->v, k, st); });
@@ -654,72 +666,84 @@ void fill_thermo(const rbmd_sys* s, const NhcState& S, int status, int max_iter,
   o->status_flags = status;
 }
 
+// a workspace of at least `bytes` that stays with the system
+rbmd_status ewald_ws(rbmd_sys* s, int64_t bytes, void** out) {
+  if (s->ws_bytes < bytes) {
+    if (s->ws) {
+      HIP_TRY(hipStreamSynchronize(s->ctx->stream));
+      s->allocs.erase(std::find(s->allocs.begin(), s->allocs.end(), s->ws));
+      s->bytes -= s->ws_bytes;
+      (void)hipFree(s->ws);
+      s->ws = nullptr;
+      s->ws_bytes = 0;
+    }
+    char* p = nullptr;
+    RC_TRY(s->dalloc(&p, (size_t)bytes));
+    s->ws = p;
+    s->ws_bytes = bytes;
+  }
+  *out = s->ws;
+  return RBMD_OK;
+}
+
+// phase tables and partials of the Ewald calls: whole systems up to 512 MiB of
+// tables, and in batches of atoms above; the no-alloc scratch's share below it
+constexpr int64_t kEwTables = int64_t(512) << 20, kEwPartials = int64_t(256) << 20;
+constexpr int64_t kEwTablesSmall = int64_t(14) << 20, kEwPartialsSmall = int64_t(10) << 20;
+
+// the grid sum from the energy rows of the weight pass
+rbmd_status ewald_grid_sum(rbmd_sys* s, const EwView& v, double* sum) {
+  std::vector<double> e(ewald_energy_rows(v));
+  HIP_TRY(hipMemcpyAsync(e.data(), v.erow, e.size() * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream));
+  HIP_TRY(hipStreamSynchronize(s->ctx->stream));
+  double t = 0;
+  for (double x : e) t += x;
+  *sum = t;
+  return RBMD_OK;
+}
+
 // e_long = qqr2e (2 pi / V) sum_grid e^{-k^2/4a}|rho|^2/k^2 / N + self / N
 // (ComputeEwaldEnergy + ComputeSelfEnergy, ExecutionMD.cpp:405-443, 508-558).
-// The k grid, the structure-factor partials and the reduced rho live in
-// device memory allocated for the call, or, with `scratch` (the no-alloc
-// entry point), in that buffer of scratch_bytes, which every launch below
-// overwrites in full before reading it (no clearing needed).
+// The phase tables and the structure-factor partials live in the system's
+// workspace, or, with `scratch` (the no-alloc entry point), in that buffer of
+// scratch_bytes, which every launch overwrites in full before reading it (no
+// clearing needed).  Grids that the scratch takes run the same plan, to the
+// same bits, in both.
 rbmd_status long_energy(rbmd_sys* s, const int kmax[3], double* e_avg, double* grid_sum_out,
                         void* scratch = nullptr, size_t scratch_bytes = 0) {
-  std::vector<double> kg;
-  for (int i = -kmax[0]; i <= kmax[0]; ++i)
-    for (int j = -kmax[1]; j <= kmax[1]; ++j)
-      for (int k = -kmax[2]; k <= kmax[2]; ++k)
-        if (i || j || k) {
-          kg.push_back(2 * kPi * i / s->v.box[0]);
-          kg.push_back(2 * kPi * j / s->v.box[1]);
-          kg.push_back(2 * kPi * k / s->v.box[2]);
-        }
-  int K = (int)(kg.size() / 3);
-  const int atoms = rho_atoms_per_block(s->n, rho_kblocks(s->v, K));
+  int64_t K = 1;
+  for (int d = 0; d < 3; ++d) K *= kmax[d] < 0 ? 0 : 2 * (int64_t)kmax[d] + 1;
+  K = K > 0 ? K - 1 : 0;
+  if (K == 0) return fail(RBMD_ERR_HIP, "Ewald energy: the kmax grid holds no k vector");
+  // the scratch takes the grids whose k vectors, reduced and partial structure
+  // factors per atom block fit it, in slices on 256-byte boundaries
+  const int64_t kper = (int64_t)kWave * s->v.rho_kb;
+  const int atoms = rho_atoms_per_block(s->n, (int)std::min<int64_t>((K + kper - 1) / kper, 1 << 30));
   const int nblk = (s->n + atoms - 1) / atoms;
-  // three slices, each starting on a 256-byte boundary
-  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t b_k = up(kg.size() * sizeof(double)), b_rp = up((size_t)nblk * 2 * K * sizeof(double)),
-               b_rr = up((size_t)2 * K * sizeof(double));
-  double *kdev = nullptr, *rp = nullptr, *rr = nullptr;
+  auto up = [](int64_t b) { return (b + 255) & ~int64_t(255); };
+  const int64_t need = up(3 * K * 8) + up((int64_t)nblk * 2 * K * 8) + up(2 * K * 8);
+  const bool small = need <= (int64_t)kScratchBytes;
+  if (scratch && need > (int64_t)scratch_bytes)
+    return fail(RBMD_ERR_ARG,
+                "the kmax grid (%lld k vectors over %d atom blocks) needs %lld bytes of scratch; the no-alloc "
+                "scratch holds %zu",
+                (long long)K, nblk, (long long)need, scratch_bytes);
+  EwView v;
+  ewald_plan(s->n, kmax, small ? kEwTablesSmall : kEwTables, small ? kEwPartialsSmall : kEwPartials, &v);
+  const int64_t bytes = ewald_bytes(v, false);
+  void* base = scratch;
   if (scratch) {
-    if (b_k + b_rp + b_rr > scratch_bytes)
-      return fail(RBMD_ERR_ARG,
-                  "the kmax grid (%d k vectors over %d atom blocks) needs %zu bytes of scratch; the no-alloc "
-                  "scratch holds %zu",
-                  K, nblk, b_k + b_rp + b_rr, scratch_bytes);
-    kdev = static_cast<double*>(scratch);
-    rp = reinterpret_cast<double*>(static_cast<char*>(scratch) + b_k);
-    rr = reinterpret_cast<double*>(static_cast<char*>(scratch) + b_k + b_rp);
+    if (bytes > (int64_t)scratch_bytes)
+      return fail(RBMD_ERR_ARG, "the kmax grid needs %lld bytes of scratch; the no-alloc scratch holds %zu",
+                  (long long)bytes, scratch_bytes);
   } else {
-    HIP_TRY(hipMalloc(&kdev, b_k + b_rp + b_rr));
-    rp = reinterpret_cast<double*>(reinterpret_cast<char*>(kdev) + b_k);
-    rr = reinterpret_cast<double*>(reinterpret_cast<char*>(kdev) + b_k + b_rp);
+    RC_TRY(ewald_ws(s, bytes, &base));
   }
-  std::vector<double> rho((size_t)2 * K);
-  std::vector<double> q(s->n);
-  hipError_t e = hipMemcpyAsync(kdev, kg.data(), kg.size() * sizeof(double), hipMemcpyHostToDevice, s->ctx->stream);
-  if (e == hipSuccess) {
-    KView k{K, 1.0, kdev, rp, rr, nblk, 0, nullptr, 1, atoms};  // energy only: no force records
-    launch_rho_partial(s->v, k, s->ctx->stream);
-    launch_rho_reduce(s->v, k, s->ctx->stream);
-    e = hipMemcpyAsync(rho.data(), rr, rho.size() * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream);
-  }
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(q.data(), s->v.q, s->n * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(s->ctx->stream);
-  if (!scratch) (void)hipFree(kdev);
-  if (e != hipSuccess) return fail(RBMD_ERR_HIP, "Ewald energy: %s", hipGetErrorString(e));
-  double sum = 0, cmp = 0;
-  for (int l = 0; l < K; ++l) {
-    double kx = kg[3 * l], ky = kg[3 * l + 1], kz = kg[3 * l + 2];
-    double k2 = kx * kx + ky * ky + kz * kz;
-    double term = std::exp(-k2 / (4 * s->p.alpha)) * (rho[2 * l] * rho[2 * l] + rho[2 * l + 1] * rho[2 * l + 1]) / k2;
-    double t = sum + term;
-    cmp += std::fabs(sum) >= std::fabs(term) ? (sum - t) + term : (term - t) + sum;
-    sum = t;
-  }
-  sum += cmp;
-  double q2 = 0;
-  for (int i = 0; i < s->n; ++i) q2 += q[i] * q[i];
-  double self = -std::sqrt(s->p.alpha / kPi) * q2;
+  ewald_buffers(&v, base, false);
+  launch_ewald_rho(s->v, v, s->ctx->stream);
+  double sum = 0;
+  RC_TRY(ewald_grid_sum(s, v, &sum));
+  const double self = -std::sqrt(s->p.alpha / kPi) * s->q2;
   if (grid_sum_out) *grid_sum_out = sum;
   *e_avg = s->u.qqr2e * sum * (2 * kPi / s->v.volume) / s->n + s->u.qqr2e * self / s->n;
   return check_launch("long_energy");
@@ -810,6 +834,10 @@ rbmd_status rbmd_footprint_estimate(const rbmd_sys_desc* d, const rbmd_params* p
     slots = 9 * (int64_t)round_up((int)(1.15 * f * c + 64), kMaxLanes);
   }
   int64_t b = n * (8 * 60 + 4 * 24) + cells * 16 + slots * n * 4;
+  if (p->coulomb_type == RBMD_COULOMB_EWALD) {
+    EwView v;
+    if (ewald_plan(d->n_atoms, p->kmax, INT64_MAX, kEwPartials, &v)) b += ewald_bytes(v, true);
+  }
   b += (int64_t)3 * std::max(p->rbe_p, 1) * 8 * 512 + ((n + 1023) / 1024) * 2 * std::max(p->rbe_p, 1) * 8;
   *bytes = b;
   return RBMD_OK;
@@ -959,7 +987,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   // lanes per atom in the pair kernel: enough threads to fill 256 CUs for
   // small systems, fewer lanes (longer per-lane loops) for large ones
   v.lanes_lg = n <= 60000 ? 4 : (n <= 250000 ? 3 : 2);
-  v.compact = !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes && stencil_pays(v) ? 1 : 0;
+  v.compact = p->coulomb_type != RBMD_COULOMB_EWALD && !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes && stencil_pays(v) ? 1 : 0;
   v.st_cfg = stencil_choice(v);
   if (p->pair_lanes) v.lanes_lg = p->pair_lanes == 4 ? 2 : (p->pair_lanes == 8 ? 3 : 4);
   if (v.compact) v.lanes_lg = 4;  // as the stencil kernel sums
@@ -988,6 +1016,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   A(s->dalloc(&v.vir_near, 18 * (size_t)n));
   v.nslab = 1;
   A(s->upload(&v.q, d->charge, n));
+  for (int i = 0; i < n; ++i) s->q2 += d->charge[i] * d->charge[i];
   A(s->upload(&v.mass, d->mass, n));
   A(s->upload(&v.type, d->type, n));
   A(s->dalloc(&v.img, 3 * (size_t)n));
@@ -1254,6 +1283,15 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
       s->P = (int)(kg.size() / 3);
       A(s->upload(&s->kcur, kg.data(), kg.size()));
       A(ensure_rho(s, s->P));
+      // one batch (packs take a system's tables whole)
+      if (rc == RBMD_OK && ewald_plan(n, p->kmax, INT64_MAX, kEwPartials, &s->ew)) {
+        char* base = nullptr;
+        A(s->dalloc(&base, (size_t)ewald_bytes(s->ew, true)));
+        if (rc == RBMD_OK) {
+          ewald_buffers(&s->ew, base, true);
+          s->ew_on = true;
+        }
+      }
     }
   }
   if (rc != RBMD_OK) {
@@ -1620,20 +1658,9 @@ rbmd_status rbmd_rbe_structure_factor(rbmd_sys* s, double* rho_out) {
   return RBMD_OK;
 }
 
-static rbmd_status kforce_out(rbmd_sys* s, int ewald, double* force, double* vir) {
-  KView k = s->kv;
-  k.P = s->P;
-  k.kvec = s->kcur;
-  k.S_over_P = ewald ? 1.0 : s->S / (double)s->P;
-  k.f32 = ewald ? 0 : s->v.mixed;  // the converged Ewald sum is always FP64
-  k.ewald = ewald;
+// the k-space forces (and virials) of the launches just made, to the host
+static rbmd_status download_kforce(rbmd_sys* s, double* force, double* vir) {
   hipStream_t st = s->ctx->stream;
-  s->ctx->run("rho_partial", [&] { launch_rho_partial(s->v, k, st); });
-  s->ctx->run("rho_reduce", [&] { launch_rho_reduce(s->v, k, st); });
-  s->ctx->run("kforce", [&] {
-    launch_kforce(s->v, k, st, 1, 1, s->seg_rows(SEG_K), &s->seg_used[SEG_K]);
-  });
-  RC_TRY(check_launch("kforce"));
   int n = s->n;
   std::vector<double> fx(n), fy(n), fz(n);
   HIP_TRY(hipMemcpyAsync(fx.data(), s->v.fkx, n * 8, hipMemcpyDeviceToHost, st));
@@ -1653,42 +1680,38 @@ static rbmd_status kforce_out(rbmd_sys* s, int ewald, double* force, double* vir
 rbmd_status rbmd_rbe_force(rbmd_sys* s, double* force, double* vir) {
   if (!s) return fail(RBMD_ERR_ARG, "null sys");
   if (s->p.coulomb_type != RBMD_COULOMB_RBE || !s->kcur) return fail(RBMD_ERR_STATE, "no RBE k vectors");
-  return kforce_out(s, 0, force, vir);
+  const KView k = step_kview(s, s->kcur);
+  hipStream_t st = s->ctx->stream;
+  s->ctx->run("rho_partial", [&] { launch_rho_partial(s->v, k, st); });
+  s->ctx->run("rho_reduce", [&] { launch_rho_reduce(s->v, k, st); });
+  s->ctx->run("kforce", [&] {
+    launch_kforce(s->v, k, st, 1, 1, s->seg_rows(SEG_K), &s->seg_used[SEG_K]);
+  });
+  RC_TRY(check_launch("kforce"));
+  return download_kforce(s, force, vir);
 }
 
 rbmd_status rbmd_ewald_force(rbmd_sys* s, const int32_t kmax[3], double* force, double* vir, double* energy_total) {
   if (!s || !kmax) return fail(RBMD_ERR_ARG, "bad arguments");
   if (s->v.lj_only) return fail(RBMD_ERR_STATE, "LJ/CUT has no k space");
-  std::vector<double> kg;
-  for (int i = -kmax[0]; i <= kmax[0]; ++i)
-    for (int j = -kmax[1]; j <= kmax[1]; ++j)
-      for (int k = -kmax[2]; k <= kmax[2]; ++k)
-        if (i || j || k) {
-          kg.push_back(2 * kPi * i / s->v.box[0]);
-          kg.push_back(2 * kPi * j / s->v.box[1]);
-          kg.push_back(2 * kPi * k / s->v.box[2]);
-        }
-  int K = (int)(kg.size() / 3);
-  double* saved_k = s->kcur;
-  int saved_P = s->P;
-  double* kdev = nullptr;
-  HIP_TRY(hipMalloc(&kdev, kg.size() * 8));
-  HIP_TRY(hipMemcpy(kdev, kg.data(), kg.size() * 8, hipMemcpyHostToDevice));
-  s->P = K;
-  s->kcur = kdev;
-  rbmd_status rc = ensure_rho(s, K);
-  if (rc == RBMD_OK) rc = kforce_out(s, 1, force, vir);
-  s->kcur = saved_k;
-  s->P = saved_P;
-  if (rc == RBMD_OK) rc = ensure_rho(s, saved_P);  // the step's block sizes again
-  (void)hipFree(kdev);
-  if (rc != RBMD_OK) return rc;
+  EwView v;
+  if (!ewald_plan(s->n, kmax, kEwTables, kEwPartials, &v))
+    return fail(RBMD_ERR_HIP, "Ewald force: the kmax grid holds no k vector");
+  void* base = nullptr;
+  RC_TRY(ewald_ws(s, ewald_bytes(v, true), &base));
+  ewald_buffers(&v, base, true);
+  hipStream_t st = s->ctx->stream;
+  s->ctx->run("ewald_rho", [&] { launch_ewald_rho(s->v, v, st); });
+  s->ctx->run("ewald_force", [&] {
+    launch_ewald_force(s->v, v, st, 1, 1, s->seg_rows(SEG_K), &s->seg_used[SEG_K]);
+  });
+  RC_TRY(check_launch("ewald_force"));
   if (energy_total) {
-    double e_avg = 0, grid = 0;
-    RC_TRY(long_energy(s, kmax, &e_avg, &grid));
+    double grid = 0;
+    RC_TRY(ewald_grid_sum(s, v, &grid));
     *energy_total = s->u.qqr2e * grid * (2 * kPi / s->v.volume);
   }
-  return RBMD_OK;
+  return download_kforce(s, force, vir);
 }
 
 rbmd_status rbmd_static_table_gnear(rbmd_ctx* c, int32_t n, const double* dis, double* g) {
@@ -2133,14 +2156,15 @@ struct rbmd_pack {
 static const char* const kPackName[PK_COUNT] = {
     "pk_nhc",   "pk_kvec_slot", "pk_first_half", "pk_scan", "pk_scatter",     "pk_cell_sort",
     "pk_one",   "pk_shake",     "pk_nbr_build", "pk_pair",   "pk_rho_partial",
-    "pk_rho_reduce", "pk_kforce", "pk_kforce", "pk_bonded",   "pk_second_half", "pk_scale_v", "pk_rattle"};
+    "pk_rho_reduce", "pk_kforce", "pk_kforce", "pk_ewald_rho", "pk_ewald_rho", "pk_ewald_rho", "pk_ewald_rho",
+    "pk_ewald_rho", "pk_ewald_force", "pk_ewald_force", "pk_bonded",   "pk_second_half", "pk_scale_v", "pk_rattle"};
 
 // the thermo-row descriptor a system's own step reduces (rows per producer =
 // the grid of that producer's launch)
 static RowsDesc pack_rows_desc(rbmd_sys* s, bool has_kk, bool has_bb, bool shk) {
   int used[NSEG];
   used[SEG_PAIR] = pair_blocks(s->v);
-  used[SEG_K] = has_kk ? kforce_blocks(s->v) : 0;
+  used[SEG_K] = has_kk ? (s->ew_on ? (s->n + kBlock - 1) / kBlock : kforce_blocks(s->v)) : 0;
   used[SEG_BOND] = has_bb ? (s->n + kBlock - 1) / kBlock : 0;
   used[SEG_KE] = (s->n + kWave - 1) / kWave;
   used[SEG_SHAKE] = shk ? (s->nmol + kBlock - 1) / kBlock : 0;
@@ -2183,6 +2207,9 @@ static void pack_enqueue_step(rbmd_pack* p, bool thermo) {
   if (p->has_k) {
     for (int k : {PK_RHO, PK_RHO_RED, PK_KFORCE, PK_KFORCE_C})
       if (p->nblk[k] > 0) ksp(k, sk);
+    for (int k = PK_EW_TABLE; k <= PK_EW_FINISH; ++k)
+      if (p->nblk[k] > 0)
+        c->run(kPackName[k], [&] { launch_pack_ewald(k, p->L[k], p->nblk[k], sig.thermo, sk); });
   }
   if (p->has_b) integ(PK_BONDED, 0, 0, sk);
   if (fork) (void)hipEventRecord(p->ev_join, sk);
@@ -2281,6 +2308,7 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
     e.kv.S_over_P = s->p.coulomb_type == RBMD_COULOMB_RBE ? s->S / (double)s->P : 1.0;
     e.kv.f32 = s->v.mixed;
     e.kv.ewald = s->p.coulomb_type == RBMD_COULOMB_EWALD;
+    e.ew = s->ew;
     e.nhc = s->nhc;
     e.np = s->np;
     e.rd = pack_rows_desc(s, p->has_k, p->has_b, p->shake);
@@ -2295,7 +2323,11 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
     for (int q = 0; q < PK_COUNT; ++q) {
       bool on = true;
       if (q == PK_KSLOT) on = p->ring;
-      if (q == PK_RHO || q == PK_RHO_RED || q == PK_KFORCE || q == PK_KFORCE_C) on = p->has_k;
+      if (q == PK_RHO || q == PK_RHO_RED || q == PK_KFORCE || q == PK_KFORCE_C) on = p->has_k && !s->ew_on;
+      if (q >= PK_EW_TABLE && q <= PK_EW_FINISH) {
+        blocks[q][k] = p->has_k && s->ew_on ? pack_ewald_blocks(s->ew, q) : 0;
+        continue;
+      }
       if (q == PK_BONDED) on = p->has_b;
       if (q == PK_SHAKE || q == PK_RATTLE) on = p->shake;
       blocks[q][k] = on ? pack_blocks(s->v, s->iv, s->P, q) : 0;

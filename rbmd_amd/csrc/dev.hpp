@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "ewald.hpp"
+
 struct rbmd_ctx;  // the C ABI's context (include/rbmd_mi355x.h), defined in api.cpp
 
 namespace rbmd {
@@ -250,6 +252,11 @@ void launch_rho_reduce(const SysView& s, const KView& k, hipStream_t st);
 void launch_kforce(const SysView& s, const KView& k, hipStream_t st, int thermo, int peratom, double* partials,
                    int* nblocks);
 int kforce_blocks(const SysView& s);
+// the Ewald sum over a kmax grid (k_ewald.hip): structure factor, force weights
+// and energy rows, then the forces (thermo rows as launch_kforce)
+void launch_ewald_rho(const SysView& s, EwView v, hipStream_t st);
+void launch_ewald_force(const SysView& s, EwView v, hipStream_t st, int thermo, int peratom, double* rows,
+                        int* nblocks);
 void launch_kvec_slot(double* dst, const double* ring, int R, int per, const int64_t* step, hipStream_t st);
 
 // ---------------------------------------------------------------- integrate
@@ -340,6 +347,7 @@ struct PackSys {
   SysView v;
   IntView iv;
   KView kv;               // kv.kvec: this step's k vectors
+  EwView ew;              // grid Ewald systems
   NhcState* nhc;
   NhcParams np;
   RowsDesc rd;            // thermo rows, reduced by the NHC phase 2 launch
@@ -373,6 +381,13 @@ enum PackKernel {
   PK_RHO_RED,
   PK_KFORCE,
   PK_KFORCE_C,  // compact systems
+  PK_EW_TABLE,  // grid Ewald systems
+  PK_EW_RHO1,
+  PK_EW_RHO2,
+  PK_EW_RHO4,
+  PK_EW_WEIGHT,
+  PK_EW_FORCE,
+  PK_EW_FINISH,
   PK_BONDED,
   PK_SECOND,
   PK_ATOMS,  // one thread per atom (velocity scale)
@@ -395,6 +410,8 @@ struct PackSig {  // launch-wide choices, equal for every system of a pack
 // 1 = copy every status word to out[k].
 void launch_pack_cells(int kernel, const PackLaunch& L, int nblocks, size_t lds, hipStream_t st);
 void launch_pack_pair(const PackLaunch& L, int nblocks, const PackSig& g, hipStream_t st);
+int pack_ewald_blocks(const EwView& v, int kernel);
+void launch_pack_ewald(int kernel, const PackLaunch& L, int nblocks, int thermo, hipStream_t st);
 void launch_pack_kspace(int kernel, const PackLaunch& L, int nblocks, const PackSig& g, hipStream_t st);
 void launch_pack_integrate(int kernel, const PackLaunch& L, int nblocks, const PackSig& g, int arg, size_t lds,
                            int* out, hipStream_t st);
