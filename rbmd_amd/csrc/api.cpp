@@ -1014,6 +1014,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   double** slabbed[] = {&v.fnx, &v.fny, &v.fnz, &v.e_lj, &v.e_coul};
   for (double** f : slabbed) A(s->dalloc(f, 3 * (size_t)n));
   A(s->dalloc(&v.vir_near, 18 * (size_t)n));
+  if (v.rbl) A(s->dalloc(&v.rbl_rows, 9 * (size_t)rbl_pair_blocks(v)));
   v.nslab = 1;
   A(s->upload(&v.q, d->charge, n));
   for (int i = 0; i < n; ++i) s->q2 += d->charge[i] * d->charge[i];

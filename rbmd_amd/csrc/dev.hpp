@@ -117,6 +117,7 @@ struct SysView {
   double *fkx, *fky, *fkz;  // k space
   double *fbx, *fby, *fbz;  // bonded
   // per-atom optional outputs (sorted order for real space)
+  double* rbl_rows;  // [rbl_pair_blocks][9] RBL force and virial sums of the pair kernel's workgroups
   double* vir_near;  // [6n] or null
   double* e_lj;      // [n] or null
   double* e_coul;    // [n] or null
@@ -216,6 +217,10 @@ int stencil_choice(const SysView& s);
 // (energies + the mean-removed RBL virial); e_lj/e_coul per atom when peratom
 void launch_rbl_energy(const SysView& s, hipStream_t st, int peratom, double* rows, int* nblocks);
 int rbl_energy_blocks(const SysView& s);
+// random-batch lists; the corrected pair force with its means removed (and its virial)
+void launch_nbr_build_rbl(const SysView& s, hipStream_t st);
+void launch_pair_rbl(const SysView& s, hipStream_t st, int virial);
+int rbl_pair_blocks(const SysView& s);
 // the RBL erfc step table at n distances (device arrays)
 void launch_static_table(const double* dis, double* g, int n, hipStream_t st);
 // fused cell-stencil real-space force (no stored list); fn* get 3 slab partials

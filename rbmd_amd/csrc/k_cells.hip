@@ -8,12 +8,11 @@
 // the result is bit-exact and independent of atomic ordering.
 //
 // Neighbour lists follow ComputeNeighboursWorklet (RunWorklet.cpp:296-355) and
-// ComputeRBLNeighboursOnceWorklet (:906-980): the (2nc+1)^3 stencil around
-// InWhichCell(p_i) in x-outer / z-inner order, cells in sorted order, accept
-// when rc^2 - d^2 > 1e-4 and d^2 > 1e-4 (RBL: core d < rs, every pice_num-th
-// shell atom), with d^2 rounded as the oracle rounds it (dist2).  One
-// wavefront owns 64 i-atoms of a cell and one stencil column (VERLET) or
-// the whole stencil (RBL); candidates are loaded coalesced and broadcast
+// ComputeRBLNeighboursOnceWorklet (:906-980, k_rbl.hip): the (2nc+1)^3 stencil
+// around InWhichCell(p_i) in x-outer / z-inner order, cells in sorted order,
+// accept when rc^2 - d^2 > 1e-4 and d^2 > 1e-4, with d^2 rounded as the oracle
+// rounds it (dist2).  One wavefront owns 64 i-atoms of a cell and one stencil
+// column; candidates are loaded coalesced and broadcast
 // through LDS.  Lists are row-major (one row of segments per atom), so the
 // pair kernel's lanes of one atom read consecutive entries.
 #include "dev.hpp"
@@ -667,160 +666,9 @@ __global__ __launch_bounds__(kNbrWaves * kWave) void k_nbr_build_verlet(SysView 
   nbr_build_verlet_body(s, (int)blockIdx.x);
 }
 
-// RBL list state: core slots [0, rs_num), kept shell slots from rs_num (every
-// pice_num-th shell atom in traversal order, so one lane walks the whole stencil)
-struct RblState {
-  int core, shell_seen, shell_kept;
-};
-
-__device__ __forceinline__ void rbl_consider(const SysView& s, RblState& L, int i, int entry, double d2) {
-  if (s.cut2 - d2 > 0.0001 && d2 - s.rs2 > 0.0001) {
-    if (L.shell_seen % s.pice_num == 0) {
-      int slot = s.rs_num + L.shell_kept;
-      if (slot < s.cap)
-        s.nbr[nbr_index(slot, i, s.cap)] = entry;
-      else
-        atomicOr(s.status, 4);
-      L.shell_kept++;
-    }
-    L.shell_seen++;
-  } else if (s.rs2 - d2 > 0.0001 && d2 > 0.0001) {
-    if (L.core < s.rs_num)
-      s.nbr[nbr_index(L.core, i, s.cap)] = entry;
-    else
-      atomicOr(s.status, 4);
-    L.core++;
-  }
-}
-
-__device__ __forceinline__ void rbl_finish(const SysView& s, const RblState& L, int i) {
-  s.nbr_num[2 * i] = L.core < s.rs_num ? L.core : s.rs_num;
-  int kept = L.shell_kept;
-  if (s.rs_num + kept > s.cap) kept = s.cap - s.rs_num;
-  s.nbr_num[2 * i + 1] = kept;
-}
-
-// RBL list build: one wavefront per work item; the j loop is wave-uniform
-// (scalar loads broadcast to all lanes)
-__global__ __launch_bounds__(kBlock) void k_nbr_build_rbl(SysView s) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int lane = threadIdx.x & (kWave - 1);
-  const int item_idx = blockIdx.x * (kBlock / kWave) + wave;
-  if (item_idx >= s.n_items_dev[0]) return;
-  const int item = __builtin_amdgcn_readfirstlane(s.items[item_idx]);
-  const int c = item >> 8;
-  const int chunk = item & 255;
-  const int start = s.cell_start[c];
-  const int cnt_c = s.cell_start[c + 1] - start;
-  const int local = chunk * kChunk + lane;
-  const int i = start + local;
-  bool active = local < cnt_c;
-  double4 pi = make_double4(0, 0, 0, 0);
-  if (active) {
-    pi = s.spos[i];
-    if (s.misfit[i]) active = false;
-  }
-  const int ca = c % s.dims[0];
-  const int cb = (c / s.dims[0]) % s.dims[1];
-  const int cc = c / (s.dims[0] * s.dims[1]);
-  RblState L = {0, 0, 0};
-  const int nc = s.nc;
-  for (int a = -nc; a <= nc; ++a)
-    for (int b = -nc; b <= nc; ++b)
-      for (int e = -nc; e <= nc; ++e) {
-        StencilCell t = stencil_cell(s, ca, cb, cc, a, b, e);
-        if (!t.ok) {
-          if (lane == 0) atomicOr(s.status, 4);
-          continue;
-        }
-        const int code = pack_entry(0, t.sa, t.sb, t.sc);
-        for (int j = t.js; j < t.je; ++j) {
-          double4 pj = s.spos[j];  // wave-uniform address -> scalar load
-          double rx = (pj.x - t.ox) - pi.x;
-          double ry = (pj.y - t.oy) - pi.y;
-          double rz = (pj.z - t.oz) - pi.z;
-          double d2 = dist2(rx, ry, rz);
-          if (active) rbl_consider(s, L, i, (j << kShiftBits) | code, d2);
-        }
-      }
-  if (active) rbl_finish(s, L, i);
-}
-
-// RBL misfit atoms, one wavefront each: core entries at their ballot prefix;
-// shell candidates get their ordinal in traversal order from the ballot prefix
-// and every pice_num-th one is kept, again at its ballot prefix among the kept
-__global__ __launch_bounds__(kBlock) void k_nbr_misfit_rbl(SysView s) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int gw = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
-  const int nw = gridDim.x * blockDim.x / kWave;
-  const int count = s.misfit_count[0];
-  const unsigned long long below = (1ull << lane) - 1ull;
-  for (int m = gw; m < count; m += nw) {
-    const int i = __builtin_amdgcn_readfirstlane(s.misfit_list[m]);
-    const double4 pi = s.spos[i];
-    const int ca = cell_axis(pi.x, s.lo[0], s.dxdydz[0]);
-    const int cb = cell_axis(pi.y, s.lo[1], s.dxdydz[1]);
-    const int cc = cell_axis(pi.z, s.lo[2], s.dxdydz[2]);
-    int core = 0, seen = 0, kept = 0;
-    const int nc = s.nc;
-    for (int a = -nc; a <= nc; ++a)
-      for (int b = -nc; b <= nc; ++b)
-        for (int e = -nc; e <= nc; ++e) {
-          StencilCell t = stencil_cell(s, ca, cb, cc, a, b, e);
-          if (!t.ok) {
-            if (lane == 0) atomicOr(s.status, 1);
-            continue;
-          }
-          const int code = pack_entry(0, t.sa, t.sb, t.sc);
-          for (int base = t.js; base < t.je; base += kWave) {
-            const int j = base + lane;
-            bool is_shell = false, is_core = false;
-            if (j < t.je) {
-              double4 pj = s.spos[j];
-              double rx = (pj.x - t.ox) - pi.x;
-              double ry = (pj.y - t.oy) - pi.y;
-              double rz = (pj.z - t.oz) - pi.z;
-              double d2 = dist2(rx, ry, rz);
-              is_shell = s.cut2 - d2 > 0.0001 && d2 - s.rs2 > 0.0001;
-              is_core = !is_shell && s.rs2 - d2 > 0.0001 && d2 > 0.0001;
-            }
-            const int entry = (j << kShiftBits) | code;
-            const unsigned long long bc = __ballot(is_core);
-            if (is_core) {
-              int slot = core + __popcll(bc & below);
-              if (slot < s.rs_num)
-                s.nbr[nbr_index(slot, i, s.cap)] = entry;
-              else
-                atomicOr(s.status, 4);
-            }
-            core += __popcll(bc);
-            const unsigned long long bs = __ballot(is_shell);
-            const bool keep = is_shell && ((seen + __popcll(bs & below)) % s.pice_num == 0);
-            const unsigned long long bk = __ballot(keep);
-            if (keep) {
-              int slot = s.rs_num + kept + __popcll(bk & below);
-              if (slot < s.cap)
-                s.nbr[nbr_index(slot, i, s.cap)] = entry;
-              else
-                atomicOr(s.status, 4);
-            }
-            seen += __popcll(bs);
-            kept += __popcll(bk);
-          }
-        }
-    if (lane == 0) {
-      RblState L = {core, seen, kept};
-      rbl_finish(s, L, i);
-    }
-  }
-}
-
 void launch_nbr_build(const SysView& s, hipStream_t st) {
   if (s.rbl) {
-    int grid = (s.n_items + (kBlock / kWave) - 1) / (kBlock / kWave);
-    hipLaunchKernelGGL(k_nbr_build_rbl, dim3(grid), dim3(kBlock), 0, st, s);
-    int waves = s.n < 1024 ? s.n : 1024;
-    hipLaunchKernelGGL(k_nbr_misfit_rbl, dim3((waves * kWave + kBlock - 1) / kBlock), dim3(kBlock), 0, st, s);
+    launch_nbr_build_rbl(s, st);
   } else {
     hipLaunchKernelGGL(k_nbr_build_verlet, dim3(kNbrParts * (s.n_items + kMisfitBlocks)), dim3(kNbrWaves * kWave), 0,
                        st, s);

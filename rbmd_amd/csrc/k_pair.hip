@@ -11,10 +11,10 @@
 //   VERLET plain    ComputeNearForceVerletVirialWorklet, RunWorklet.cpp:2890-2985
 //   VERLET weighted ComputeNearForceVerletWeightVirialWorklet1, RunWorklet.cpp:2767-2888
 //   LJ/CUT only     ComputeLJForceVerletWorklet, RunWorklet.cpp:498-575
-//   RBL             ComputeNearForceRBLERF(SpecialBonds)Worklet, RunWorklet.cpp:982-1266
+//   (random-batch lists: k_rbl.hip)
 //   LJ      ExecForceFunction.h:412-435 (force), :818-841 (energy)
 //   G(r)    ExecForceFunction.h:682-689, erfc(sqrt(alpha) r)/r^2 + 2 sqrt(alpha/pi) e^{-alpha r^2}/r
-//   virial  ComputePairVirial_fix (+1/2, plain) / ComputePairVirial (-1/2, weighted, RBL), :304-332
+//   virial  ComputePairVirial_fix (+1/2, plain) / ComputePairVirial (-1/2, weighted), :304-332
 #include <type_traits>
 
 #include "dev.hpp"
@@ -297,275 +297,16 @@ void launch_pair_t(const SysView& s, hipStream_t st, int thermo, int peratom, do
     launch_pair_v<MODE, SP, false, false>(s, st, thermo, peratom, rows, grid);
 }
 
-// RBL: per-atom corrected force before the mean removal; the virial keeps the
-// reference's assignment of the running-sum force of the last pair (hazard Q5).
-template <bool WEIGHTED>
-__global__ __launch_bounds__(kBlock) void k_pair_rbl(SysView s) {
-#pragma clang fp contract(off)  // the pair vector and d2 rounded as the list build and the oracle round them
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= s.n) return;
-  const double4 pi = s.spos[i];
-  const int ti = s.stype[i];
-  const double qi = pi.w;
-  int spn = 0;
-  int spj[kMaxSpecial];
-  double spw[kMaxSpecial];
-  if (WEIGHTED) {
-    int id = s.point_ids[i];
-    int b = s.sp_off[id], e = s.sp_off[id + 1];
-    spn = e - b;
-    if (spn > kMaxSpecial) {
-      atomicOr(s.status, 4);
-      spn = kMaxSpecial;
-    }
-#pragma unroll
-    for (int k = 0; k < kMaxSpecial; ++k) {
-      spj[k] = k < spn ? s.rank[s.sp_ids[b + k]] : -1;
-      spw[k] = k < spn ? s.sp_w[b + k] : 1.0;
-    }
-  }
-  const double* eps_row = s.eps_ij + ti * s.ntypes;
-  const double* sig_row = s.sig6_ij + ti * s.ntypes;
-  double lj_rs[3] = {0, 0, 0}, lj_rcs[3] = {0, 0, 0}, el_rs[3] = {0, 0, 0}, el_rcs[3] = {0, 0, 0};
-  double vir_rs[6] = {0, 0, 0, 0, 0, 0}, vir_rcs[6] = {0, 0, 0, 0, 0, 0};
-  const double pice = (double)s.pice_num;
-  for (int part = 0; part < 2; ++part) {
-    const int num = s.nbr_num[2 * i + part];
-    const int base = part == 0 ? 0 : s.rs_num;
-    for (int k = 0; k < num; ++k) {
-      int j;
-      double ox, oy, oz;
-      decode(s, s.nbr[nbr_index(base + k, i, s.cap)], j, ox, oy, oz);
-      const double4 pj = s.spos[j];
-      double rx = (pj.x - ox) - pi.x;
-      double ry = (pj.y - oy) - pi.y;
-      double rz = (pj.z - oz) - pi.z;
-      min_image(s, rx, ry, rz);
-      const double d2 = dist2(rx, ry, rz);
-      const double dis = sqrt(d2);
-      const int tj = s.stype[j];
-      const double epsij = eps_row[tj];
-      const double sig6 = sig_row[tj];
-      const double qq = qi * pj.w;
-      const double g = s.erfc_table ? gnear_table(dis) : gnear(s.alpha, s.sqrt_alpha, dis);
-      double w = 1.0;
-      if (WEIGHTED) {
-#pragma unroll
-        for (int t = 0; t < kMaxSpecial; ++t)
-          if (spj[t] == j) w = spw[t];
-      }
-      double d6 = d2 * d2 * d2;
-      double sd6 = sig6 / d6;
-      double ljs = -24.0 * epsij * ((2.0 * sd6 - 1.0) * sd6) / d2;
-      if (part == 0) {
-        if (d2 < s.cut2 && d2 > 0.0001) {
-          double e = -qq * g / dis;
-          el_rs[0] += e * rx;
-          el_rs[1] += e * ry;
-          el_rs[2] += e * rz;
-        }
-        if (d2 < s.rs2 && d2 > 0.0001) {  // LJ core with cutoff rs (hazard Q4)
-          lj_rs[0] += w * (ljs * rx);
-          lj_rs[1] += w * (ljs * ry);
-          lj_rs[2] += w * (ljs * rz);
-        }
-        for (int t = 0; t < 6; ++t) vir_rs[t] = 0;
-        vir_add(vir_rs, rx, ry, rz, lj_rs[0] + s.qqr2e * el_rs[0], lj_rs[1] + s.qqr2e * el_rs[1],
-                lj_rs[2] + s.qqr2e * el_rs[2], -0.5);
-      } else {
-        bool inshell = WEIGHTED ? (d2 < s.cut2 && d2 > s.rs2) : (d2 < s.cut2 && d2 > 0.0001);
-        if (inshell) {
-          double e = -qq * g / dis;
-          el_rcs[0] += pice * (e * rx);
-          el_rcs[1] += pice * (e * ry);
-          el_rcs[2] += pice * (e * rz);
-        }
-        if (d2 < s.cut2 && d2 > s.rs2) {
-          lj_rcs[0] += w * (pice * (ljs * rx));
-          lj_rcs[1] += w * (pice * (ljs * ry));
-          lj_rcs[2] += w * (pice * (ljs * rz));
-        }
-        for (int t = 0; t < 6; ++t) vir_rcs[t] = 0;
-        vir_add(vir_rcs, rx, ry, rz, lj_rcs[0] + s.qqr2e * el_rcs[0], lj_rcs[1] + s.qqr2e * el_rcs[1],
-                lj_rcs[2] + s.qqr2e * el_rcs[2], -0.5);
-      }
-    }
-  }
-  s.fnx[i] = (lj_rs[0] + lj_rcs[0]) + s.qqr2e * (el_rs[0] + el_rcs[0]);
-  s.fny[i] = (lj_rs[1] + lj_rcs[1]) + s.qqr2e * (el_rs[1] + el_rcs[1]);
-  s.fnz[i] = (lj_rs[2] + lj_rcs[2]) + s.qqr2e * (el_rs[2] + el_rcs[2]);
-  if (s.vir_near)
-    for (int k = 0; k < 6; ++k) s.vir_near[(size_t)6 * i + k] = vir_rs[k] + vir_rcs[k];
-}
-
-// mean removal of the RBL correction force and virial (SumRBLCorrForce /
-// SumRBLCorrVirial, ExecutionMD.cpp:663-667): one workgroup sums the per-atom
-// values deterministically, then subtracts the means
-__global__ __launch_bounds__(1024) void k_rbl_mean(SysView s) {
-  __shared__ double lds[16][9];
-  double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const bool vir = s.vir_near != nullptr;
-  for (int i = threadIdx.x; i < s.n; i += blockDim.x) {
-    acc[0] += s.fnx[i];
-    acc[1] += s.fny[i];
-    acc[2] += s.fnz[i];
-    if (vir)
-      for (int k = 0; k < 6; ++k) acc[3 + k] += s.vir_near[(size_t)6 * i + k];
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int k = 0; k < 9; ++k) {
-    double t = wave_sum(acc[k]);
-    if (lane == 0) lds[wave][k] = t;
-  }
-  __syncthreads();
-  double m[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int w = 0; w < (int)(blockDim.x / 64); ++w)
-    for (int k = 0; k < 9; ++k) m[k] += lds[w][k];
-  for (int k = 0; k < 9; ++k) m[k] /= (double)s.n;
-  __syncthreads();
-  for (int i = threadIdx.x; i < s.n; i += blockDim.x) {
-    s.fnx[i] -= m[0];
-    s.fny[i] -= m[1];
-    s.fnz[i] -= m[2];
-    if (vir)
-      for (int k = 0; k < 6; ++k) s.vir_near[(size_t)6 * i + k] -= m[3 + k];
-  }
-}
-
-// RBL energies.  The reference forms them every RBL step over a full Verlet
-// list to rc (ExecutionMD::ComputeLJCoulEnergy, ExecutionMD.cpp:670-750:
-// ComputeNeighbours over the RBL locator, then LJCoulEnergyVerletVirialWorklet
-// RunWorklet.cpp:3145-3221, or SpecialLJCoulEnergyVerletWeightVirialWorklet
-// :3047-3143 with special bonds): per pair with rc^2 - d^2 > 1e-4, d^2 > 1e-4
-// on the cell-offset vector, the minimum-image vector gives
-//   e_lj   += w * 4 eps (s6/d6 - 1) s6/d6 / 2            (ComputePotentialEn_fix)
-//   e_coul += qqr2e (q q erfc(sqrt(alpha) r) / 2r - (1 - w) q q / 2r)
-// with the analytic erfc at the configured alpha (not the step table).  No
-// list is stored: one wavefront per atom walks the (2nc+1)^3 stencil around
-// the cell its current position lies in (InWhichCell, so misfit atoms need no
-// separate path), lanes over each cell's atoms.  Runs on the steps that form
-// thermo sums; its rows also carry the mean-removed RBL virial of each atom.
-template <bool WEIGHTED, bool PERATOM>
-__global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) {
-#pragma clang fp contract(off)
-  const int lane = threadIdx.x & (kWave - 1);
-  const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave);
-  double elj = 0.0, ec = 0.0;
-  double vir[6] = {0, 0, 0, 0, 0, 0};
-  if (i < s.n) {
-    const double4 pi = s.spos[i];
-    const int ti = s.stype[i];
-    int spj[kMaxSpecial];
-    double spw[kMaxSpecial];
-    if (WEIGHTED) {
-      const int id = s.point_ids[i];
-      const int b = s.sp_off[id];
-      const int spn = min(s.sp_off[id + 1] - b, kMaxSpecial);  // longer lists are refused at creation
-#pragma unroll
-      for (int k = 0; k < kMaxSpecial; ++k) {
-        spj[k] = k < spn ? s.rank[s.sp_ids[b + k]] : -1;
-        spw[k] = k < spn ? s.sp_w[b + k] : 1.0;
-      }
-    }
-    const int ca = cell_axis(pi.x, s.lo[0], s.dxdydz[0]);
-    const int cb = cell_axis(pi.y, s.lo[1], s.dxdydz[1]);
-    const int cc = cell_axis(pi.z, s.lo[2], s.dxdydz[2]);
-    const int nc = s.nc;
-    for (int a = -nc; a <= nc; ++a)
-      for (int b = -nc; b <= nc; ++b)
-        for (int e = -nc; e <= nc; ++e) {
-          const StencilCell t = stencil_cell(s, ca, cb, cc, a, b, e);
-          if (!t.ok) continue;  // an atom more than a box away: flagged by the force pass
-          for (int base = t.js; base < t.je; base += kWave) {
-            const int j = base + lane;
-            if (j >= t.je) continue;
-            const double4 pj = s.spos[j];
-            double rx = (pj.x - t.ox) - pi.x;
-            double ry = (pj.y - t.oy) - pi.y;
-            double rz = (pj.z - t.oz) - pi.z;
-            double d2 = dist2(rx, ry, rz);
-            if (!(s.cut2 - d2 > 0.0001 && d2 > 0.0001)) continue;
-            min_image(s, rx, ry, rz);  // MinDistanceVec(p_j, p_i)
-            d2 = dist2(rx, ry, rz);
-            if (!(d2 < s.cut2 && d2 > 0.0001)) continue;
-            const int tix = ti * s.ntypes + s.stype[j];
-            const double eps = s.eps_ij[tix], s6 = s.sig6_ij[tix];
-            const double d6 = d2 * d2 * d2;
-            const double el = 0.5 * (4.0 * eps * (s6 / d6 - 1.0) * (s6 / d6));
-            const double dis = sqrt(d2);
-            const double qq = pi.w * pj.w;
-            const double eco = 0.5 * qq * erfc(s.sqrt_alpha * dis) / dis;
-            double w = 1.0;
-            if (WEIGHTED) {
-#pragma unroll
-              for (int u = 0; u < kMaxSpecial; ++u)
-                if (spj[u] == j) w = spw[u];
-              elj += w * el;
-              ec += s.qqr2e * (eco - (1.0 - w) * (0.5 * qq / dis));
-            } else {
-              elj += el;
-              ec += s.qqr2e * eco;
-            }
-          }
-        }
-    elj = wave_sum(elj);
-    ec = wave_sum(ec);
-    if (lane == 0) {
-      if (PERATOM) {
-        s.e_lj[i] = elj;
-        s.e_coul[i] = ec;
-      }
-      for (int k = 0; k < 6; ++k) vir[k] = s.vir_near[(size_t)6 * i + k];
-    } else {
-      elj = ec = 0.0;
-    }
-  }
-  const double vals[kRowPair] = {elj, ec, vir[0], vir[1], vir[2], vir[3], vir[4], vir[5]};
-  block_write_row<kRowPair>(vals, rows + (size_t)blockIdx.x * kRowPair);
-}
-
-int rbl_energy_blocks(const SysView& s) { return (s.n + kBlock / kWave - 1) / (kBlock / kWave); }
-
-void launch_rbl_energy(const SysView& s, hipStream_t st, int peratom, double* rows, int* nblocks) {
-  const int grid = rbl_energy_blocks(s);
-  if (nblocks) *nblocks = grid;
-  if (s.weighted) {
-    if (peratom)
-      hipLaunchKernelGGL((k_rbl_energy<true, true>), dim3(grid), dim3(kBlock), 0, st, s, rows);
-    else
-      hipLaunchKernelGGL((k_rbl_energy<true, false>), dim3(grid), dim3(kBlock), 0, st, s, rows);
-  } else {
-    if (peratom)
-      hipLaunchKernelGGL((k_rbl_energy<false, true>), dim3(grid), dim3(kBlock), 0, st, s, rows);
-    else
-      hipLaunchKernelGGL((k_rbl_energy<false, false>), dim3(grid), dim3(kBlock), 0, st, s, rows);
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void k_static_table(const double* dis, double* g, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) g[i] = gnear_table(dis[i]);
-}
-
-void launch_static_table(const double* dis, double* g, int n, hipStream_t st) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_static_table, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, dis, g, n);
-}
-
 int pair_blocks(const SysView& s) {
-  if (s.rbl && !s.lj_only) return (s.n + kBlock - 1) / kBlock;
+  if (s.rbl) return rbl_pair_blocks(s);
   return (int)(((size_t)s.n << s.lanes_lg) + kBlock - 1) / kBlock;
 }
 
 void launch_pair(const SysView& s, hipStream_t st, int thermo, int peratom, double* rows, int* nblocks) {
   const int grid = pair_blocks(s);
   if (nblocks) *nblocks = grid;
-  if (s.rbl && !s.lj_only) {
-    if (s.weighted)
-      hipLaunchKernelGGL(k_pair_rbl<true>, dim3(grid), dim3(kBlock), 0, st, s);
-    else
-      hipLaunchKernelGGL(k_pair_rbl<false>, dim3(grid), dim3(kBlock), 0, st, s);
-    hipLaunchKernelGGL(k_rbl_mean, dim3(1), dim3(1024), 0, st, s);
+  if (s.rbl) {  // (LJ/CUT over random-batch lists is refused at creation)
+    launch_pair_rbl(s, st, thermo || peratom);
     return;
   }
   if (s.lj_only)
