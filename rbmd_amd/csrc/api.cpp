@@ -372,27 +372,21 @@ int default_cap(const rbmd_sys* s) {
   return (int)std::min<long>((long)(1.15 * f * c + 64), maxc);
 }
 
-// cap: the width the caller exports (0: default).  VERLET keeps one segment of
-// round_up(cap) slots per stencil column, so no segment can overflow below cap.
+// cap: the width the caller exports (0: default).  A VERLET row holds nine
+// times that, rounded up (a default row: nine times the fullest stencil
+// column's share), so no list overflows below cap.
 rbmd_status ensure_nbr(rbmd_sys* s, int cap) {
-  int seg_cap, nseg, export_cap;
+  int row, export_cap;
   if (s->v.rbl) {
-    nseg = 1;
     export_cap = cap > 0 ? cap : default_cap(s);
-    seg_cap = round_up(export_cap, kMaxLanes);
-    if (seg_cap < s->v.rs_num + 1) return fail(RBMD_ERR_ARG, "RBL capacity %d below the core region %d", cap, s->v.rs_num);
+    row = round_up(export_cap, kMaxLanes);
+    if (row < s->v.rs_num + 1) return fail(RBMD_ERR_ARG, "RBL capacity %d below the core region %d", cap, s->v.rs_num);
   } else {
-    nseg = 9;
-    if (cap > 0) {
-      seg_cap = round_up(cap, kMaxLanes);
-      export_cap = cap;
-    } else {
-      seg_cap = round_up(default_cap(s), kMaxLanes);
-      export_cap = nseg * seg_cap;
-    }
+    row = 9 * round_up(cap > 0 ? cap : default_cap(s), kMaxLanes);
+    export_cap = cap > 0 ? cap : row;
   }
   s->export_cap = export_cap;
-  if (s->v.nbr && seg_cap == s->v.seg_cap && nseg == s->v.nseg) return RBMD_OK;
+  if (s->v.nbr && row == s->v.cap) return RBMD_OK;
   if (s->v.nbr) {
     auto it = std::find(s->allocs.begin(), s->allocs.end(), (void*)s->v.nbr);
     if (it != s->allocs.end()) s->allocs.erase(it);
@@ -400,9 +394,7 @@ rbmd_status ensure_nbr(rbmd_sys* s, int cap) {
     (void)hipFree(s->v.nbr);
     s->v.nbr = nullptr;
   }
-  s->v.nseg = nseg;
-  s->v.seg_cap = seg_cap;
-  s->v.cap = nseg * seg_cap;
+  s->v.cap = row;
   s->graph_ok = false;
   return s->dalloc(&s->v.nbr, (size_t)s->v.cap * s->n);
 }
@@ -1094,7 +1086,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
     v.stencil_tab = dt;
   }
   A(s->dalloc(&v.stype, n));
-  A(s->dalloc(&v.nbr_num, 9 * (size_t)n));
+  A(s->dalloc(&v.nbr_num, (v.rbl ? 2 : 1) * (size_t)n));
   A(s->dalloc(&v.vir_k, 6 * (size_t)n));
   A(s->dalloc(&v.status, 1));
   if (rc == RBMD_OK) A(ensure_nbr(s, 0));
@@ -1490,7 +1482,7 @@ rbmd_status rbmd_neighbors_export(rbmd_sys* s, int32_t cap, int32_t* ids, double
   if (cap != s->export_cap) return fail(RBMD_ERR_ARG, "cap %d differs from the built width %d", cap, s->export_cap);
   int n = s->n;
   hipStream_t st = s->ctx->stream;
-  std::vector<int> nbr((size_t)s->v.cap * n), cnt(9 * (size_t)n), pid(n), rank(n);
+  std::vector<int> nbr((size_t)s->v.cap * n), cnt((s->v.rbl ? 2 : 1) * (size_t)n), pid(n), rank(n);
   HIP_TRY(hipMemcpyAsync(nbr.data(), s->v.nbr, nbr.size() * 4, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipMemcpyAsync(cnt.data(), s->v.nbr_num, cnt.size() * 4, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipMemcpyAsync(pid.data(), s->v.point_ids, n * 4, hipMemcpyDeviceToHost, st));
@@ -1520,10 +1512,8 @@ rbmd_status rbmd_neighbors_export(rbmd_sys* s, int32_t cap, int32_t* ids, double
           offsets[((size_t)a * cap + out_slot) * 3 + d] = s->v.dxdydz[d] * (double)(sh[d] * s->v.dims[d]);
     };
     if (!s->v.rbl) {
-      int out = 0;
-      for (int g = 0; g < s->v.nseg; ++g)
-        for (int k = 0; k < cnt[(size_t)g * n + i]; ++k) emit(out++, g * s->v.seg_cap + k);
-      if (num) num[a] = out;
+      for (int k = 0; k < cnt[i]; ++k) emit(k, k);
+      if (num) num[a] = cnt[i];
     } else {
       for (int k = 0; k < cnt[2 * i]; ++k) emit(k, k);
       for (int k = 0; k < cnt[2 * i + 1]; ++k) emit(s->v.rs_num + k, s->v.rs_num + k);
@@ -1546,7 +1536,7 @@ rbmd_status rbmd_neighbors_capacity(const rbmd_sys* s, int32_t* cap) {
 rbmd_status rbmd_neighbors_count(rbmd_sys* s, int64_t* entries) {
   if (!s || !entries) return fail(RBMD_ERR_ARG, "bad arguments");
   if (!s->nbr_built) return fail(RBMD_ERR_STATE, "neighbour lists not built");
-  int m = s->v.rbl ? 2 * s->n : s->v.nseg * s->n;
+  int m = s->v.rbl ? 2 * s->n : s->n;
   std::vector<int> cnt(m);
   HIP_TRY(hipMemcpyAsync(cnt.data(), s->v.nbr_num, (size_t)m * 4, hipMemcpyDeviceToHost, s->ctx->stream));
   HIP_TRY(hipStreamSynchronize(s->ctx->stream));

@@ -9,12 +9,6 @@ namespace rbmd {
 constexpr int kMisfitBlocks = 64;  // workgroups that take the misfit atoms
 constexpr int kColWaves = 9;        // stencil columns of the VERLET list build
 constexpr int kScanScatterCells = 2048;  // most cells for the one-launch scan + scatter
-constexpr int kNbrWaves = 3;        // columns (wavefronts) per list-build workgroup
-constexpr int kNbrParts = kColWaves / kNbrWaves;  // list-build workgroups per work item
-constexpr int kStageRounds = 2;    // 64-candidate rounds staged per list-build batch
-constexpr int kStageCap = kStageRounds * 64;  // staged candidates per wavefront (one batch)
-constexpr int kListRing = 8;        // list-build LDS ring of accepted entries per lane (two groups of four)
-constexpr int kListRingStride = 9;  // words between two lanes' rings (odd: distinct banks)
 
 // InWhichCell (ExecPointLocator.h:271-274): unclamped trunc
 __device__ __forceinline__ int cell_axis(double x, double lo, double d) {
@@ -138,21 +132,6 @@ __device__ __forceinline__ void column_candidate(const SysView& s, int t, int n0
   pj = make_double4(p.x - ox, p.y - oy, p.z - oz, p.w);
   entry = (j << kShiftBits) | code;
 }
-
-// where candidate t of a column stream lives, without loading it: its sorted
-// index, packed entry and z image offset (x and y are the column's), so a
-// caller can issue several loads back to back before using any of them
-__device__ __forceinline__ int column_locate(int t, int n0, int n01, int jb0, int jb1, int jb2, int c0, int c1,
-                                             int c2, double oz0, double oz1, double oz2, int& entry, double& oz) {
-  const bool q1 = t >= n0, q2 = t >= n01;
-  const int j = t + (q2 ? jb2 : (q1 ? jb1 : jb0));
-  oz = q2 ? oz2 : (q1 ? oz1 : oz0);
-  entry = (j << kShiftBits) | (q2 ? c2 : (q1 ? c1 : c0));
-  return j;
-}
-
-#define COLUMN_LOCATE(t, entry, oz) \
-  column_locate(t, col.n0, col.n01, col.jb0, col.jb1, col.jb2, col.c0, col.c1, col.c2, col.oz0, col.oz1, col.oz2, entry, oz)
 
 #define COLUMN_CANDIDATE(t, pj, entry)                                                                             \
   column_candidate(s, t, col.n0, col.n01, col.jb0, col.jb1, col.jb2, col.c0, col.c1, col.c2, col.ox, col.oy, \

@@ -46,9 +46,7 @@ struct SysView {
   int ncell;        // dims0*dims1*dims2
   int dims[3];
   int nc;           // stencil half width (ceil(rc / rs))
-  int cap;          // neighbour-list slots per atom (VERLET: nseg * seg_cap)
-  int nseg;         // VERLET: one list segment per (x, y) column of the 3x3x3 stencil (9); RBL: 1
-  int seg_cap;      // slots per segment (multiple of the lane count)
+  int cap;          // neighbour-list slots per atom
   int lanes_lg;     // log2 of the lanes per atom in the pair kernel (2..4)
   int compact;      // few atoms: steps without thermo sums take the stencil pair kernel, without a stored list
   int st_cfg;       // compact: how the stencil pair kernel splits the work (stencil_choice)
@@ -111,7 +109,7 @@ struct SysView {
   // neighbour lists, column-major [cap][n] of packed (j_sorted << 9 | shift code)
   int* nbr;         // layout nbr_index(slot, i, cap): one row per atom
   int lds_bins;     // binning kernels aggregate counts in LDS (ncell small enough)
-  int* nbr_num;     // VERLET [nseg][n] counts per segment; RBL [2n] (core, shell kept)
+  int* nbr_num;     // VERLET [n]; RBL [2n] (core, shell kept)
   // per-atom force components (original order)
   double *fnx, *fny, *fnz;  // real space, sorted order, [nslab][n] partials added in order
   double *fkx, *fky, *fkz;  // k space
@@ -219,6 +217,7 @@ void launch_rbl_energy(const SysView& s, hipStream_t st, int peratom, double* ro
 int rbl_energy_blocks(const SysView& s);
 // random-batch lists; the corrected pair force with its means removed (and its virial)
 void launch_nbr_build_rbl(const SysView& s, hipStream_t st);
+int list_blocks(const SysView& s);
 void launch_pair_rbl(const SysView& s, hipStream_t st, int virial);
 int rbl_pair_blocks(const SysView& s);
 // the RBL erfc step table at n distances (device arrays)
@@ -413,6 +412,7 @@ struct PackSig {  // launch-wide choices, equal for every system of a pack
 // (+8: reduce the thermo rows), PK_FIRST_HALF 1 = apply the NHC scale,
 // PK_SECOND the kick flag, PK_ONE 0 = zero the SHAKE iteration counters,
 // 1 = copy every status word to out[k].
+void launch_pack_list(const PackLaunch& L, int nblocks, hipStream_t st);
 void launch_pack_cells(int kernel, const PackLaunch& L, int nblocks, size_t lds, hipStream_t st);
 void launch_pack_pair(const PackLaunch& L, int nblocks, const PackSig& g, hipStream_t st);
 int pack_ewald_blocks(const EwView& v, int kernel);

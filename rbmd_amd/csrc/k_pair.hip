@@ -25,7 +25,6 @@
 
 namespace rbmd {
 
-constexpr int kMaxSeg = 9;  // VERLET list segments per atom (stencil columns)
 
 // Raw buffer loads (32-bit byte offsets from a wave-uniform base, bounds
 // checked by the hardware: a load past num_records returns zeros).  The pair
@@ -47,32 +46,18 @@ __device__ __forceinline__ int buf_int(BufRsrc r, unsigned off) {
   return (int)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
 }
 
-// A lane's position in an atom's concatenated segments: `seg` (nseg past the
-// end), the offset in it, its length (INT_MAX past the end) and the byte
-// offset of the segment's start from the wavefront's first list row.
+// A lane's position in an atom's list: its length and the byte offset of the
+// row from the wavefront's first one.
 struct ListCursor {
-  int seg, off, num;
+  int off, num;
   unsigned po;
 };
 
-// entry at the cursor (0 past the end: a list entry is never 0, its image
-// code is at least 2 + (2 << 3) + (2 << 6)), then one stride forward; crossing
-// into the next segment is the rare path.  seg_cnt: the workgroup's segment
-// counts in LDS, one column per thread, so a crossing reads the next count at
-// an address computed from the segment index.
-__device__ __forceinline__ int cursor_take(ListCursor& c, BufRsrc rows, const int (&seg_cnt)[kMaxSeg][kBlock],
-                                           int nseg, int seg_cap, int stride) {
-  if (__builtin_expect(c.off >= c.num, 0)) {
-    do {
-      c.off -= c.num;
-      ++c.seg;
-      // past the last segment the offset lies beyond the buffer (2^31 and
-      // more), where loads return 0
-      c.po = c.seg < nseg ? c.po + 4u * (unsigned)seg_cap : 0x80000000u;
-      c.num = c.seg < nseg ? seg_cnt[c.seg][threadIdx.x] : 0x7fffffff;
-    } while (c.off >= c.num);
-  }
-  const int e = buf_int(rows, c.po + 4u * (unsigned)c.off);
+// entry at the cursor, then one stride forward; past the end the offset lies
+// beyond the buffer, where loads return 0 (a list entry is never 0, its image
+// code is at least 2 + (2 << 3) + (2 << 6))
+__device__ __forceinline__ int cursor_take(ListCursor& c, BufRsrc rows, int stride) {
+  const int e = buf_int(rows, c.off < c.num ? c.po + 4u * (unsigned)c.off : 0x80000000u);
   c.off += stride;
   return e;
 }
@@ -96,7 +81,6 @@ __device__ __forceinline__ void pair_verlet_body(const SysView& s, double* rows,
   constexpr int kTab = F32 ? kCoulTab32 : kCoulTab;
   __shared__ TT teps[LTAB ? kMaxTypes * kMaxTypes : 1], tsig[LTAB ? kMaxTypes * kMaxTypes : 1];
   __shared__ CT ctab[MODE == 2 ? 1 : kTab];
-  __shared__ int seg_cnt[kMaxSeg][kBlock];  // each thread's list segment counts (one column per thread)
   const int nt = s.ntypes;
   if (LTAB)
     for (int k = threadIdx.x; k < nt * nt; k += blockDim.x) {
@@ -139,10 +123,6 @@ __device__ __forceinline__ void pair_verlet_body(const SysView& s, double* rows,
         spw[k] = k < spn ? s.sp_w[b + k] : 1.0;
       }
     }
-#pragma unroll
-    for (int g = 0; g < kMaxSeg; ++g) seg_cnt[g][threadIdx.x] = g < s.nseg ? s.nbr_num[g * s.n + i] : 0;
-    const int cnt0 = s.nseg > 0 ? s.nbr_num[i] : 0;
-    const int nseg = s.nseg, seg_cap = s.seg_cap;
     // the wavefront's list rows (its 64 / L atoms, fewer in the last one)
     // and the sorted positions and types as buffers
     const int i0 = __builtin_amdgcn_readfirstlane(i);
@@ -150,10 +130,10 @@ __device__ __forceinline__ void pair_verlet_body(const SysView& s, double* rows,
     const BufRsrc rrows = buf_rsrc(s.nbr + (size_t)i0 * s.cap, 4u * (unsigned)s.cap * (unsigned)rows_here);
     const BufRsrc rpos = buf_rsrc(s.spos, 32u * (unsigned)s.n);
     const BufRsrc rtyp = buf_rsrc(s.stype, 4u * (unsigned)s.n);
-    ListCursor cur{0, sub, cnt0, 4u * (unsigned)(i - i0) * (unsigned)s.cap};
+    ListCursor cur{sub, s.nbr_num[i], 4u * (unsigned)(i - i0) * (unsigned)s.cap};
     // pipeline: entries two iterations ahead, positions one iteration ahead
-    int ea = cursor_take(cur, rrows, seg_cnt, nseg, seg_cap, L);
-    int eb = cursor_take(cur, rrows, seg_cnt, nseg, seg_cap, L);
+    int ea = cursor_take(cur, rrows, L);
+    int eb = cursor_take(cur, rrows, L);
     // an entry's neighbour as a byte offset into the positions (0 past the
     // end: atom 0, loaded and not used)
     auto jof = [](int e) -> unsigned { return (unsigned)e >> kShiftBits; };
@@ -161,15 +141,15 @@ __device__ __forceinline__ void pair_verlet_body(const SysView& s, double* rows,
     double4 pb = buf_double4(rpos, 32u * jof(eb));
     int ta = buf_int(rtyp, 4u * jof(ea));
     int tb = buf_int(rtyp, 4u * jof(eb));
-    int na = cursor_take(cur, rrows, seg_cnt, nseg, seg_cap, L);
-    int nb = cursor_take(cur, rrows, seg_cnt, nseg, seg_cap, L);
+    int na = cursor_take(cur, rrows, L);
+    int nb = cursor_take(cur, rrows, L);
     while (ea > 0) {
       const double4 qa = buf_double4(rpos, 32u * jof(na));
       const double4 qb = buf_double4(rpos, 32u * jof(nb));
       const int ua = buf_int(rtyp, 4u * jof(na));
       const int ub = buf_int(rtyp, 4u * jof(nb));
-      const int ma = cursor_take(cur, rrows, seg_cnt, nseg, seg_cap, L);
-      const int mb = cursor_take(cur, rrows, seg_cnt, nseg, seg_cap, L);
+      const int ma = cursor_take(cur, rrows, L);
+      const int mb = cursor_take(cur, rrows, L);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int e = h == 0 ? ea : eb;

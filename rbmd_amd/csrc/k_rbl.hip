@@ -29,6 +29,7 @@
 #include "dev.hpp"
 #include "pair.hpp"
 #include "reduce.hpp"
+#include "stream.hpp"
 
 namespace rbmd {
 
@@ -36,70 +37,7 @@ constexpr int kRblWaves = kBlock / kWave;
 constexpr int kRblAtoms = 8;                                        // atoms per wavefront, at most
 constexpr int kRblParts = kChunk / (kRblWaves * kRblAtoms);         // workgroups per 64-atom work item
 constexpr int kRblCells = 128;                                      // stencil cells per table (two per lane)
-
-struct RblTable {
-  int pre[kRblCells], jb[kRblCells], code[kRblCells];
-};
-
-// The stencil cells c0 .. c0 + 127 around cell (ca, cb, cc) into the table;
-// returns the number of their candidates.  shifts: some image offset is not
-// zero; bad: status bit of a stencil cell out of reach.  One wavefront.
-__device__ __forceinline__ int rbl_table(const SysView& s, int ca, int cb, int cc, int c0, RblTable& tab, int bad,
-                                         bool& shifts) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wd = 2 * s.nc + 1, cells = wd * wd * wd;
-  int js[2] = {0, 0}, num[2] = {0, 0}, code[2];
-  code[0] = code[1] = pack_entry(0, 0, 0, 0);
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int k = c0 + 2 * lane + u;
-    if (k < cells) {
-      const StencilCell t = stencil_cell(s, ca, cb, cc, k / (wd * wd) - s.nc, (k / wd) % wd - s.nc, k % wd - s.nc);
-      if (t.ok) {
-        js[u] = t.js;
-        num[u] = t.je - t.js;
-        code[u] = pack_entry(0, t.sa, t.sb, t.sc);
-      } else {
-        atomicOr(s.status, bad);
-      }
-    }
-  }
-  int inc = num[0] + num[1];
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const int t = __shfl_up(inc, off, kWave);
-    if (lane >= off) inc += t;
-  }
-  const int p0 = inc - num[0] - num[1], p1 = p0 + num[0];
-  tab.pre[2 * lane] = p0;
-  tab.pre[2 * lane + 1] = p1;
-  tab.jb[2 * lane] = js[0] - p0;
-  tab.jb[2 * lane + 1] = js[1] - p1;
-  tab.code[2 * lane] = code[0];
-  tab.code[2 * lane + 1] = code[1];
-  shifts = __ballot(code[0] != pack_entry(0, 0, 0, 0) || code[1] != pack_entry(0, 0, 0, 0)) != 0ull;
-  return __builtin_amdgcn_readlane(inc, kWave - 1);
-}
-
-// candidate t (< total) of a table: its entry
-__device__ __forceinline__ int rbl_entry(const RblTable& tab, int t) {
-  int k = 0;
-#pragma unroll
-  for (int step = kRblCells / 2; step > 0; step >>= 1) k += tab.pre[k + step] <= t ? step : 0;
-  return ((t + tab.jb[k]) << kShiftBits) | tab.code[k];
-}
-
-// an entry's position less its image offset (w: charge)
-__device__ __forceinline__ double4 rbl_position(const SysView& s, int e, bool shifts) {
-#pragma clang fp contract(off)
-  double4 p = s.spos[e >> kShiftBits];
-  if (shifts) {
-    p.x -= s.dxdydz[0] * (double)(((e & 7) - 3) * s.dims[0]);
-    p.y -= s.dxdydz[1] * (double)((((e >> 3) & 7) - 3) * s.dims[1]);
-    p.z -= s.dxdydz[2] * (double)((((e >> 6) & 7) - 3) * s.dims[2]);
-  }
-  return p;
-}
+using RblTable = StreamTable<kRblCells>;
 
 // Candidates staged for a workgroup: positions less the image offset, entries
 constexpr int kRblStage = 512;
@@ -122,7 +60,7 @@ __device__ __forceinline__ void rbl_stream_shared(const SysView& s, int c, bool 
     __syncthreads();  // the last table's reads
     if (threadIdx.x < kWave) {
       bool shifts;
-      const int total = rbl_table(s, ca, cb, cc, c0, tab, 4, shifts);
+      const int total = stream_table(s, s.nc, ca, cb, cc, c0, tab, 4, shifts);
       if (lane == 0) {
         shared_int[0] = total;
         shared_int[1] = shifts ? 1 : 0;
@@ -135,8 +73,8 @@ __device__ __forceinline__ void rbl_stream_shared(const SysView& s, int c, bool 
       const int m = min(kRblStage, total - base);
       if (base > 0) __syncthreads();  // the last stage's reads
       for (int t = threadIdx.x; t < m; t += kBlock) {
-        const int e = rbl_entry(tab, base + t);
-        const double4 p = rbl_position(s, e, shifts);
+        const int e = stream_entry(tab, base + t);
+        const double4 p = stream_position(s, e, shifts);
         stage.x[t] = p.x;
         stage.y[t] = p.y;
         stage.z[t] = p.z;
@@ -148,30 +86,6 @@ __device__ __forceinline__ void rbl_stream_shared(const SysView& s, int c, bool 
           const int t = t0 + lane;  // past m: an earlier window's candidate, dead
           f(t < m, stage.e[t], stage.x[t], stage.y[t], stage.z[t]);
         }
-    }
-  }
-}
-
-// the same for one wavefront and any cell (misfit atoms)
-template <class F>
-__device__ __forceinline__ void rbl_stream(const SysView& s, int ca, int cb, int cc, RblTable& tab, F&& f) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wd = 2 * s.nc + 1, cells = wd * wd * wd;
-  for (int c0 = 0; c0 < cells; c0 += kRblCells) {
-    bool shifts;
-    wave_sync();  // the last table's reads
-    const int total = rbl_table(s, ca, cb, cc, c0, tab, 1, shifts);  // more than a box away: status bit 0
-    wave_sync();
-    if (total == 0) continue;
-    // the next batch's positions are in flight over this one's tests
-    int e = rbl_entry(tab, min(lane, total - 1));
-    double4 p = rbl_position(s, e, shifts);
-    for (int base = 0; base < total; base += kWave) {
-      const int en = rbl_entry(tab, min(base + kWave + lane, total - 1));
-      const double4 pn = rbl_position(s, en, shifts);
-      f(base + lane < total, e, p.x, p.y, p.z);
-      e = en;
-      p = pn;
     }
   }
 }
@@ -194,13 +108,6 @@ __device__ __forceinline__ bool rbl_atoms(const SysView& s, int bid, int& c, int
   return bid % kRblParts < parts;
 }
 
-__device__ __forceinline__ int rbl_below(unsigned long long m) {
-  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-}
-
-// this lane's bit of a ballot, as the condition of a branch
-__device__ __forceinline__ bool rbl_in(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
-
 // One atom's list: core slots [0, rs_num), kept shell slots from rs_num, every
 // pice_num-th shell atom in traversal order.  The shell atoms of a batch are a
 // ballot; among them, the kept ones are those whose prefix count is a set bit
@@ -215,9 +122,6 @@ __device__ __forceinline__ unsigned long long rbl_multiples(int pice) {
   for (int r = 0; r < kWave; r += pice) m |= 1ull << r;
   return m;
 }
-__device__ __forceinline__ void rbl_store(int* row, int slot, int entry) {
-  *(int*)((char*)row + 4u * (unsigned)slot) = entry;  // a row is far below 2^32 bytes
-}
 __device__ __forceinline__ void rbl_consider(const SysView& s, RblList& L, int i, int entry, double d2, int pice,
                                              unsigned long long multiples) {
 #pragma clang fp contract(off)
@@ -227,16 +131,16 @@ __device__ __forceinline__ void rbl_consider(const SysView& s, RblList& L, int i
   int* const row = s.nbr + nbr_index(0, i, s.cap);
   if (~far != 0ull) {  // wave-uniform
     const unsigned long long bc = __ballot(-e > 0.0001) & __ballot(d2 > 0.0001);
-    const int slot = L.core + rbl_below(bc);
-    if (rbl_in(bc) & (slot < s.rs_num)) rbl_store(row, slot, entry);
+    const int slot = L.core + lanes_below(bc);
+    if (lane_in(bc) & (slot < s.rs_num)) row_store(row, slot, entry);
     L.core += __popcll(bc);
   }
   const int num = __popcll(bs);
   if (L.wait < num) {  // wave-uniform; wait < 64 here
     const unsigned long long pick = multiples << L.wait;
-    const unsigned long long bk = bs & __ballot((pick >> rbl_below(bs)) & 1ull);
-    const int slot = s.rs_num + L.kept + rbl_below(bk);
-    if (rbl_in(bk) & (slot < s.cap)) rbl_store(row, slot, entry);
+    const unsigned long long bk = bs & __ballot((pick >> lanes_below(bs)) & 1ull);
+    const int slot = s.rs_num + L.kept + lanes_below(bk);
+    if (lane_in(bk) & (slot < s.cap)) row_store(row, slot, entry);
     const int kept = __popcll(bk);
     L.kept += kept;
     L.wait += kept * pice;
@@ -269,8 +173,8 @@ __global__ __launch_bounds__(kBlock) void k_nbr_build_rbl(SysView s) {
       const int i = __builtin_amdgcn_readfirstlane(s.misfit_list[m]);
       const double4 pi = s.spos[i];
       RblList L = {0, 0, 0};
-      rbl_stream(s, cell_axis(pi.x, s.lo[0], s.dxdydz[0]), cell_axis(pi.y, s.lo[1], s.dxdydz[1]),
-                 cell_axis(pi.z, s.lo[2], s.dxdydz[2]), tabs[w],
+      wave_stream(s, s.nc, cell_axis(pi.x, s.lo[0], s.dxdydz[0]), cell_axis(pi.y, s.lo[1], s.dxdydz[1]),
+                 cell_axis(pi.z, s.lo[2], s.dxdydz[2]), tabs[w], 1,
                  [&](bool live, int entry, double x, double y, double z) {
                    if (!live) x = __builtin_nan("");
                    rbl_consider(s, L, i, entry, dist2(x - pi.x, y - pi.y, z - pi.z), pice, multiples);
@@ -579,7 +483,7 @@ __global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) 
       const int n = min(cnt, kWave);
       cnt -= n;
       const int2 q = queue[w][cnt + (lane < n ? lane : 0)];
-      const double4 p = rbl_position(s, q.y, true), pa = atom[w][q.x];
+      const double4 p = stream_position(s, q.y, true), pa = atom[w][q.x];
       const int j = q.y >> kShiftBits;
       double rx = p.x - pa.x, ry = p.y - pa.y, rz = p.z - pa.z;
       min_image(s, rx, ry, rz);  // MinDistanceVec(p_j, p_i)
@@ -619,7 +523,7 @@ __global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) 
     };
     auto push = [&](int a, double d2, int entry) __attribute__((always_inline)) {
       const unsigned long long b = __ballot(d2 <= s.accept_d2) & __ballot(d2 > 0.0001);
-      if (rbl_in(b)) queue[w][cnt + rbl_below(b)] = make_int2(a, entry);
+      if (lane_in(b)) queue[w][cnt + lanes_below(b)] = make_int2(a, entry);
       cnt += __popcll(b);
       if (PERATOM ? cnt > 0 : cnt >= kWave) drain();  // wave-uniform
     };
@@ -637,8 +541,8 @@ __global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) 
       const int a = __builtin_ctz(todo);
       todo &= todo - 1;
       const double4 pa = atom[w][a];
-      rbl_stream(s, cell_axis(pa.x, s.lo[0], s.dxdydz[0]), cell_axis(pa.y, s.lo[1], s.dxdydz[1]),
-                 cell_axis(pa.z, s.lo[2], s.dxdydz[2]), tabs[w],
+      wave_stream(s, s.nc, cell_axis(pa.x, s.lo[0], s.dxdydz[0]), cell_axis(pa.y, s.lo[1], s.dxdydz[1]),
+                 cell_axis(pa.z, s.lo[2], s.dxdydz[2]), tabs[w], 1,
                  [&](bool live, int entry, double x, double y, double z) {
                    if (!live) x = __builtin_nan("");
                    push(a, dist2(x - pa.x, y - pa.y, z - pa.z), entry);
