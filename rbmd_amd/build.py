@@ -18,7 +18,7 @@ LIB = os.path.join(OUT, "librbmd_mi355x.so")
 ARCH = os.environ.get("RBMD_OFFLOAD_ARCH", "gfx950")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-SOURCES = ["k_cells.hip", "k_list.hip", "k_force.hip", "k_pair.hip", "k_stencil.hip", "k_rbl.hip", "k_kspace.hip", "k_ewald.hip", "k_integrate.hip", "noalloc.hip", "api.cpp", "sampler.cpp"]
+SOURCES = ["k_cells.hip", "k_list.hip", "k_force.hip", "k_pair.hip", "k_stencil.hip", "k_rbl.hip", "k_kspace.hip", "k_ewald.hip", "k_integrate.hip", "k_transfer.hip", "noalloc.hip", "api.cpp", "sampler.cpp"]
 # matrix instructions accumulate in vector registers (their sums are read by
 # vector instructions right after)
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1"]

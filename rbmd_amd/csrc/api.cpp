@@ -216,6 +216,14 @@ struct rbmd_sys {
   bool locator_built = false, nbr_built = false, initialized = false;
   double e_long = 0;
   int64_t energy_step = -1;
+  // pinned staging of the caller's arrays: two halves in turn, each with the
+  // event of the last device work on it, and the small results
+  char* pin[2] = {nullptr, nullptr};
+  hipEvent_t pin_ev[2] = {nullptr, nullptr};
+  size_t pin_bytes = 0;  // of a half
+  int pin_next = 0;
+  ThermoOut* small = nullptr;
+  double* bond_rows = nullptr;
   int64_t step = 0;
   std::vector<int> host_angles;
 
@@ -436,8 +444,141 @@ rbmd_status prepare_skin(rbmd_sys* s) {
 }
 
 rbmd_status read_status(rbmd_sys* s, int* st) {
-  HIP_TRY(hipMemcpyAsync(st, s->v.status, sizeof(int), hipMemcpyDeviceToHost, s->ctx->stream));
+  HIP_TRY(hipMemcpyAsync(&s->small->status, s->v.status, sizeof(int), hipMemcpyDeviceToHost, s->ctx->stream));
   HIP_TRY(hipStreamSynchronize(s->ctx->stream));
+  *st = s->small->status;
+  return RBMD_OK;
+}
+
+// staging for n atoms: all arrays of a call for small systems (21 doubles a
+// state), parts of 1 MiB for large ones
+constexpr size_t kPinMost = size_t(1) << 20;
+rbmd_status pin_create(rbmd_sys* s) {
+  s->pin_bytes = std::min(kPinMost, std::max<size_t>(4096, (size_t)s->n * 12 * sizeof(double)));
+  for (int h = 0; h < 2; ++h) {
+    if (hipHostMalloc((void**)&s->pin[h], s->pin_bytes) != hipSuccess) return fail(RBMD_ERR_OOM, "hipHostMalloc staging");
+    if (hipEventCreateWithFlags(&s->pin_ev[h], hipEventDisableTiming) != hipSuccess)
+      return fail(RBMD_ERR_HIP, "hipEventCreate");
+  }
+  const size_t rows = (size_t)((s->n + kBlock - 1) / kBlock) * kRowBond;
+  if (hipHostMalloc((void**)&s->small, sizeof(ThermoOut) + rows * sizeof(double)) != hipSuccess)
+    return fail(RBMD_ERR_OOM, "hipHostMalloc staging");
+  s->bond_rows = (double*)(s->small + 1);
+  return RBMD_OK;
+}
+
+void pin_destroy(rbmd_sys* s) {
+  for (int h = 0; h < 2; ++h) {
+    if (s->pin[h]) (void)hipHostFree(s->pin[h]);
+    if (s->pin_ev[h]) (void)hipEventDestroy(s->pin_ev[h]);
+  }
+  if (s->small) (void)hipHostFree(s->small);
+}
+
+// Arrays of a call, as fields of a transfer and the caller's side of each
+struct Transfer {
+  TransferDesc d{};
+  char* user[kTransferFields];
+  Transfer(rbmd_sys* s) { d.n = s->n; }
+  TransferField& add(const void* host, int width) {
+    TransferField& f = d.field[d.nfield];
+    user[d.nfield++] = (char*)host;
+    f.width = width;
+    f.first = d.width;
+    f.slabs = 1;
+    d.width += width;
+    return f;
+  }
+  // an array per component
+  void split(const void* host, double* x, double* y, double* z, int slabs = 1, const int* rank = nullptr) {
+    if (!host) return;
+    TransferField& f = add(host, 3);
+    f.p[0] = x;
+    f.p[1] = y;
+    f.p[2] = z;
+    f.split = 1;
+    f.slabs = slabs;
+    f.rank = rank;
+  }
+  // records of `width` doubles
+  void records(const void* host, double* p, int width, int slabs = 1, const int* rank = nullptr) {
+    if (!host) return;
+    TransferField& f = add(host, width);
+    f.p[0] = p;
+    f.slabs = slabs;
+    f.rank = rank;
+  }
+  // records of three whole numbers
+  void ints(const void* host, int* p) {
+    if (!host) return;
+    TransferField& f = add(host, 3);
+    f.p[0] = (double*)p;
+    f.is_int = 1;
+  }
+  size_t bytes(int f, int atoms) const { return (size_t)d.field[f].width * atoms * (d.field[f].is_int ? 4 : 8); }
+  // between the caller's arrays and a half, atoms a0 .. a0 + atoms - 1
+  void host_copy(char* pin, int a0, int atoms, bool out) {
+    for (int f = 0; f < d.nfield; ++f) {
+      char* mine = pin + (size_t)d.field[f].first * atoms * 8;
+      char* theirs = user[f] + bytes(f, a0);
+      if (out)
+        std::memcpy(theirs, mine, bytes(f, atoms));
+      else
+        std::memcpy(mine, theirs, bytes(f, atoms));
+    }
+  }
+};
+
+// The caller's arrays to the device.  Returns with the last parts' kernels in
+// the stream (the caller's memory has been read).
+rbmd_status transfer_in(rbmd_sys* s, Transfer& t) {
+  if (t.d.width == 0 || s->n <= 0) return RBMD_OK;
+  const int per = (int)(s->pin_bytes / (8 * (size_t)t.d.width));
+  for (int a0 = 0; a0 < s->n; a0 += per) {
+    const int h = s->pin_next;
+    s->pin_next ^= 1;
+    t.d.a0 = a0;
+    t.d.atoms = std::min(per, s->n - a0);
+    t.d.host = (double*)s->pin[h];
+    HIP_TRY(hipEventSynchronize(s->pin_ev[h]));
+    t.host_copy(s->pin[h], a0, t.d.atoms, false);
+    launch_transfer(t.d, false, s->ctx->stream);
+    HIP_TRY(hipEventRecord(s->pin_ev[h], s->ctx->stream));
+  }
+  return check_launch("transfer_in");
+}
+
+// Device arrays to the caller's, and the status flags with them: the device
+// writes one half while the host reads the other.
+rbmd_status transfer_out(rbmd_sys* s, Transfer& t, int* status = nullptr) {
+  hipStream_t st = s->ctx->stream;
+  if (status)
+    HIP_TRY(hipMemcpyAsync(&s->small->status, s->v.status, sizeof(int), hipMemcpyDeviceToHost, st));
+  if (t.d.width > 0 && s->n > 0) {
+    const int per = (int)(s->pin_bytes / (8 * (size_t)t.d.width));
+    const int parts = (s->n + per - 1) / per;
+    int half[2];
+    for (int k = 0; k <= parts; ++k) {
+      if (k < parts) {
+        const int h = half[k & 1] = s->pin_next;
+        s->pin_next ^= 1;
+        t.d.a0 = k * per;
+        t.d.atoms = std::min(per, s->n - t.d.a0);
+        t.d.host = (double*)s->pin[h];
+        launch_transfer(t.d, true, st);
+        HIP_TRY(hipEventRecord(s->pin_ev[h], st));
+      }
+      if (k > 0) {
+        const int a0 = (k - 1) * per, h = half[(k - 1) & 1];
+        HIP_TRY(hipEventSynchronize(s->pin_ev[h]));
+        t.host_copy(s->pin[h], a0, std::min(per, s->n - a0), true);
+      }
+    }
+    RC_TRY(check_launch("transfer_out"));
+  } else {
+    HIP_TRY(hipStreamSynchronize(st));
+  }
+  if (status) *status = s->small->status;
   return RBMD_OK;
 }
 
@@ -685,11 +826,17 @@ constexpr int64_t kEwTablesSmall = int64_t(14) << 20, kEwPartialsSmall = int64_t
 
 // the grid sum from the energy rows of the weight pass
 rbmd_status ewald_grid_sum(rbmd_sys* s, const EwView& v, double* sum) {
-  std::vector<double> e(ewald_energy_rows(v));
-  HIP_TRY(hipMemcpyAsync(e.data(), v.erow, e.size() * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream));
-  HIP_TRY(hipStreamSynchronize(s->ctx->stream));
+  const size_t rows = ewald_energy_rows(v), most = s->pin_bytes / sizeof(double);
+  const int h = s->pin_next;
+  s->pin_next ^= 1;
   double t = 0;
-  for (double x : e) t += x;
+  for (size_t r = 0; r < rows; r += most) {
+    const size_t len = std::min(most, rows - r);
+    HIP_TRY(hipMemcpyAsync(s->pin[h], v.erow + r, len * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream));
+    HIP_TRY(hipStreamSynchronize(s->ctx->stream));
+    const double* e = (const double*)s->pin[h];
+    for (size_t k = 0; k < len; ++k) t += e[k];
+  }
   *sum = t;
   return RBMD_OK;
 }
@@ -1287,6 +1434,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
       }
     }
   }
+  A(pin_create(s));
   if (rc != RBMD_OK) {
     rbmd_sys_destroy(s);
     return rc;
@@ -1362,6 +1510,7 @@ rbmd_status rbmd_sys_destroy(rbmd_sys* s) {
     if (s->stage[h]) (void)hipHostFree(s->stage[h]);
     if (s->stage_ev[h]) (void)hipEventDestroy(s->stage_ev[h]);
   }
+  pin_destroy(s);
   (void)hipEventDestroy(s->ev_fork);
   (void)hipEventDestroy(s->ev_join);
   delete s;
@@ -1376,27 +1525,11 @@ rbmd_status rbmd_sys_footprint(const rbmd_sys* s, int64_t* bytes) {
 
 rbmd_status rbmd_sys_upload_state(rbmd_sys* s, const double* x, const double* v, const int32_t* image) {
   if (!s) return fail(RBMD_ERR_ARG, "null sys");
-  int n = s->n;
-  std::vector<double> a(n), b(n), c(n);
-  hipStream_t st = s->ctx->stream;
-  auto put = [&](const double* src, double* dx, double* dy, double* dz) -> rbmd_status {
-    for (int i = 0; i < n; ++i) {
-      a[i] = src[3 * i];
-      b[i] = src[3 * i + 1];
-      c[i] = src[3 * i + 2];
-    }
-    HIP_TRY(hipMemcpyAsync(dx, a.data(), n * 8, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(dy, b.data(), n * 8, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(dz, c.data(), n * 8, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    return RBMD_OK;
-  };
-  if (x) RC_TRY(put(x, s->v.x, s->v.y, s->v.z));
-  if (v) RC_TRY(put(v, s->v.vx, s->v.vy, s->v.vz));
-  if (image) {
-    HIP_TRY(hipMemcpyAsync(s->v.img, image, (size_t)3 * n * 4, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
-  }
+  Transfer t(s);
+  t.split(x, s->v.x, s->v.y, s->v.z);
+  t.split(v, s->v.vx, s->v.vy, s->v.vz);
+  t.ints(image, s->v.img);
+  RC_TRY(transfer_in(s, t));
   s->locator_built = s->nbr_built = false;
   s->skin_ready = false;  // a skin list is rebuilt on the next step
   return RBMD_OK;
@@ -1404,29 +1537,12 @@ rbmd_status rbmd_sys_upload_state(rbmd_sys* s, const double* x, const double* v,
 
 rbmd_status rbmd_sys_download_state(rbmd_sys* s, double* x, double* v, double* f, int32_t* image) {
   if (!s) return fail(RBMD_ERR_ARG, "null sys");
-  int n = s->n;
-  hipStream_t st = s->ctx->stream;
-  std::vector<double> a(n), b(n), c(n);
-  auto get = [&](double* dst, const double* dx, const double* dy, const double* dz) -> rbmd_status {
-    HIP_TRY(hipMemcpyAsync(a.data(), dx, n * 8, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(b.data(), dy, n * 8, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(c.data(), dz, n * 8, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    for (int i = 0; i < n; ++i) {
-      dst[3 * i] = a[i];
-      dst[3 * i + 1] = b[i];
-      dst[3 * i + 2] = c[i];
-    }
-    return RBMD_OK;
-  };
-  if (x) RC_TRY(get(x, s->v.x, s->v.y, s->v.z));
-  if (v) RC_TRY(get(v, s->v.vx, s->v.vy, s->v.vz));
-  if (f) RC_TRY(get(f, s->v.fx, s->v.fy, s->v.fz));
-  if (image) {
-    HIP_TRY(hipMemcpyAsync(image, s->v.img, (size_t)3 * n * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-  }
-  return RBMD_OK;
+  Transfer t(s);
+  t.split(x, s->v.x, s->v.y, s->v.z);
+  t.split(v, s->v.vx, s->v.vy, s->v.vz);
+  t.split(f, s->v.fx, s->v.fy, s->v.fz);
+  t.ints(image, s->v.img);
+  return transfer_out(s, t);
 }
 
 rbmd_status rbmd_locator_geometry(const rbmd_sys* s, int32_t dims[3], int32_t* nc, double dx[3]) {
@@ -1554,41 +1670,16 @@ rbmd_status rbmd_force_real(rbmd_sys* s, double* force, double* vir, double* elj
   } else if (!s->nbr_built) {
     RC_TRY(rbmd_neighbors_build(s, s->v.cap));
   }
-  hipStream_t st = s->ctx->stream;
   launch_real(s, 1, 1);
   RC_TRY(check_launch("force_real"));
-  const int n = s->n, ns = s->v.nslab;
-  std::vector<double> fx((size_t)ns * n), fy((size_t)ns * n), fz((size_t)ns * n), vv(6 * (size_t)ns * n),
-      el((size_t)ns * n), ec((size_t)ns * n);
-  std::vector<int> rank(n);
-  HIP_TRY(hipMemcpyAsync(fx.data(), s->v.fnx, fx.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(fy.data(), s->v.fny, fy.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(fz.data(), s->v.fnz, fz.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(vv.data(), s->v.vir_near, vv.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(el.data(), s->v.e_lj, el.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(ec.data(), s->v.e_coul, ec.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(rank.data(), s->v.rank, n * 4, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  // slab partials added in slab order, as the integrator does
-  auto slab_sum = [&](const std::vector<double>& a, size_t i, int stride, int k) {
-    double t = a[i * stride + k];
-    for (int sl = 1; sl < ns; ++sl) t += a[((size_t)sl * n + i) * stride + k];
-    return t;
-  };
-  for (int a = 0; a < n; ++a) {
-    const size_t i = rank[a];
-    if (force) {
-      force[3 * a] = slab_sum(fx, i, 1, 0);
-      force[3 * a + 1] = slab_sum(fy, i, 1, 0);
-      force[3 * a + 2] = slab_sum(fz, i, 1, 0);
-    }
-    if (vir)
-      for (int k = 0; k < 6; ++k) vir[6 * a + k] = slab_sum(vv, i, 6, k);
-    if (elj) elj[a] = slab_sum(el, i, 1, 0);
-    if (ecoul) ecoul[a] = slab_sum(ec, i, 1, 0);
-  }
+  const int ns = s->v.nslab;  // slab partials added in slab order, as the integrator does
+  Transfer t(s);
+  t.split(force, s->v.fnx, s->v.fny, s->v.fnz, ns, s->v.rank);
+  t.records(vir, s->v.vir_near, 6, ns, s->v.rank);
+  t.records(elj, s->v.e_lj, 1, ns, s->v.rank);
+  t.records(ecoul, s->v.e_coul, 1, ns, s->v.rank);
   int stt = 0;
-  RC_TRY(read_status(s, &stt));
+  RC_TRY(transfer_out(s, t, &stt));
   return status_to_rc(stt);
 }
 
@@ -1619,7 +1710,15 @@ rbmd_status rbmd_rbe_set_kvectors(rbmd_sys* s, int32_t p, const double* m) {
   std::vector<double> k(3 * (size_t)p);
   for (int l = 0; l < p; ++l)
     for (int d = 0; d < 3; ++d) k[3 * l + d] = 2 * kPi * m[3 * l + d] / s->v.box[d];
-  HIP_TRY(hipMemcpy(s->kcur, k.data(), k.size() * 8, hipMemcpyHostToDevice));
+  for (size_t k0 = 0; k0 < k.size(); k0 += s->pin_bytes / 8) {
+    const int h = s->pin_next;
+    const size_t len = std::min(k.size() - k0, s->pin_bytes / 8);
+    s->pin_next ^= 1;
+    HIP_TRY(hipEventSynchronize(s->pin_ev[h]));
+    std::memcpy(s->pin[h], k.data() + k0, len * 8);
+    HIP_TRY(hipMemcpyAsync(s->kcur + k0, s->pin[h], len * 8, hipMemcpyHostToDevice, s->ctx->stream));
+    HIP_TRY(hipEventRecord(s->pin_ev[h], s->ctx->stream));
+  }
   s->injected = true;
   return RBMD_OK;
 }
@@ -1651,21 +1750,10 @@ rbmd_status rbmd_rbe_structure_factor(rbmd_sys* s, double* rho_out) {
 
 // the k-space forces (and virials) of the launches just made, to the host
 static rbmd_status download_kforce(rbmd_sys* s, double* force, double* vir) {
-  hipStream_t st = s->ctx->stream;
-  int n = s->n;
-  std::vector<double> fx(n), fy(n), fz(n);
-  HIP_TRY(hipMemcpyAsync(fx.data(), s->v.fkx, n * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(fy.data(), s->v.fky, n * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(fz.data(), s->v.fkz, n * 8, hipMemcpyDeviceToHost, st));
-  if (vir) HIP_TRY(hipMemcpyAsync(vir, s->v.vir_k, 6 * (size_t)n * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  if (force)
-    for (int i = 0; i < n; ++i) {
-      force[3 * i] = fx[i];
-      force[3 * i + 1] = fy[i];
-      force[3 * i + 2] = fz[i];
-    }
-  return RBMD_OK;
+  Transfer t(s);
+  t.split(force, s->v.fkx, s->v.fky, s->v.fkz);
+  t.records(vir, s->v.vir_k, 6);
+  return transfer_out(s, t);
 }
 
 rbmd_status rbmd_rbe_force(rbmd_sys* s, double* force, double* vir) {
@@ -1732,19 +1820,12 @@ rbmd_status rbmd_force_bonded(rbmd_sys* s, double* force, double* eb, double* ea
   s->ctx->run("bonded", [&] { launch_bonded(s->v, s->iv, st, 1, s->seg_rows(SEG_BOND), &nblk); });
   s->seg_used[SEG_BOND] = nblk;
   RC_TRY(check_launch("bonded"));
-  int n = s->n;
-  std::vector<double> fx(n), fy(n), fz(n), rows((size_t)nblk * kRowBond);
-  HIP_TRY(hipMemcpyAsync(fx.data(), s->v.fbx, n * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(fy.data(), s->v.fby, n * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(fz.data(), s->v.fbz, n * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(rows.data(), s->seg_rows(SEG_BOND), rows.size() * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  if (force)
-    for (int i = 0; i < n; ++i) {
-      force[3 * i] = fx[i];
-      force[3 * i + 1] = fy[i];
-      force[3 * i + 2] = fz[i];
-    }
+  const double* rows = s->bond_rows;
+  if (eb || ea)
+    HIP_TRY(hipMemcpyAsync(s->bond_rows, s->seg_rows(SEG_BOND), (size_t)nblk * kRowBond * 8, hipMemcpyDeviceToHost, st));
+  Transfer t(s);
+  t.split(force, s->v.fbx, s->v.fby, s->v.fbz);
+  RC_TRY(transfer_out(s, t));
   double b = 0, a = 0;
   for (int r = 0; r < nblk; ++r) {
     b += rows[(size_t)r * kRowBond + (S_EBOND - S_VIR_BOND)];
@@ -1763,9 +1844,7 @@ rbmd_status rbmd_md_init(rbmd_sys* s) {
   launch_fill_int(s->v.status, 0, 1, st);
   s->injected = false;
   s->graph_ok = false;
-  NhcState zero;
-  std::memset(&zero, 0, sizeof(zero));
-  HIP_TRY(hipMemcpyAsync(s->nhc, &zero, sizeof(zero), hipMemcpyHostToDevice, st));
+  launch_fill_double((double*)s->nhc, 0.0, (int)(sizeof(NhcState) / 8), st);  // all-zero words
   if (s->skin) {  // build the skin list now (step counter 0)
     RC_TRY(use_geom(s, true));
     launch_skin_request(s->v, 0, st);
@@ -2058,17 +2137,12 @@ rbmd_status rbmd_md_query(rbmd_sys* s, int32_t* idle) {
 
 rbmd_status rbmd_md_thermo(rbmd_sys* s, rbmd_thermo* o) {
   if (!s || !o) return fail(RBMD_ERR_ARG, "bad arguments");
-  NhcState S;
-  int stt = 0, it = 0, mf = 0, lb = 0;
-  HIP_TRY(hipMemcpyAsync(&mf, s->v.misfit_count, 4, hipMemcpyDeviceToHost, s->ctx->stream));
-  HIP_TRY(hipMemcpyAsync(&S, s->nhc, sizeof(S), hipMemcpyDeviceToHost, s->ctx->stream));
-  HIP_TRY(hipMemcpyAsync(&stt, s->v.status, 4, hipMemcpyDeviceToHost, s->ctx->stream));
-  HIP_TRY(hipMemcpyAsync(&it, s->shake_iter, 4, hipMemcpyDeviceToHost, s->ctx->stream));
-  HIP_TRY(hipMemcpyAsync(&lb, s->v.list_builds, 4, hipMemcpyDeviceToHost, s->ctx->stream));
+  launch_thermo_out(s->nhc, s->v.misfit_count, s->v.status, s->shake_iter, s->v.list_builds, s->small, s->ctx->stream);
+  RC_TRY(check_launch("thermo"));
   HIP_TRY(hipStreamSynchronize(s->ctx->stream));
-  fill_thermo(s, S, stt, it, o);
-  o->misfit_atoms = mf;
-  o->list_builds = lb;
+  fill_thermo(s, s->small->nhc, s->small->status, s->small->iter, o);
+  o->misfit_atoms = s->small->misfit;
+  o->list_builds = s->small->builds;
   return RBMD_OK;
 }
 

@@ -332,6 +332,30 @@ struct NhcParams {
   int lj_only, cvff, shake_vir;
   int* shake_iter;       // SHAKE iteration maximum of the step, zeroed at the step start (phases 1, 5)
 };
+
+// A part of a call's arrays (atoms a0 .. a0 + atoms - 1 of n) between the
+// device and pinned host memory: on the host the fields lie one after the
+// other, each as whole records.
+struct TransferField {
+  double* p[3];     // split: one array per component; else p[0] holds records
+  const int* rank;  // list position of an atom, or null
+  int width, first; // doubles per atom, and those of the fields before it
+  int slabs;        // partial arrays to add (outwards)
+  int split, is_int;
+};
+constexpr int kTransferFields = 5;
+struct TransferDesc {
+  TransferField field[kTransferFields];
+  int nfield, width, n, a0, atoms;
+  double* host;
+};
+struct ThermoOut {
+  NhcState nhc;
+  int misfit, status, iter, builds;
+};
+void launch_transfer(const TransferDesc& d, bool out, hipStream_t st);
+void launch_thermo_out(const NhcState* nhc, const int* misfit, const int* status, const int* iter, const int* builds,
+                       ThermoOut* out, hipStream_t st);
 // phase 1: step++ and NHC half step (InitialIntegrate); 2: ComputeTempe + pressure + NHC
 // (FinalIntegrate); 3: SetUp; 4: Berendsen/rescale end of step; 5: step++ only;
 // 6: phase 2 then phase 1 (between two steps of one call)
