@@ -18,6 +18,7 @@ struct EwView {
   int per, split0, splits;  // structure factor: atoms per split, this batch's first split and their number
   int total_splits;
   int rper, rsplits;  // force: row tiles per split, splits
+  int wgroups;        // weight pass: threads that share the partials of a grid point
   double *tx, *ty, *tz;  // phase tables of the batch: (cos, sin) of m 2 pi x / L, x's times the charge
   double* part;       // [total_splits][2][Rpad][ldz] structure-factor partials
   double* W;          // [4][Kd][Rpad] force weights

@@ -69,6 +69,7 @@ bool ewald_plan(int n, const int kmax[3], int64_t tab_bytes, int64_t part_bytes,
   v->per = std::max(64, up((int)((v->batch + sp - 1) / sp), 16));
   v->splits = (v->batch + v->per - 1) / v->per;
   v->total_splits = (batches - 1) * v->splits + (n - (batches - 1) * v->batch + v->per - 1) / v->per;
+  for (v->wgroups = 1; v->wgroups < 16 && v->total_splits > 8 * v->wgroups;) v->wgroups *= 2;
   // force: 128 atoms a workgroup, the row tiles split until about 2,048 wavefronts run
   const int wg = (v->batch + 127) / 128;
   const int tiles = v->Rpad / 16;
@@ -81,7 +82,10 @@ bool ewald_plan(int n, const int kmax[3], int64_t tab_bytes, int64_t part_bytes,
 
 static int64_t ew_up(int64_t doubles) { return (doubles * 8 + 255) / 256 * 256; }
 
-int ewald_energy_rows(const EwView& v) { return (v.Rpad * (v.Kd / 2) + kBlock - 1) / kBlock; }
+int ewald_energy_rows(const EwView& v) {
+  const int points = kBlock / v.wgroups;
+  return (v.Rpad * (v.Kd / 2) + points - 1) / points;
+}
 
 int64_t ewald_bytes(const EwView& v, bool force) {
   int64_t b = ew_up((int64_t)v.batch * v.ldx) + ew_up((int64_t)v.batch * v.ldy) + ew_up((int64_t)v.batch * v.ldz) +
@@ -213,43 +217,64 @@ static int ew_rho_blocks(const EwView& v) {
   return (v.Rpad / 16 + 3) / 4 * (v.ldz / (16 * v.nt)) * ((v.n + v.per - 1) / v.per);
 }
 
-// Sum of the partials, the force weights and the energy: one thread a (row,
+// Sum of the partials, the force weights and the energy of each grid point (row,
 // kz).  With rho+ = rho(kx, ky, kz), rho- = rho(kx, ky, -kz), U = rho+ + rho-,
 // V = rho+ - rho- and the prefactor 2 e^{-k^2/4 alpha} / (V k^2) of k and -k:
 //   sum over +-kz of rho conj(ez)    = U cos - i V sin
 //   sum over +-kz of rho conj(ez) kz = kz (V cos - i U sin)
 // On the row kx = ky = 0 the conjugate of +kz is -kz itself: rho- = 0 there.
+//
+// wgroups threads add the partials of a grid point (a small grid has few
+// points and up to hundreds of partials: one thread each took 32 us at 6000
+// atoms, this one 7), their sums added in order.
 __device__ __forceinline__ void ew_weight_body(const SysView& s, const EwView& v, const int bid) {
 #pragma clang fp contract(off)
+  __shared__ double4 sums[kBlock];
   const int nz = v.Kd / 2;
-  const int t = bid * kBlock + threadIdx.x;
+  const int points = kBlock / v.wgroups;
+  const int g = threadIdx.x / points;
+  const int t = bid * points + threadIdx.x % points;
   const int r = t / nz, z = t % nz;
+  const bool in = r < v.R && z <= v.K[2] && (r > 0 || z > 0);
+  double2 a = make_double2(0, 0), b = make_double2(0, 0);
+  if (in) {
+    const size_t plane = (size_t)v.Rpad * v.ldz, at = (size_t)r * v.ldz + 2 * z;
+#pragma unroll 8
+    for (int sp = g; sp < v.total_splits; sp += v.wgroups) {
+      const double2 p = *reinterpret_cast<const double2*>(v.part + (size_t)sp * 2 * plane + at);
+      const double2 q = *reinterpret_cast<const double2*>(v.part + ((size_t)sp * 2 + 1) * plane + at);
+      a.x += p.x;
+      a.y += p.y;
+      b.x += q.x;
+      b.y += q.y;
+    }
+  }
+  if (v.wgroups > 1) {
+    sums[threadIdx.x] = make_double4(a.x, a.y, b.x, b.y);
+    __syncthreads();
+    if (g == 0)
+      for (int u = 1; u < v.wgroups; ++u) {
+        const double4 o = sums[u * points + threadIdx.x];
+        a.x += o.x;
+        a.y += o.y;
+        b.x += o.z;
+        b.y += o.w;
+      }
+  }
   double e = 0.0;
-  if (r < v.Rpad) {
-    const bool in = r < v.R && z <= v.K[2] && (r > 0 || z > 0);
+  if (g == 0 && r < v.Rpad) {
     double w[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
     if (in) {
-      double2 a = make_double2(0, 0), b = make_double2(0, 0);
-      const size_t plane = (size_t)v.Rpad * v.ldz, at = (size_t)r * v.ldz + 2 * z;
-#pragma unroll 8
-      for (int sp = 0; sp < v.total_splits; ++sp) {
-        const double2 p = *reinterpret_cast<const double2*>(v.part + (size_t)sp * 2 * plane + at);
-        const double2 q = *reinterpret_cast<const double2*>(v.part + ((size_t)sp * 2 + 1) * plane + at);
-        a.x += p.x;
-        a.y += p.y;
-        b.x += q.x;
-        b.y += q.y;
-      }
       int mx, my;
       ew_row(v, r, mx, my);
       const double kx = 2 * kPi * mx / s.box[0], ky = 2 * kPi * my / s.box[1], kz = 2 * kPi * z / s.box[2];
       const double k2 = kx * kx + ky * ky + kz * kz;
-      const double g = exp(-k2 / (4 * s.alpha)) / k2;
+      const double gk = exp(-k2 / (4 * s.alpha)) / k2;
       const double pr = a.x - b.y, pi = a.y + b.x;  // rho+
       const bool two = r > 0 && z > 0;
       const double nr = two ? a.x + b.y : 0.0, ni = two ? b.x - a.y : 0.0;  // rho-
-      e = 2.0 * g * ((pr * pr + pi * pi) + (nr * nr + ni * ni));
-      const double c = 2.0 * g / s.volume;
+      e = 2.0 * gk * ((pr * pr + pi * pi) + (nr * nr + ni * ni));
+      const double c = 2.0 * gk / s.volume;
       const double ur = c * (pr + nr), ui = c * (pi + ni), vr = c * (pr - nr), vi = c * (pi - ni);
       w[0][0] = ur;
       w[0][1] = vi;

@@ -47,37 +47,41 @@ int rho_atoms_per_block(int n, int kblocks) {
   } while (0)
 
 // rho[t] = sum over the partial rows b of rho_part[b][t].  One workgroup per
-// kRedCols columns (one per lane, coalesced rows); wavefront w sums rows w,
-// w + kRedWaves, ... (independent loads, in flight together), and the
-// kRedWaves partial sums are added in wavefront order: a fixed order, and
-// ~300 rows at 300,000 atoms take ~20 loads per wavefront instead of one
-// thread's chain of 300.
-constexpr int kRedCols = kWave;
+// kRedCols columns; row group g of its kRedGroups sums rows g, g + kRedGroups,
+// ... (independent loads, in flight together), and the groups' sums are added
+// in order: a fixed order.  16 columns (128 bytes of a row) and 64 groups: the
+// 469 rows of 30,000 atoms are 8 loads a thread.  With 64 columns and 16
+// groups 400 columns were 7 workgroups of 30 loads: 13.5 us, now
+// 7 (99,000 atoms: 33 and 12).
+constexpr int kRedCols = 16;
 constexpr int kRedWaves = 16;
+constexpr int kRedGroups = kRedWaves * kWave / kRedCols;
 
 __device__ __forceinline__ void rho_reduce_body(const SysView& s, const KView& kv, const int bid) {
 #pragma clang fp contract(off)
-  __shared__ double part[kRedWaves][kRedCols];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int w = threadIdx.x / kWave;
+  __shared__ double part[kRedGroups][kRedCols];
+  const int col = threadIdx.x % kRedCols;
+  const int g = threadIdx.x / kRedCols;
   const int n2 = 2 * kv.P;
-  const int t = bid * kRedCols + lane;
+  const int t = bid * kRedCols + col;
   double acc = 0.0;
-  if (t < n2)
-    for (int b = w; b < kv.nblk_rho; b += kRedWaves) acc += kv.rho_part[(size_t)b * n2 + t];
-  part[w][lane] = acc;
+  if (t < n2) {
+#pragma unroll 8
+    for (int b = g; b < kv.nblk_rho; b += kRedGroups) acc += kv.rho_part[(size_t)b * n2 + t];
+  }
+  part[g][col] = acc;
   __syncthreads();
-  if (w == 0) {
+  if (threadIdx.x < kWave) {  // four threads a column, 16 groups each, and a fixed tree
+    constexpr int per = kRedGroups * kRedCols / kWave;
     double r = 0.0;
-    if (t < n2) {
-      r = part[0][lane];
-      for (int v = 1; v < kRedWaves; ++v) r += part[v][lane];
-      kv.rho[t] = r;
-    }
+    for (int v = 0; v < per; ++v) r += part[g * per + v][col];
+#pragma unroll
+    for (int off = kRedCols; off < kWave; off <<= 1) r += __shfl_xor(r, off);
+    if (t < n2 && g == 0) kv.rho[t] = r;
     // Im rho from the odd neighbour lane (2P is even: both lanes of a pair
     // are in range or both out); the whole wavefront takes part
     const double r_im = __shfl_xor(r, 1);
-    if (kv.krec && t < n2 && !(t & 1)) {
+    if (kv.krec && t < n2 && !(t & 1) && g == 0) {
       KRec& rec = kv.krec[t >> 1];
       const int l = t >> 1;
       const double kx = kv.kvec[3 * l], ky = kv.kvec[3 * l + 1], kz = kv.kvec[3 * l + 2];

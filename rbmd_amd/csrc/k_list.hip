@@ -64,7 +64,7 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
   __shared__ float sx[kListWindow + kWave], sy[kListWindow + kWave], sz[kListWindow + kWave];
   __shared__ int se[kListWindow + kWave];
   __shared__ ListTable tabs[kListWaves];
-  __shared__ int kept[kListWaves], table[2];
+  __shared__ int kept[kListWaves], candidates;
   __shared__ float box[6];
   if (!list_rebuild(s)) return;  // skin list between builds
   const int lane = threadIdx.x & (kWave - 1);
@@ -160,10 +160,7 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
   if (w == 0) {  // the stencil
     bool sh;
     const int t = stream_table<32, true>(s, 1, ca, cb, cc, 0, tabs[0], 4, sh);
-    if (lane == 0) {
-      table[0] = t;
-      table[1] = sh ? 1 : 0;
-    }
+    if (lane == 0) candidates = t;
   } else if (w == 1) {  // the atoms' bounding box
     float bl[3] = {fit ? x : 3e38f, fit ? y : 3e38f, fit ? z : 3e38f};
     float bh[3] = {fit ? x : -3e38f, fit ? y : -3e38f, fit ? z : -3e38f};
@@ -181,8 +178,7 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
       }
   }
   __syncthreads();
-  const int total = __builtin_amdgcn_readfirstlane(table[0]);
-  const bool shifts = __builtin_amdgcn_readfirstlane(table[1]) != 0;
+  const int total = __builtin_amdgcn_readfirstlane(candidates);
   float bl[3], bh[3], ra2 = 0.0f;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -239,7 +235,7 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
 #pragma unroll
     for (int r = 0; r < kListRounds; ++r) {
       e[r] = stream_entry(tabs[0], min(t0 + r * kWave, total - 1));
-      p[r] = stream_position(s, e[r], shifts);
+      p[r] = stream_next_position(s, e[r]);
     }
     unsigned long long keep[kListRounds];
     float px[kListRounds], py[kListRounds], pz[kListRounds];
@@ -318,7 +314,7 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
           near |= (bal[a] ^ __ballot(d[a / 4][a % 4] < out_f)) & ~__ballot(entry == pack_entry(first + a, 0, 0, 0));
         if (near != 0ull) {
           const bool live = b + lane < m;
-          const double4 pj = stream_position(s, live ? entry : pack_entry(0, 0, 0, 0), shifts);
+          const double4 pj = stream_next_position(s, live ? entry : pack_entry(0, 0, 0, 0));
 #pragma unroll
           for (int a = 0; a < kListAtoms; ++a) {
             if (a >= nmine) break;  // wave-uniform

@@ -101,6 +101,19 @@ __device__ __forceinline__ double4 stream_position(const SysView& s, int e, bool
   return p;
 }
 
+// the same for an entry whose offsets are at most one box: shift_len is the
+// product above for an offset of one, and times 1, 0 or -1 exact
+__device__ __forceinline__ double4 stream_next_position(const SysView& s, int e) {
+#pragma clang fp contract(off)
+  double4 p = s.spos[e >> kShiftBits];
+  if (__ballot((e & ((1 << kShiftBits) - 1)) != pack_entry(0, 0, 0, 0)) != 0ull) {
+    p.x -= (double)((e & 7) - 3) * s.shift_len[0];
+    p.y -= (double)(((e >> 3) & 7) - 3) * s.shift_len[1];
+    p.z -= (double)(((e >> 6) & 7) - 3) * s.shift_len[2];
+  }
+  return p;
+}
+
 // The stream around one cell for one wavefront: f(live, entry, x, y, z) for 64
 // candidates at a time (misfit atoms).
 template <int N, class F>
