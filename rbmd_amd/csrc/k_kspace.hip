@@ -47,14 +47,15 @@ int rho_atoms_per_block(int n, int kblocks) {
   } while (0)
 
 // rho[t] = sum over the partial rows b of rho_part[b][t].  One workgroup per
-// kRedCols columns; row group g of its kRedGroups sums rows g, g + kRedGroups,
-// ... (independent loads, in flight together), and the groups' sums are added
-// in order: a fixed order.  16 columns (128 bytes of a row) and 64 groups: the
-// 469 rows of 30,000 atoms are 8 loads a thread.  With 64 columns and 16
-// groups 400 columns were 7 workgroups of 30 loads: 13.5 us, now
-// 7 (99,000 atoms: 33 and 12).
-constexpr int kRedCols = 16;
-constexpr int kRedWaves = 16;
+// kRedCols columns (64 bytes of a row); row group g of its kRedGroups sums
+// rows g, g + kRedGroups, ... (independent loads, in flight together), and the
+// groups' sums are added in a fixed order.  With 64 columns and 16 groups the
+// 400 columns of 30,000 atoms were 7 workgroups of 30 loads a thread: 13.5 us,
+// now 7 (99,000 atoms: 33 and 12).  Four wavefronts, not more: the kernel runs
+// beside the list build, whose small workgroups leave no room for 1024 threads
+// at once (a pack's launch then waited 98 us for it).
+constexpr int kRedCols = 8;
+constexpr int kRedWaves = 4;
 constexpr int kRedGroups = kRedWaves * kWave / kRedCols;
 
 __device__ __forceinline__ void rho_reduce_body(const SysView& s, const KView& kv, const int bid) {
@@ -71,7 +72,7 @@ __device__ __forceinline__ void rho_reduce_body(const SysView& s, const KView& k
   }
   part[g][col] = acc;
   __syncthreads();
-  if (threadIdx.x < kWave) {  // four threads a column, 16 groups each, and a fixed tree
+  if (threadIdx.x < kWave) {  // eight threads a column, four groups each, and a fixed tree
     constexpr int per = kRedGroups * kRedCols / kWave;
     double r = 0.0;
     for (int v = 0; v < per; ++v) r += part[g * per + v][col];
