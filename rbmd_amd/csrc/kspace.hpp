@@ -9,15 +9,19 @@
 namespace rbmd {
 
 // e^{i k.r} with k = 2 pi m / L is e^{2 pi i t} with the phase t = m.(r/L) in
-// turns (several hundred radians at |m| ~ 30): sincos_turns reduces it
-// exactly to a quadrant and a remainder of at most 1/8 turn before its
-// polynomials, so no large-argument reduction is needed.  F32 (mixed
+// turns (several hundred radians at |m| ~ 30): sincos_turns_table reduces it
+// exactly to a 64th of a turn and a remainder before its polynomials, so no
+// large-argument reduction is needed (its table is copied to LDS: the lanes'
+// entries differ).  Against sincos_turns: structure factor and force 17.8 + 23.7
+// -> 13.7 + 15.3 us at 30,000 atoms x 200 vectors, 112 + 121 -> 76 + 83 us at
+// 100,000 x 667.  F32 (mixed
 // precision): the phase reduced exactly in FP64 to at most 1/2 turn, rounded
 // to FP32, and the hardware sin / cos (sincos_turns32_hw, |error| <= 1.2e-7);
 // the phase, the reduction and every sum stay FP64.
 template <bool F32>
 __device__ __forceinline__ void phase_sincos(double mx, double my, double mz, double sx, double sy, double sz,
-                                             double* sn, double* cs) {
+                                             const double* turn, double* sn, double* cs) {
+#pragma clang fp contract(off)
   const double t = fma(mz, sz, fma(my, sy, mx * sx));
   if constexpr (F32) {
     float s32, c32;
@@ -25,8 +29,13 @@ __device__ __forceinline__ void phase_sincos(double mx, double my, double mz, do
     *sn = s32;
     *cs = c32;
   } else {
-    sincos_turns(t, sn, cs);
+    sincos_turns_table(t, turn, sn, cs);
   }
+}
+
+// the workgroup's copy of the table (a barrier follows before its use)
+__device__ __forceinline__ void load_turns(double* turn) {
+  for (int k = threadIdx.x; k < 2 * kTurns; k += blockDim.x) turn[k] = kTurnTable[k];
 }
 
 // m = k L / (2 pi), an integer held in k to ~1e-13: the product with the
@@ -46,6 +55,11 @@ __device__ __forceinline__ void rho_partial_body(const SysView& s, const KView& 
 #pragma clang fp contract(off)  // fused multiply-adds are written out: the same rounding in every kernel
   constexpr int NW = kBlock / kWave;
   __shared__ double part[NW][2 * KB][kWave];
+  __shared__ __attribute__((aligned(16))) double turn[F32 ? 2 : 2 * kTurns];
+  if constexpr (!F32) {
+    load_turns(turn);
+    __syncthreads();
+  }
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int kb0 = bk * kWave * KB;
@@ -87,7 +101,7 @@ __device__ __forceinline__ void rho_partial_body(const SysView& s, const KView& 
 #pragma unroll
     for (int t = 0; t < KB; ++t) {
       double sn, cs;
-      phase_sincos<F32>(mx[t], my[t], mz[t], sx, sy, sz, &sn, &cs);
+      phase_sincos<F32>(mx[t], my[t], mz[t], sx, sy, sz, turn, &sn, &cs);
       re[t] = fma(q, cs, re[t]);
       im[t] = fma(q, sn, im[t]);
     }
@@ -127,6 +141,11 @@ __device__ __forceinline__ void kforce_body(const SysView& s, const KView& kv, d
   constexpr int KS = 1 << LG;
   constexpr int NX = PERATOM ? 9 : 3;  // per-atom sums the wavefronts hand over
   __shared__ double part[KS][NX][kWave];
+  __shared__ __attribute__((aligned(16))) double turn[F32 ? 2 : 2 * kTurns];
+  if constexpr (!F32) {
+    load_turns(turn);
+    __syncthreads();
+  }
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int i = bid * kWave + lane;
@@ -182,10 +201,11 @@ __device__ __forceinline__ void kforce_body(const SysView& s, const KView& kv, d
       v[5] = y * fz + z * fy;
     }
   } else {
+#pragma unroll 2
     for (int l = l0; l < l1; ++l) {
       const double kx = rec[l].kx, ky = rec[l].ky, kz = rec[l].kz;
       double sn, cs;
-      phase_sincos<F32>(rec[l].mx, rec[l].my, rec[l].mz, sx, sy, sz, &sn, &cs);
+      phase_sincos<F32>(rec[l].mx, rec[l].my, rec[l].mz, sx, sy, sz, turn, &sn, &cs);
       const double fs = (q4 * rec[l].pre) * fma(cs, rec[l].ri, -(sn * rec[l].rr));
       fx = fma(fs, kx, fx);
       fy = fma(fs, ky, fy);

@@ -82,6 +82,62 @@ RBMD_HD inline void sincos_turns(double t, double* sn, double* cs) {
   sincos_rotate<double>(q, r * ps, pc, sn, cs);
 }
 
+// FP64 with a table of the 64ths of a turn (kTurnTable, or a copy in LDS): the
+// remainder is at most 1/128 turn, so 4 + 4 polynomial terms do, and the
+// addition theorem puts them together.  At most 1.17e-16 absolute error (the
+// polynomials above: 1.38e-16), in about 20 instructions instead of 36.
+constexpr int kTurns = 64;
+constexpr double kTurnTable[2 * kTurns] = {  // cos, sin of j / 64 turn
+    0x1p+0, 0x0p+0, 0x1.fd88da3d12526p-1, 0x1.917a6bc29b42cp-4,
+    0x1.f6297cff75cbp-1, 0x1.8f8b83c69a60bp-3, 0x1.e9f4156c62ddap-1, 0x1.294062ed59f06p-2,
+    0x1.d906bcf328d46p-1, 0x1.87de2a6aea963p-2, 0x1.c38b2f180bdb1p-1, 0x1.e2b5d3806f63bp-2,
+    0x1.a9b66290ea1a3p-1, 0x1.1c73b39ae68c8p-1, 0x1.8bc806b151741p-1, 0x1.44cf325091dd6p-1,
+    0x1.6a09e667f3bcdp-1, 0x1.6a09e667f3bcdp-1, 0x1.44cf325091dd6p-1, 0x1.8bc806b151741p-1,
+    0x1.1c73b39ae68c8p-1, 0x1.a9b66290ea1a3p-1, 0x1.e2b5d3806f63bp-2, 0x1.c38b2f180bdb1p-1,
+    0x1.87de2a6aea963p-2, 0x1.d906bcf328d46p-1, 0x1.294062ed59f06p-2, 0x1.e9f4156c62ddap-1,
+    0x1.8f8b83c69a60bp-3, 0x1.f6297cff75cbp-1, 0x1.917a6bc29b42cp-4, 0x1.fd88da3d12526p-1,
+    0x0p+0, 0x1p+0, -0x1.917a6bc29b42cp-4, 0x1.fd88da3d12526p-1,
+    -0x1.8f8b83c69a60bp-3, 0x1.f6297cff75cbp-1, -0x1.294062ed59f06p-2, 0x1.e9f4156c62ddap-1,
+    -0x1.87de2a6aea963p-2, 0x1.d906bcf328d46p-1, -0x1.e2b5d3806f63bp-2, 0x1.c38b2f180bdb1p-1,
+    -0x1.1c73b39ae68c8p-1, 0x1.a9b66290ea1a3p-1, -0x1.44cf325091dd6p-1, 0x1.8bc806b151741p-1,
+    -0x1.6a09e667f3bcdp-1, 0x1.6a09e667f3bcdp-1, -0x1.8bc806b151741p-1, 0x1.44cf325091dd6p-1,
+    -0x1.a9b66290ea1a3p-1, 0x1.1c73b39ae68c8p-1, -0x1.c38b2f180bdb1p-1, 0x1.e2b5d3806f63bp-2,
+    -0x1.d906bcf328d46p-1, 0x1.87de2a6aea963p-2, -0x1.e9f4156c62ddap-1, 0x1.294062ed59f06p-2,
+    -0x1.f6297cff75cbp-1, 0x1.8f8b83c69a60bp-3, -0x1.fd88da3d12526p-1, 0x1.917a6bc29b42cp-4,
+    -0x1p+0, 0x0p+0, -0x1.fd88da3d12526p-1, -0x1.917a6bc29b42cp-4,
+    -0x1.f6297cff75cbp-1, -0x1.8f8b83c69a60bp-3, -0x1.e9f4156c62ddap-1, -0x1.294062ed59f06p-2,
+    -0x1.d906bcf328d46p-1, -0x1.87de2a6aea963p-2, -0x1.c38b2f180bdb1p-1, -0x1.e2b5d3806f63bp-2,
+    -0x1.a9b66290ea1a3p-1, -0x1.1c73b39ae68c8p-1, -0x1.8bc806b151741p-1, -0x1.44cf325091dd6p-1,
+    -0x1.6a09e667f3bcdp-1, -0x1.6a09e667f3bcdp-1, -0x1.44cf325091dd6p-1, -0x1.8bc806b151741p-1,
+    -0x1.1c73b39ae68c8p-1, -0x1.a9b66290ea1a3p-1, -0x1.e2b5d3806f63bp-2, -0x1.c38b2f180bdb1p-1,
+    -0x1.87de2a6aea963p-2, -0x1.d906bcf328d46p-1, -0x1.294062ed59f06p-2, -0x1.e9f4156c62ddap-1,
+    -0x1.8f8b83c69a60bp-3, -0x1.f6297cff75cbp-1, -0x1.917a6bc29b42cp-4, -0x1.fd88da3d12526p-1,
+    0x0p+0, -0x1p+0, 0x1.917a6bc29b42cp-4, -0x1.fd88da3d12526p-1,
+    0x1.8f8b83c69a60bp-3, -0x1.f6297cff75cbp-1, 0x1.294062ed59f06p-2, -0x1.e9f4156c62ddap-1,
+    0x1.87de2a6aea963p-2, -0x1.d906bcf328d46p-1, 0x1.e2b5d3806f63bp-2, -0x1.c38b2f180bdb1p-1,
+    0x1.1c73b39ae68c8p-1, -0x1.a9b66290ea1a3p-1, 0x1.44cf325091dd6p-1, -0x1.8bc806b151741p-1,
+    0x1.6a09e667f3bcdp-1, -0x1.6a09e667f3bcdp-1, 0x1.8bc806b151741p-1, -0x1.44cf325091dd6p-1,
+    0x1.a9b66290ea1a3p-1, -0x1.1c73b39ae68c8p-1, 0x1.c38b2f180bdb1p-1, -0x1.e2b5d3806f63bp-2,
+    0x1.d906bcf328d46p-1, -0x1.87de2a6aea963p-2, 0x1.e9f4156c62ddap-1, -0x1.294062ed59f06p-2,
+    0x1.f6297cff75cbp-1, -0x1.8f8b83c69a60bp-3, 0x1.fd88da3d12526p-1, -0x1.917a6bc29b42cp-4};
+RBMD_HD inline void sincos_turns_table(double t, const double* cs64, double* sn, double* cs) {
+  using namespace sincos_detail;
+  // 64 t rounded to a whole number in the low bits of its sum with 1.5 2^52
+  // (for |t| below 2^45 turns)
+  const double shifted = fma(64.0, t, 0x1.8p52);
+  long long bits;
+  __builtin_memcpy(&bits, &shifted, 8);
+  const double r = fma(-1.0 / 64.0, shifted - 0x1.8p52, t);
+  const double* e = cs64 + 2 * ((int)bits & (kTurns - 1));
+  const double z = r * r;
+  constexpr double S1 = taylor(1), S3 = taylor(3), S5 = taylor(5), S7 = taylor(7);
+  constexpr double C2 = taylor(2), C4 = taylor(4), C6 = taylor(6), C8 = taylor(8);
+  const double s = r * fma(z, fma(z, fma(z, S7, S5), S3), S1);
+  const double c = z * fma(z, fma(z, fma(z, C8, C6), C4), C2);  // cos - 1
+  *sn = e[1] + fma(e[1], c, e[0] * s);
+  *cs = e[0] + fma(e[0], c, -(e[1] * s));
+}
+
 // FP32 polynomial on the FP64-reduced phase: sin(2 pi t), cos(2 pi t)
 RBMD_HD inline void sincos_turns32(double t, float* sn, float* cs) {
   using namespace sincos_detail;
