@@ -1124,8 +1124,10 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   const int ncell_max = std::max(s->g_ref.ncell, s->g_skin.ncell);
   const int items_max = std::max(s->g_ref.n_items, s->g_skin.n_items);
   // lanes per atom in the pair kernel: enough threads to fill 256 CUs for
-  // small systems, fewer lanes (longer per-lane loops) for large ones
-  v.lanes_lg = n <= 60000 ? 4 : (n <= 250000 ? 3 : 2);
+  // small systems, fewer lanes (longer per-lane loops) for large ones.  With 4,
+  // 8 and 16: salt 20,000 23, 19 and 18 us, 99,000 57, 57 and 62, 300,000 144,
+  // 138 and 167; water (mixed) 300,000 457, 381 and 359
+  v.lanes_lg = n <= 60000 ? 4 : 3;
   v.compact = p->coulomb_type != RBMD_COULOMB_EWALD && !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes && stencil_pays(v) ? 1 : 0;
   v.st_cfg = stencil_choice(v);
   if (p->pair_lanes) v.lanes_lg = p->pair_lanes == 4 ? 2 : (p->pair_lanes == 8 ? 3 : 4);

@@ -295,8 +295,9 @@ __device__ __forceinline__ void cell_sort_body(const SysView& s, const int bid) 
     return;
   }
   int c = bid;
-  int start = s.cell_start[c];
-  int cnt = s.cell_start[c + 1] - start;
+  // the same in all lanes, which a packed kernel's table does not tell
+  const int start = __builtin_amdgcn_readfirstlane(s.cell_start[c]);
+  const int cnt = __builtin_amdgcn_readfirstlane(s.cell_start[c + 1]) - start;
   if (threadIdx.x == 0) {  // read by the binning and scatter kernels before this one
     s.cell_count[c] = 0;
     s.cursor[c] = 0;

@@ -7,6 +7,19 @@
 
 namespace rbmd {
 
+// Loads from memory that is known to be global: in the packed kernels the
+// pointers come out of a table, where the compiler would otherwise use flat
+// loads (which wait for LDS accesses and theirs for them)
+typedef double StreamD4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ int global_int(const int* p) { return *(const __attribute__((address_space(1))) int*)p; }
+__device__ __forceinline__ int global_scalar(const int* p) {  // the same address in all lanes
+  return __builtin_amdgcn_readfirstlane(global_int(p));
+}
+__device__ __forceinline__ double4 global_double4(const double4* p) {
+  const StreamD4 v = *(const __attribute__((address_space(1))) StreamD4*)p;
+  return make_double4(v.x, v.y, v.z, v.w);
+}
+
 // stencil_cell for a grid cell and a step of at most one cell: one wrap at
 // most, no division
 __device__ __forceinline__ StencilCell stencil_next(const SysView& s, int ca, int cb, int cc, int a, int b, int e) {
@@ -20,8 +33,8 @@ __device__ __forceinline__ StencilCell stencil_next(const SysView& s, int ca, in
   ne += t.sc * s.dims[2];
   const int cell = na + nb * s.dims[0] + ne * s.dims[0] * s.dims[1];
   t.ok = true;
-  t.js = s.cell_start[cell];
-  t.je = s.cell_start[cell + 1];
+  t.js = global_int(s.cell_start + cell);
+  t.je = global_int(s.cell_start + cell + 1);
   return t;
 }
 
@@ -92,7 +105,7 @@ __device__ __forceinline__ int stream_entry(const StreamTable<N>& tab, int t) {
 // an entry's position less its image offset (w: charge)
 __device__ __forceinline__ double4 stream_position(const SysView& s, int e, bool shifts) {
 #pragma clang fp contract(off)
-  double4 p = s.spos[e >> kShiftBits];
+  double4 p = global_double4(s.spos + (e >> kShiftBits));
   if (shifts) {
     p.x -= s.dxdydz[0] * (double)(((e & 7) - 3) * s.dims[0]);
     p.y -= s.dxdydz[1] * (double)((((e >> 3) & 7) - 3) * s.dims[1]);
@@ -105,7 +118,7 @@ __device__ __forceinline__ double4 stream_position(const SysView& s, int e, bool
 // product above for an offset of one, and times 1, 0 or -1 exact
 __device__ __forceinline__ double4 stream_next_position(const SysView& s, int e) {
 #pragma clang fp contract(off)
-  double4 p = s.spos[e >> kShiftBits];
+  double4 p = global_double4(s.spos + (e >> kShiftBits));
   if (__ballot((e & ((1 << kShiftBits) - 1)) != pack_entry(0, 0, 0, 0)) != 0ull) {
     p.x -= (double)((e & 7) - 3) * s.shift_len[0];
     p.y -= (double)(((e >> 3) & 7) - 3) * s.shift_len[1];
