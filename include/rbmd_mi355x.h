@@ -140,7 +140,8 @@ typedef struct rbmd_params {
    * of the k-space force kernel (2, 4, 8; default 4), k vectors per lane of
    * the structure-factor kernel (1, 2, 4; default 1).  rbmd_amd/tune.py
    * measures them per kind, precision and size and rbmd_amd/tiles.json holds
-   * the result. */
+   * the result.  Systems of up to a few thousand atoms whose steps compute the
+   * pair forces from the cells keep 16 lanes and 16 wavefronts. */
   int32_t pair_lanes;
   int32_t kforce_lanes;
   int32_t rho_kblock;

@@ -366,7 +366,7 @@ double column_fraction(double wx, double wy, double rc) {
   return acc * (2.0 * hx / m) * (2.0 * hy / m) / (4.0 / 3.0 * kPi);
 }
 
-// Default list capacity.  VERLET: per column segment, 1.15 x the mean count
+// Default list capacity.  VERLET: per stencil column, 1.15 x the mean count
 // in the largest column share of the list's cutoff sphere (rc, or rc + skin)
 // + 64; RBL: the core region plus twice the mean shell sample + 64.
 int default_cap(const rbmd_sys* s) {
@@ -964,7 +964,7 @@ rbmd_status rbmd_footprint_estimate(const rbmd_sys_desc* d, const rbmd_params* p
   double c = d->n_atoms / vol * 4.0 / 3.0 * kPi * p->cut_off * p->cut_off * p->cut_off;
   int64_t n = d->n_atoms;
   int64_t cells = (int64_t)dims[0] * dims[1] * dims[2];
-  // list slots per atom as ensure_nbr sizes them (VERLET: 9 column segments)
+  // list slots per atom as ensure_nbr sizes them (VERLET: 9 columns' shares)
   int64_t slots;
   if (p->neighbor_type == RBMD_NEIGHBOR_RBL) {
     slots = (int64_t)(2.0 * c + 64);

@@ -1,13 +1,12 @@
-// cells.hpp -- device helpers shared by the neighbour-list build and the
-// fused cell-stencil force kernel: cell coordinates, the 3x3x3 stencil with
-// periodic images, and the candidate stream of one stencil column.
+// cells.hpp -- device helpers shared by the neighbour-list builds and the
+// cell-stencil force kernels: cell coordinates, the 3x3x3 stencil with
+// periodic images, and the candidate stream of one stencil column (k_force.hip).
 #pragma once
 #include "dev.hpp"
 
 namespace rbmd {
 
-constexpr int kMisfitBlocks = 64;  // workgroups that take the misfit atoms
-constexpr int kColWaves = 9;        // stencil columns of the VERLET list build
+constexpr int kMisfitBlocks = 64;  // workgroups of the fused kernel that take the misfit atoms
 constexpr int kScanScatterCells = 2048;  // most cells for the one-launch scan + scatter
 
 // InWhichCell (ExecPointLocator.h:271-274): unclamped trunc

@@ -13,7 +13,7 @@ namespace rbmd {
 constexpr double kPi = 3.14159265358979323846;
 constexpr int kBlock = 256;     // threads per workgroup (4 wavefronts of 64)
 constexpr int kWave = 64;       // CDNA wavefront width
-constexpr int kChunk = 64;      // i-atoms per neighbour-build work item (one wavefront)
+constexpr int kChunk = 64;      // i-atoms per work item of the neighbour builds
 constexpr int kMaxSpecial = 8;  // special-list entries held in registers per atom (RBL kernels)
 constexpr int kShiftBits = 9;   // 3 bits per axis image shift in packed neighbour entries
 constexpr int kMaxLanes = 16;   // most lanes sharing one atom's neighbour list

@@ -1,11 +1,13 @@
 // k_pair.hip -- real-space LJ + erfc pair forces over the neighbour lists.
 //
 // L consecutive threads share one atom (cell-sorted order); each lane walks the
-// atom's list row, whose 9 column segments it treats as one concatenated list
-// (lane `sub` takes positions sub, sub + L, ...), gathers neighbour positions
+// atom's list row (lane `sub` takes positions sub, sub + L, ...), gathers neighbour positions
 // from the sorted double4 array (resident in L2) and keeps its partial sums in
 // registers; the L partials are combined with a fixed xor-shuffle tree.
 // Forces are gathered, never scattered: no atomics, deterministic sums.
+// The gathers bound it (54 us at 30,000 water atoms, 355 at 300,000 mixed): a
+// loop of 15 % fewer instructions with one position less in flight ran at 52.5
+// and 414 us.
 //
 // Formulas (FP64; the mixed-precision variant evaluates the pair scalar in FP32):
 //   VERLET plain    ComputeNearForceVerletVirialWorklet, RunWorklet.cpp:2890-2985
