@@ -390,8 +390,11 @@ rbmd_status ensure_nbr(rbmd_sys* s, int cap) {
     row = round_up(export_cap, kMaxLanes);
     if (row < s->v.rs_num + 1) return fail(RBMD_ERR_ARG, "RBL capacity %d below the core region %d", cap, s->v.rs_num);
   } else {
-    row = 9 * round_up(cap > 0 ? cap : default_cap(s), kMaxLanes);
-    export_cap = cap > 0 ? cap : row;
+    const int64_t slots = 9 * (int64_t)round_up(cap > 0 ? cap : default_cap(s), kMaxLanes);
+    export_cap = cap > 0 ? cap : (int)slots;
+    // 27 n entries are all there can be, so a wavefront's rows stay below the
+    // 2^32 bytes the list kernels address whatever width is asked for
+    row = (int)std::min<int64_t>(slots, round_up(27 * s->n, kMaxLanes));
   }
   s->export_cap = export_cap;
   if (s->v.nbr && row == s->v.cap) return RBMD_OK;

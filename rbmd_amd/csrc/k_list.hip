@@ -224,12 +224,12 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
   }
   const unsigned long long mine = fits >> (a0 - wg0);
   // the wavefront's rows as a buffer, and where each atom's next entry goes
-  // (bytes; 8 rows are below 2^31)
+  // (bytes)
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
-      s.nbr + nbr_index(0, first, s.cap), (short)0, 4 * s.cap * nmine, 0x00020000);
-  int at4[kListAtoms];
+      s.nbr + nbr_index(0, first, s.cap), (short)0, (int)(4u * (unsigned)s.cap * (unsigned)nmine), 0x00020000);
+  unsigned at4[kListAtoms];
 #pragma unroll
-  for (int a = 0; a < kListAtoms; ++a) at4[a] = 4 * a * s.cap;
+  for (int a = 0; a < kListAtoms; ++a) at4[a] = 4u * a * (unsigned)s.cap;
 
   for (int base = 0; base < total; base += kListWindow) {
     // this wavefront's quarter of the window: loads back to back
@@ -336,15 +336,15 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
       // into the next rows of the wavefront, but no further.
 #pragma unroll
       for (int a = 0; a < kListAtoms; ++a) {
-        const unsigned off = 4u * (unsigned)lanes_below(bal[a]) + (unsigned)at4[a];
+        const unsigned off = 4u * (unsigned)lanes_below(bal[a]) + at4[a];
         __builtin_amdgcn_raw_buffer_store_b32((unsigned)entry, rows, lane_in(bal[a]) ? off : 0xfffffff0u, 0, 0);
-        at4[a] += 4 * __popcll(bal[a]);
+        at4[a] += 4u * (unsigned)__popcll(bal[a]);
       }
     }
   }
 #pragma unroll
   for (int a = 0; a < kListAtoms; ++a)
-    if (a < nmine && ((mine >> a) & 1ull) && lane == 0) list_finish(s, first + a, (at4[a] - 4 * a * s.cap) / 4);
+    if (a < nmine && ((mine >> a) & 1ull) && lane == 0) list_finish(s, first + a, (int)((at4[a] - 4u * a * (unsigned)s.cap) / 4u));
 }
 
 __global__ __launch_bounds__(kBlock) void k_nbr_build_verlet(SysView s) { list_body(s, (int)blockIdx.x); }

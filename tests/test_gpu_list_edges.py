@@ -80,3 +80,14 @@ def test_export_width(ctx):
     assert same_lists(g, o, longest).max() == longest
     with pytest.raises(RbmdError):
         g.neighbors(longest - 1)
+
+
+def test_wide_rows(ctx):
+    """an export width beyond all candidates there are, and one near 2^28"""
+    s = make_salt(n_ions=64, seed=3)
+    g, o = pair(ctx, s, salt_config(cut_off=2.0, r_core=2.0))
+    same_lists(g, o, 27 * 64 + 100)
+    g.build_neighbors(1 << 28)
+    near = g.neighbor_entries()
+    g.build_neighbors(0)
+    assert near == g.neighbor_entries() > 0
