@@ -453,18 +453,20 @@ rbmd_status read_status(rbmd_sys* s, int* st) {
   return RBMD_OK;
 }
 
-// staging for n atoms: all arrays of a call for small systems (21 doubles a
-// state), parts of 1 MiB for large ones
+// Staging for n atoms: all arrays of a call for small systems (12 words an
+// atom), parts of 1 MiB for large ones.  Coherent memory, and events that
+// release to the system: what the kernels wrote is the host's to read once the
+// event is reached.
 constexpr size_t kPinMost = size_t(1) << 20;
 rbmd_status pin_create(rbmd_sys* s) {
   s->pin_bytes = std::min(kPinMost, std::max<size_t>(4096, (size_t)s->n * 12 * sizeof(double)));
   for (int h = 0; h < 2; ++h) {
-    if (hipHostMalloc((void**)&s->pin[h], s->pin_bytes) != hipSuccess) return fail(RBMD_ERR_OOM, "hipHostMalloc staging");
-    if (hipEventCreateWithFlags(&s->pin_ev[h], hipEventDisableTiming) != hipSuccess)
+    if (hipHostMalloc((void**)&s->pin[h], s->pin_bytes, hipHostMallocCoherent) != hipSuccess) return fail(RBMD_ERR_OOM, "hipHostMalloc staging");
+    if (hipEventCreateWithFlags(&s->pin_ev[h], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess)
       return fail(RBMD_ERR_HIP, "hipEventCreate");
   }
   const size_t rows = (size_t)((s->n + kBlock - 1) / kBlock) * kRowBond;
-  if (hipHostMalloc((void**)&s->small, sizeof(ThermoOut) + rows * sizeof(double)) != hipSuccess)
+  if (hipHostMalloc((void**)&s->small, sizeof(ThermoOut) + rows * sizeof(double), hipHostMallocCoherent) != hipSuccess)
     return fail(RBMD_ERR_OOM, "hipHostMalloc staging");
   s->bond_rows = (double*)(s->small + 1);
   return RBMD_OK;
