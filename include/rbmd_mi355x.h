@@ -288,8 +288,8 @@ rbmd_status rbmd_md_energy_noalloc(rbmd_sys* sys);
  * thermostats, energy_every 0, sampled (not injected) RBE k vectors or Ewald,
  * and agree on force field, special-bond mode, precision, SHAKE and
  * thermostat; sizes, boxes and step counts may differ.  A pack keeps the
- * systems' device pointers: do not resize, re-initialise or destroy a system
- * while a pack holds it. ---- */
+ * systems' device pointers (a list built at another width is followed): do not
+ * resize, re-initialise or destroy a system while a pack holds it. ---- */
 rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n, rbmd_pack** out);
 rbmd_status rbmd_pack_destroy(rbmd_pack* pack);
 rbmd_status rbmd_pack_step(rbmd_pack* pack, int64_t n_steps);    /* n packed steps, launched kernel by kernel */

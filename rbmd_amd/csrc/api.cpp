@@ -2212,6 +2212,7 @@ struct rbmd_pack {
   PackSig sig{};
   int tc = 0;
   bool ring = false, nh = false, shake = false, scale_v = false, has_k = false, has_b = false;
+  std::vector<PackSys> tab;  // host copy of dsys
   PackSys* dsys = nullptr;
   int* dmap = nullptr;
   int* dfirst = nullptr;
@@ -2360,7 +2361,8 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
     p->allocs.push_back(*q);
     return RBMD_OK;
   };
-  std::vector<PackSys> tab(n);
+  std::vector<PackSys>& tab = p->tab;
+  tab.resize(n);
   std::vector<int> first((size_t)PK_COUNT * (n + 1));
   std::vector<std::vector<int>> blocks(PK_COUNT, std::vector<int>(n, 0));
   for (int k = 0; k < n; ++k) {
@@ -2457,10 +2459,29 @@ rbmd_status rbmd_pack_destroy(rbmd_pack* p) {
   return pack_fail_free(p, RBMD_OK);
 }
 
+// A member whose lists were built at another width since (rbmd_neighbors_build)
+// has new rows: the table follows.  Captured steps read the table as they run,
+// so they stay valid.
+static rbmd_status pack_lists(rbmd_pack* p) {
+  bool moved = false;
+  for (size_t k = 0; k < p->sys.size(); ++k) {
+    const SysView& now = p->sys[k]->v;
+    SysView& v = p->tab[k].v;
+    moved |= v.nbr != now.nbr || v.cap != now.cap;
+    v.nbr = now.nbr;
+    v.cap = now.cap;
+  }
+  if (!moved) return RBMD_OK;
+  HIP_TRY(hipMemcpyAsync(p->dsys, p->tab.data(), sizeof(PackSys) * p->tab.size(), hipMemcpyHostToDevice, p->ctx->stream));
+  HIP_TRY(hipStreamSynchronize(p->ctx->stream));
+  return RBMD_OK;
+}
+
 // n packed steps; graph: replay one captured packed step
 static rbmd_status pack_steps(rbmd_pack* p, int64_t n_steps, bool graph) {
   if (!p) return fail(RBMD_ERR_ARG, "null pack");
   hipStream_t st = p->ctx->stream;
+  RC_TRY(pack_lists(p));
   for (int thermo = 0; graph && thermo < 2; ++thermo) {
     if (p->graph[thermo]) continue;
     const bool prof = p->ctx->prof;
