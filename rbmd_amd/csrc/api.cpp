@@ -1590,13 +1590,18 @@ rbmd_status rbmd_locator_export(rbmd_sys* s, int32_t* cell_of, int32_t* point_id
   return status_to_rc(stt);
 }
 
+// the lists, into the rows there are
+static rbmd_status build_lists(rbmd_sys* s) {
+  s->ctx->run("nbr_build", [&] { launch_nbr_build(s->v, s->ctx->stream); });
+  s->nbr_built = true;
+  return check_launch("neighbors_build");
+}
+
 rbmd_status rbmd_neighbors_build(rbmd_sys* s, int32_t cap) {
   if (!s) return fail(RBMD_ERR_ARG, "null sys");
   if (!s->locator_built || s->skin_active) RC_TRY(rbmd_locator_build(s));
   RC_TRY(ensure_nbr(s, cap));
-  s->ctx->run("nbr_build", [&] { launch_nbr_build(s->v, s->ctx->stream); });
-  s->nbr_built = true;
-  return check_launch("neighbors_build");
+  return build_lists(s);
 }
 
 rbmd_status rbmd_neighbors_export(rbmd_sys* s, int32_t cap, int32_t* ids, double* offsets, int32_t* num) {
@@ -1675,7 +1680,9 @@ rbmd_status rbmd_force_real(rbmd_sys* s, double* force, double* vir, double* elj
   if (s->fused) {
     if (!s->locator_built) RC_TRY(rbmd_locator_build(s));
   } else if (!s->nbr_built) {
-    RC_TRY(rbmd_neighbors_build(s, s->v.cap));
+    if (!s->locator_built) RC_TRY(rbmd_locator_build(s));
+    s->export_cap = s->v.cap;  // a whole row
+    RC_TRY(build_lists(s));
   }
   launch_real(s, 1, 1);
   RC_TRY(check_launch("force_real"));

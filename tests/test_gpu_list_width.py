@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from rbmd_amd.lib import GpuSystem, Pack
-from tests.systems import salt, salt_run
+from tests.systems import salt, salt_run, water, water_run
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +33,25 @@ def test_pack_follows_a_member_list_of_another_width(ctx, graph):
     for a, b in zip(*out):
         for u, v in zip(a, b):
             assert np.array_equal(u, v)
+
+
+@pytest.mark.parametrize("make", [lambda: (salt(n=600, seed=3), salt_run()), lambda: (water(nmol=200, seed=5), water_run()),
+                                  lambda: (salt(n=2000, seed=3),
+                                           salt_run(neighbor_type="RBL", cut_off=5.0, r_core=2.5, neighbor_sample_num=50))],
+                         ids=["salt", "water", "rbl"])
+def test_real_force_keeps_the_rows(ctx, make):
+    """force_real without a list builds one in the rows there are: neither the
+    rows nor the memory held grow over new configurations"""
+    s, r = make()
+    g = GpuSystem(ctx, s, r)
+    g.md_init()
+    held, ref = g.footprint(), None
+    for _ in range(3):
+        g.set_state(s.x)
+        f = g.force_real()[0]
+        assert g.footprint() == held
+        ref = f if ref is None else ref
+        assert np.array_equal(f, ref)
+    g.md_step(2)
+    assert g.footprint() == held
+    g.close()
