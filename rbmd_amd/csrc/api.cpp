@@ -232,7 +232,10 @@ struct rbmd_sys {
     size_t b = std::max<size_t>(count, 1) * sizeof(T);
     void* q = nullptr;
     hipError_t e = hipMalloc(&q, b);
-    if (e != hipSuccess) return fail(RBMD_ERR_OOM, "hipMalloc(%zu bytes): %s", b, hipGetErrorString(e));
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next launch's check
+      return fail(RBMD_ERR_OOM, "hipMalloc(%zu bytes): %s", b, hipGetErrorString(e));
+    }
     allocs.push_back(q);
     bytes += (int64_t)b;
     *ptr = (T*)q;
@@ -405,9 +408,19 @@ rbmd_status ensure_nbr(rbmd_sys* s, int cap) {
     (void)hipFree(s->v.nbr);
     s->v.nbr = nullptr;
   }
+  const int old = s->v.cap;
   s->v.cap = row;
   s->graph_ok = false;
-  return s->dalloc(&s->v.nbr, (size_t)s->v.cap * s->n);
+  const rbmd_status rc = s->dalloc(&s->v.nbr, (size_t)row * s->n);
+  if (rc != RBMD_OK && old > 0) {  // no room: the old rows again, so that the system stays usable
+    const std::string why = g_last_error;
+    s->v.cap = old;
+    s->export_cap = old;
+    s->nbr_built = false;
+    if (s->dalloc(&s->v.nbr, (size_t)old * s->n) != RBMD_OK) s->initialized = false;
+    g_last_error = why;
+  }
+  return rc;
 }
 
 // Put the reference geometry (per-step list) or the skin geometry into the
@@ -1680,6 +1693,7 @@ rbmd_status rbmd_force_real(rbmd_sys* s, double* force, double* vir, double* elj
   if (s->fused) {
     if (!s->locator_built) RC_TRY(rbmd_locator_build(s));
   } else if (!s->nbr_built) {
+    if (!s->v.nbr) RC_TRY(ensure_nbr(s, 0));
     if (!s->locator_built) RC_TRY(rbmd_locator_build(s));
     s->export_cap = s->v.cap;  // a whole row
     RC_TRY(build_lists(s));
@@ -1853,6 +1867,7 @@ rbmd_status rbmd_force_bonded(rbmd_sys* s, double* force, double* eb, double* ea
 // ExecutionNVT::Init: locator, k-set of step 0, dof/NHC SetUp, first force
 rbmd_status rbmd_md_init(rbmd_sys* s) {
   if (!s) return fail(RBMD_ERR_ARG, "null sys");
+  if (!s->v.nbr) RC_TRY(ensure_nbr(s, 0));
   rbmd_ctx* c = s->ctx;
   hipStream_t st = c->stream;
   launch_fill_int(s->v.status, 0, 1, st);
@@ -2474,6 +2489,7 @@ static rbmd_status pack_lists(rbmd_pack* p) {
   for (size_t k = 0; k < p->sys.size(); ++k) {
     const SysView& now = p->sys[k]->v;
     SysView& v = p->tab[k].v;
+    if (!now.nbr) return fail(RBMD_ERR_OOM, "system %d holds no list rows", (int)k);
     moved |= v.nbr != now.nbr || v.cap != now.cap;
     v.nbr = now.nbr;
     v.cap = now.cap;

@@ -3,7 +3,7 @@ need a list keep the rows there are."""
 import numpy as np
 import pytest
 
-from rbmd_amd.lib import GpuSystem, Pack
+from rbmd_amd.lib import GpuSystem, Pack, RbmdError
 from tests.systems import salt, salt_run, water, water_run
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +55,23 @@ def test_real_force_keeps_the_rows(ctx, make):
     g.md_step(2)
     assert g.footprint() == held
     g.close()
+
+
+def test_a_width_that_does_not_fit_leaves_the_system_usable(ctx):
+    """rows wider than the card's memory are refused, and the steps that follow
+    are those of a system that was never asked"""
+    s = salt(n=70000, seed=4)  # rows of 27 n entries: 529 GB
+    out = []
+    for asked in (False, True):
+        g = GpuSystem(ctx, s, salt_run())
+        g.md_init()
+        held = g.footprint()
+        if asked:
+            with pytest.raises(RbmdError, match="hipMalloc"):
+                g.build_neighbors(2_000_000)
+            assert g.footprint() == held
+        g.md_step(2)
+        out.append(g.state())
+        g.close()
+    for u, v in zip(*out):
+        assert np.array_equal(u, v)
