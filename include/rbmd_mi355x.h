@@ -266,6 +266,11 @@ rbmd_status rbmd_md_run_graph(rbmd_sys* sys, int64_t n_steps);
 rbmd_status rbmd_md_enqueue(rbmd_sys* sys, int64_t n_steps);
 rbmd_status rbmd_md_wait(rbmd_sys* sys);
 rbmd_status rbmd_md_query(rbmd_sys* sys, int32_t* idle);
+/* how a system's steps form the real-space forces: stored lists, the fused pass
+ * of pair_path CELLS, straight from the cells on the steps between thermo rows
+ * (small dense systems, same sums as lists), random-batch lists */
+enum { RBMD_PATH_LISTS = 0, RBMD_PATH_CELLS = 1, RBMD_PATH_COMPACT = 2, RBMD_PATH_RBL = 3 };
+rbmd_status rbmd_md_path(const rbmd_sys* sys, int32_t* path);
 rbmd_status rbmd_md_thermo(rbmd_sys* sys, rbmd_thermo* out);
 rbmd_status rbmd_md_energy(rbmd_sys* sys); /* evaluate e_long now (ComputeEwaldEnergy) */
 /* rbmd_md_energy without device allocation.  No counterpart in the reference:

@@ -2164,6 +2164,12 @@ rbmd_status rbmd_md_query(rbmd_sys* s, int32_t* idle) {
   return RBMD_OK;
 }
 
+rbmd_status rbmd_md_path(const rbmd_sys* s, int32_t* path) {
+  if (!s || !path) return fail(RBMD_ERR_ARG, "null argument");
+  *path = s->v.rbl ? RBMD_PATH_RBL : s->fused ? RBMD_PATH_CELLS : s->v.compact ? RBMD_PATH_COMPACT : RBMD_PATH_LISTS;
+  return RBMD_OK;
+}
+
 rbmd_status rbmd_md_thermo(rbmd_sys* s, rbmd_thermo* o) {
   if (!s || !o) return fail(RBMD_ERR_ARG, "bad arguments");
   launch_thermo_out(s->nhc, s->v.misfit_count, s->v.status, s->shake_iter, s->v.list_builds, s->small, s->ctx->stream);

@@ -429,6 +429,18 @@ __global__ __launch_bounds__(kWave << 4) void k_compact_finish(SysView s, IntVie
   if (threadIdx.x < kWave) second_half_wave(s, iv, 1, 1, has_b, rows_ke, (int)blockIdx.x);  // its own lanes' forces
 }
 
+// More atoms share each candidate load and the set-up, fewer atoms and a
+// split stream give a small system more wavefronts.
+int stencil_choice(const SysView& s) {
+  const double cand = 27.0 * s.n / s.ncell;  // stencil candidates per atom
+  if (cand > 2000) return s.n <= 1000 ? 0 : 1;
+  return s.n <= 3000 ? 2 : 3;
+}
+
+static int64_t stencil_blocks_of(const SysView& s, int cfg) {
+  return s.n_items * (int64_t)(kChunk * stencil_split(cfg) / (kStWaves << stencil_lga(cfg)));
+}
+
 // The list build and the pair kernel are two dependent launches whose length
 // on a small system is one wavefront's serial work; here that is one launch
 // with the work spread over as many wavefronts as help.  The candidate test
@@ -437,22 +449,23 @@ __global__ __launch_bounds__(kWave << 4) void k_compact_finish(SysView s, IntVie
 // 600 ions 30.4 / 16.4, 2,000 36.7 / 17.9, 4,000 33.5 / 21.7, 8,000 33.0 /
 // 29.9; water 600 atoms 118 / 46, 1,800 70 / 51, 3,000 57 / 54, 6,000 mixed
 // 77 / 104.
+//
+// Three lines: on the number of candidates; on the atoms, as the list build
+// has the chip full from about 8,000 on whatever the candidates (steps with
+// lists and with this kernel, us: 8,000 ions 70 / 61 at 1,000 candidates, 75 /
+// 75 at 216; 14,000 81 / 88 at 519, 84 / 106 at 172; 20,000 89 / 124 at 246);
+// and on the workgroups, a fixed number per cell and its atoms, most of them
+// empty where a cell holds few: 600 ions in 125 cells 74 / 47, in 729 75 / 82;
+// 2,000 in 216 75 / 61, in 512 78 / 82, in 2,197 83 / 183; 4,000 in 1,000 80 /
+// 65, in 4,913 91 / 114.
+constexpr int kStAtoms = 8000, kStAtomsCrowded = 2400, kStBlocks = 5000;
 bool stencil_pays(const SysView& s) {
-  const double cand = 27.0 * s.n / s.ncell;  // stencil candidates per atom
-  return cand > 2000 ? s.n <= 2400 : (double)s.n * cand <= 8e6;
-}
-
-// More atoms share each candidate load and the set-up, fewer atoms and a
-// split stream give a small system more wavefronts.
-int stencil_choice(const SysView& s) {
   const double cand = 27.0 * s.n / s.ncell;
-  if (cand > 2000) return s.n <= 1000 ? 0 : 1;
-  return s.n <= 3000 ? 2 : 3;
+  if (stencil_blocks_of(s, stencil_choice(s)) > kStBlocks) return false;
+  return cand > 2000 ? s.n <= kStAtomsCrowded : s.n <= kStAtoms && (double)s.n * cand <= 8e6;
 }
 
-int stencil_blocks(const SysView& s) {
-  return s.n_items * (kChunk * stencil_split(s.st_cfg) / (kStWaves << stencil_lga(s.st_cfg)));
-}
+int stencil_blocks(const SysView& s) { return (int)stencil_blocks_of(s, s.st_cfg); }
 
 template <int MODE, int SP, bool F32>
 void launch_compact_cfg(const SysView& s, const IntView& iv, const KView& k, hipStream_t st, int n_pair, int n_rho,

@@ -24,7 +24,7 @@ EXPORTS = [
     "rbmd_locator_export", "rbmd_neighbors_build", "rbmd_neighbors_count", "rbmd_neighbors_capacity", "rbmd_neighbors_export", "rbmd_force_real",
     "rbmd_rbe_set_kvectors", "rbmd_rbe_sample", "rbmd_rbe_sample_host", "rbmd_rbe_S",
     "rbmd_rbe_structure_factor", "rbmd_rbe_force", "rbmd_ewald_force", "rbmd_force_bonded", "rbmd_md_init",
-    "rbmd_md_step", "rbmd_md_run_graph", "rbmd_md_enqueue", "rbmd_md_wait", "rbmd_md_query", "rbmd_md_thermo", "rbmd_md_energy",
+    "rbmd_md_step", "rbmd_md_run_graph", "rbmd_md_enqueue", "rbmd_md_wait", "rbmd_md_query", "rbmd_md_path", "rbmd_md_thermo", "rbmd_md_energy",
     "rbmd_md_energy_noalloc", "rbmd_profile_enable",
     "rbmd_profile_reset", "rbmd_profile_get", "rbmd_abi_sizeof", "rbmd_pack_create", "rbmd_pack_destroy",
     "rbmd_pack_step", "rbmd_pack_enqueue", "rbmd_pack_wait", "rbmd_static_table_gnear",
@@ -80,6 +80,7 @@ def load():
     L.rbmd_md_enqueue.argtypes = [vp, C.c_int64]
     L.rbmd_md_wait.argtypes = [vp]
     L.rbmd_md_query.argtypes = [vp, C.POINTER(C.c_int32)]
+    L.rbmd_md_path.argtypes = [vp, pi]
     L.rbmd_md_thermo.argtypes = [vp, C.POINTER(Thermo)]
     L.rbmd_md_energy.argtypes = [vp]
     L.rbmd_md_energy_noalloc.argtypes = [vp]
@@ -335,6 +336,12 @@ class GpuSystem:
         idle = C.c_int32()
         check(self.L.rbmd_md_query(self.h, C.byref(idle)))
         return bool(idle.value)
+
+    def md_path(self):
+        """how the steps form the real-space forces: lists, cells, compact or rbl"""
+        path = C.c_int32()
+        check(self.L.rbmd_md_path(self.h, C.byref(path)))
+        return ("lists", "cells", "compact", "rbl")[path.value]
 
     def thermo(self):
         t = Thermo()

@@ -1,0 +1,34 @@
+"""Which systems take the stencil pair kernel: dense ones of up to a few thousand
+atoms.  Where the lists were measured faster (sparse cells, more atoms) a
+system keeps them, and a large empty box builds no table of its cells."""
+import numpy as np
+import pytest
+
+from rbmd_amd import make_salt, salt_config
+from rbmd_amd.lib import GpuSystem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,density,cut,path", [
+    (600, 0.5, 4.0, "compact"), (4000, 0.5, 4.0, "compact"), (8000, 0.5, 4.0, "compact"),  # 8, 125, 216 cells
+    (8002, 0.5, 4.0, "lists"), (9000, 0.5, 4.0, "lists"),
+    (4000, 0.8, 2.5, "compact"), (2000, 0.5, 2.5, "compact"),                               # 216 cells
+    (1000, 0.05, 2.5, "lists"), (4000, 0.02, 2.5, "lists"),                                 # 1,000 and 12,167 cells
+    (14000, 0.2, 2.5, "lists"), (20000, 0.5, 2.5, "lists"),                                 # 4,096 and 2,197 cells
+])
+def test_path_by_size_and_density(ctx, n, density, cut, path):
+    g = GpuSystem(ctx, make_salt(n_ions=n, density=density, seed=2), salt_config(cut_off=cut, r_core=cut))
+    assert g.md_path() == path
+    g.close()
+
+
+def test_empty_box_holds_little(ctx):
+    """1,000 ions in 64,000 cells: no more than the lists and the cells"""
+    s, r = make_salt(n_ions=1000, density=0.001, seed=2), salt_config(cut_off=2.5, r_core=2.5)
+    g = GpuSystem(ctx, s, r)
+    assert g.footprint() < 20e6
+    g.md_init()
+    g.md_step(3)
+    assert np.isfinite(g.state()[2]).all()
+    g.close()
