@@ -1233,21 +1233,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   A(s->dalloc(&v.spos, n));
   if (v.compact) {
     A(s->dalloc(&v.spos32, n));
-    // stencil cells of every cell, x offset outermost, then y, then z: the
-    // wrapped cell and the image shift + 2 per axis (2 bits each)
-    std::vector<int> tab((size_t)v.ncell * 32, -1);
-    for (int c = 0; c < v.ncell; ++c)
-      for (int k = 0; k < 27; ++k) {
-        int at[3] = {c % v.dims[0] + k / 9 - 1, (c / v.dims[0]) % v.dims[1] + (k / 3) % 3 - 1,
-                     c / (v.dims[0] * v.dims[1]) + k % 3 - 1};
-        int code = 0;
-        for (int d = 0; d < 3; ++d) {
-          const int w = (at[d] + v.dims[d]) % v.dims[d];
-          code |= ((w - at[d]) / v.dims[d] + 2) << (2 * d);
-          at[d] = w;
-        }
-        tab[(size_t)c * 32 + k] = (at[0] + at[1] * v.dims[0] + at[2] * v.dims[0] * v.dims[1]) << 6 | code;
-      }
+    const std::vector<int> tab = stencil_table(v);
     int* dt = nullptr;
     A(s->upload(&dt, tab.data(), tab.size()));
     v.stencil_tab = dt;

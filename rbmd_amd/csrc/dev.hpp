@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "ewald.hpp"
 
 struct rbmd_ctx;  // the C ABI's context (include/rbmd_mi355x.h), defined in api.cpp
@@ -96,7 +98,7 @@ struct SysView {
   int *cursor;      // [ncell]
   int *point_ids;   // [n] sorted position -> atom id
   int *rank;        // [n] atom id -> sorted position
-  const int* stencil_tab;  // [ncell][32] compact: stencil cells 0..26 of every cell (cell << 6 | shift code)
+  const int* stencil_tab;  // [ncell][32] compact: stencil cells 0..26 of every cell (cell above shift code)
   int *items;       // [n_items] packed (cell << 8 | chunk)
   int *n_items_dev; // [1]
   int *misfit;      // [n] sorted position flag
@@ -211,6 +213,7 @@ void launch_pair(const SysView& s, hipStream_t st, int thermo, int peratom, doub
 int pair_blocks(const SysView& s);
 bool stencil_pays(const SysView& s);  // the rule for compact systems
 int stencil_choice(const SysView& s);
+std::vector<int> stencil_table(const SysView& s);  // SysView::stencil_tab
 // RBL energies over a full rc stencil (no list) and the pair thermo rows
 // (energies + the mean-removed RBL virial); e_lj/e_coul per atom when peratom
 void launch_rbl_energy(const SysView& s, hipStream_t st, int peratom, double* rows, int* nblocks);

@@ -64,10 +64,34 @@ __device__ __forceinline__ double lane_double(double v, int l) {
                           __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
-// LDS list entry: sorted index (22 bits), type (4 bits), image shift + 2 per
-// axis (2 bits each, 1..3, so an entry is never 0)
-constexpr int kStIdx = 10, kStType = 6;
-__device__ __forceinline__ int st_code(int sa, int sb, int sc) { return (sa + 2) | ((sb + 2) << 2) | ((sc + 2) << 4); }
+// LDS list entry: sorted index (19 bits, n at most kStAtoms), type (4 bits),
+// image shift + 4 per axis (3 bits each, 1..7 as stencil_cell gives -3..3, so
+// an entry is never 0)
+constexpr int kStType = 9, kStIdx = kStType + 4, kStZero = 4;
+__host__ __device__ __forceinline__ int st_code(int sa, int sb, int sc) {
+  return (sa + kStZero) | ((sb + kStZero) << 3) | ((sc + kStZero) << 6);
+}
+__device__ __forceinline__ int st_shift(int e, int axis) { return ((e >> (3 * axis)) & 7) - kStZero; }
+
+// Stencil cells of every cell of the grid, x offset outermost, then y, then z
+// (32 slots a cell, 27 used): the wrapped cell above its image shift code.
+std::vector<int> stencil_table(const SysView& s) {
+  std::vector<int> tab((size_t)s.ncell * 32, -1);
+  for (int c = 0; c < s.ncell; ++c)
+    for (int k = 0; k < 27; ++k) {
+      int at[3] = {c % s.dims[0] + k / 9 - 1, (c / s.dims[0]) % s.dims[1] + (k / 3) % 3 - 1,
+                   c / (s.dims[0] * s.dims[1]) + k % 3 - 1};
+      int shift[3];
+      for (int d = 0; d < 3; ++d) {
+        const int w = (at[d] + s.dims[d]) % s.dims[d];
+        shift[d] = (w - at[d]) / s.dims[d];
+        at[d] = w;
+      }
+      tab[(size_t)c * 32 + k] =
+          (at[0] + at[1] * s.dims[0] + at[2] * s.dims[0] * s.dims[1]) << kStType | st_code(shift[0], shift[1], shift[2]);
+    }
+  return tab;
+}
 
 template <int MODE, int SP, bool F32, int CFG>
 __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
@@ -153,6 +177,7 @@ __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
   while (main_pass || todo != 0ull) {  // the same passes on every wavefront of NS = 4
     // this pass's atoms and their cell
     int ca, cb, cc, only = -1;
+    bool out = false;  // the atom has left the box, by any number of lengths: the FP64 predicate throughout
     if (main_pass) {
       ca = c % s.dims[0];
       cb = (c / s.dims[0]) % s.dims[1];
@@ -164,6 +189,7 @@ __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
       ca = cell_axis(lane_double(pi.x, l), s.lo[0], s.dxdydz[0]);
       cb = cell_axis(lane_double(pi.y, l), s.lo[1], s.dxdydz[1]);
       cc = cell_axis(lane_double(pi.z, l), s.lo[2], s.dxdydz[2]);
+      out = min(ca, min(cb, cc)) < 0 || ca >= s.dims[0] || cb >= s.dims[1] || cc >= s.dims[2];
     }
     main_pass = false;
     // candidates and atoms in FP32 around the cell's centre, both from the
@@ -190,9 +216,9 @@ __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
     if (only < 0) {
       const int e = s.stencil_tab[c * 32 + (lane & 31)];
       if (lane < 27) {
-        js = s.cell_start[e >> 6];
-        num = s.cell_start[(e >> 6) + 1] - js;
-        code = e & 63;
+        js = s.cell_start[e >> kStType];
+        num = s.cell_start[(e >> kStType) + 1] - js;
+        code = e & ((1 << kStType) - 1);
       }
     } else if (lane < 27) {
       const StencilCell t = stencil_cell(s, ca, cb, cc, lane / 9 - 1, (lane / 3) % 3 - 1, lane % 3 - 1);
@@ -251,14 +277,14 @@ __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
         if (base < stop) nxt = locate();  // in flight over this batch's tests
         float cx = c4.x - gx, cy = c4.y - gy, cz = c4.z - gz;
         if (shifts) {
-          cx -= (float)((cd & 3) - 2) * s.shift32[0];
-          cy -= (float)(((cd >> 2) & 3) - 2) * s.shift32[1];
-          cz -= (float)(((cd >> 4) & 3) - 2) * s.shift32[2];
+          cx -= (float)st_shift(cd, 0) * s.shift32[0];
+          cy -= (float)st_shift(cd, 1) * s.shift32[1];
+          cz -= (float)st_shift(cd, 2) * s.shift32[2];
         }
         float c2 = fmaf(cx, cx, fmaf(cy, cy, cz * cz));
         c2 = j < 0 ? 1e30f : c2;
         const int entry = (j << kStIdx) | (__float_as_int(c4.w) << kStType) | cd;
-        unsigned long long bal[A], near = 0ull;
+        unsigned long long bal[A], near = out ? ~0ull : 0ull;
 #pragma unroll
         for (int a = 0; a < A; ++a) {
           const float d2 = fmaf(cx, mx[a], fmaf(cy, my[a], fmaf(cz, mz[a], c2 + aa[a])));
@@ -267,9 +293,9 @@ __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
         }
         if (near != 0ull) {  // some lane's decision is the FP64 predicate's (the atom itself among them)
           const double4 pj = st_double4(rpos, 32u * (unsigned)j);
-          const double x = pj.x - (double)((cd & 3) - 2) * s.shift_len[0];
-          const double y = pj.y - (double)(((cd >> 2) & 3) - 2) * s.shift_len[1];
-          const double z = pj.z - (double)(((cd >> 4) & 3) - 2) * s.shift_len[2];
+          const double x = pj.x - (double)st_shift(cd, 0) * s.shift_len[0];
+          const double y = pj.y - (double)st_shift(cd, 1) * s.shift_len[1];
+          const double z = pj.z - (double)st_shift(cd, 2) * s.shift_len[2];
 #pragma unroll
           for (int a = 0; a < A; ++a) {
             const double d2 = dist2(x - lane_double(pi.x, a * L), y - lane_double(pi.y, a * L),
@@ -347,9 +373,9 @@ __device__ __forceinline__ void stencil_body(const SysView& s, const int bid) {
             const unsigned e = h == 0 ? ea : eb;
             if (e == 0u) continue;
             const double4 p = h == 0 ? pa : pb;
-            const double ox = (double)((int)(e & 3) - 2) * s.shift_len[0];
-            const double oy = (double)((int)((e >> 2) & 3) - 2) * s.shift_len[1];
-            const double oz = (double)((int)((e >> 4) & 3) - 2) * s.shift_len[2];
+            const double ox = (double)st_shift((int)e, 0) * s.shift_len[0];
+            const double oy = (double)st_shift((int)e, 1) * s.shift_len[1];
+            const double oz = (double)st_shift((int)e, 2) * s.shift_len[2];
             double rx = (p.x - ox) - pi.x;
             double ry = (p.y - oy) - pi.y;
             double rz = (p.z - oz) - pi.z;

@@ -32,3 +32,29 @@ def test_empty_box_holds_little(ctx):
     g.md_step(3)
     assert np.isfinite(g.state()[2]).all()
     g.close()
+
+
+@pytest.mark.parametrize("n,density,cut,away", [
+    (200, 0.8, 4.0, [(2, 0, 0), (-2, 0, 0), (0, -2, 0), (0, 0, -2), (0, 0, 2), (-3, 2, -2), (3, 3, -3)]),
+    (600, 0.5, 4.0, [(2, 0, 0), (0, 2, 2), (3, 3, 3)]),  # (of two cells, those below the box are refused)
+], ids=["one cell", "two cells"])
+def test_atoms_boxes_away(ctx, n, density, cut, away):
+    """atoms two and three box lengths outside (a step wraps one): their stencils
+    hold image shifts of up to three boxes.  A step by the stencil kernel and
+    one by the lists are two by the lists, to the bit."""
+    s, r = make_salt(n_ions=n, density=density, seed=9), salt_config(cut_off=cut, r_core=cut)
+    x = s.x.copy()
+    for atom, boxes in enumerate(away):
+        x[10 * atom] += np.array(boxes) * s.box
+    out = []
+    for calls in ([2], [1, 1]):
+        g = GpuSystem(ctx, s, r)
+        g.md_init()
+        g.set_state(x)
+        assert g.md_path() == "compact"
+        for k in calls:
+            g.md_step(k)
+        out.append(g.state())
+        g.close()
+    for u, v in zip(*out):
+        assert np.array_equal(u, v)
