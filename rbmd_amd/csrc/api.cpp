@@ -1098,13 +1098,14 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   while (v.cut2 - std::nextafter(v.accept_d2, v.cut2) > 0.0001) v.accept_d2 = std::nextafter(v.accept_d2, v.cut2);
   // The error of the stencil kernel's FP32 d^2 near the cutoff: pairs within it
   // of a threshold are decided in FP64.  Coordinates from the box corner, less the image shift and the
-  // cell's centre, carry at most u (3 L + 5 w) (u = 2^-24, w the cell width,
-  // at least rc); for a pair within rc of an atom of the cell |a| <= 0.87 w
-  // and |c| <= 1.87 w, so |c|^2 - 2 c.a + |a|^2 rounds by at most 45 u w^2,
-  // and the coordinates move d^2 by at most 7 u rc (3 L + 5 w).  Twice that.
+  // cell's centre, carry at most u (3 L + 5 w) (u = 2^-24, w the cell width or
+  // rc, whichever is larger: a box narrower than rc is one cell); for a pair within rc of an atom of the
+  // cell |a| <= 0.87 w and |c| <= 1.87 w, so |c|^2 - 2 c.a + |a|^2 rounds by at
+  // most 45 u w^2, and the coordinates move d^2 by at most 7 u rc (3 L + 5 w).
+  // Twice that.
   {
     const double L = std::max(v.box[0], std::max(v.box[1], v.box[2]));
-    const double wd = std::max(v.dxdydz[0], std::max(v.dxdydz[1], v.dxdydz[2]));
+    const double wd = std::max(v.cut, std::max(v.dxdydz[0], std::max(v.dxdydz[1], v.dxdydz[2])));
     const double band = std::ldexp(45.0 * wd * wd + 7.0 * v.cut * (3.0 * L + 5.0 * wd), -23);
     v.test_band = std::nextafter((float)band, 3e38f);
     for (int k = 0; k < 3; ++k) v.shift32[k] = (float)v.shift_len[k];
