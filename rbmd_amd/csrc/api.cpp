@@ -369,6 +369,29 @@ double column_fraction(double wx, double wy, double rc) {
   return acc * (2.0 * hx / m) * (2.0 * hy / m) / (4.0 / 3.0 * kPi);
 }
 
+// The list predicate cut2 - d2 > 1e-4 as one threshold: the largest d2 it
+// accepts (cut2 - d2, rounded, falls as d2 grows), found by halving the range
+// in the order of the doubles.  Below zero for an rc near 0.01 or less: no pair.
+double accepted_most(double cut2) {
+  auto key = [](double d) {  // -1 < .. < 0 < .. in whole numbers
+    int64_t b;
+    std::memcpy(&b, &d, 8);
+    return b < 0 ? INT64_MIN - b : b;
+  };
+  auto value = [](int64_t k) {
+    const int64_t b = k < 0 ? INT64_MIN - k : k;
+    double d;
+    std::memcpy(&d, &b, 8);
+    return d;
+  };
+  int64_t yes = key(-1.0), no = key(cut2);
+  while (no - 1 > yes) {
+    const int64_t mid = yes + (int64_t)(((uint64_t)no - (uint64_t)yes) / 2);
+    (cut2 - value(mid) > 0.0001 ? yes : no) = mid;
+  }
+  return value(yes);
+}
+
 // Default list capacity.  VERLET: per stencil column, 1.15 x the mean count
 // in the largest column share of the list's cutoff sphere (rc, or rc + skin)
 // + 64; RBL: the core region plus twice the mean shell sample + 64.
@@ -1092,10 +1115,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   v.n_items = v.ncell + n / kChunk + 1;
   v.lds_bins = v.ncell <= 4096 ? 1 : 0;
   v.list_cut2 = v.cut2;
-  // the list predicate as one threshold: cut2 - d2 rounded falls as d2 grows
-  v.accept_d2 = v.cut2 - 0.0001;
-  while (!(v.cut2 - v.accept_d2 > 0.0001)) v.accept_d2 = std::nextafter(v.accept_d2, 0.0);
-  while (v.cut2 - std::nextafter(v.accept_d2, v.cut2) > 0.0001) v.accept_d2 = std::nextafter(v.accept_d2, v.cut2);
+  v.accept_d2 = accepted_most(v.cut2);
   // The error of the stencil kernel's FP32 d^2 near the cutoff: pairs within it
   // of a threshold are decided in FP64.  Coordinates from the box corner, less the image shift and the
   // cell's centre, carry at most u (3 L + 5 w) (u = 2^-24, w the cell width or
@@ -1148,6 +1168,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   // 138 and 167; water (mixed) 300,000 457, 381 and 359
   v.lanes_lg = n <= 60000 ? 4 : 3;
   v.compact = p->coulomb_type != RBMD_COULOMB_EWALD && !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes && stencil_pays(v) ? 1 : 0;
+  if (v.accept_d2 - v.test_band <= 1e-4 + 2.0 * v.test_band) v.compact = 0;  // an FP32 test has no room at such an rc
   v.st_cfg = stencil_choice(v);
   if (p->pair_lanes) v.lanes_lg = p->pair_lanes == 4 ? 2 : (p->pair_lanes == 8 ? 3 : 4);
   if (v.compact) v.lanes_lg = 4;  // as the stencil kernel sums

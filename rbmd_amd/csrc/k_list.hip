@@ -194,13 +194,14 @@ __device__ __forceinline__ void list_body(const SysView& s, const int bid) {
   // Error of the FP32 d^2 near the cutoff, u = 2^-24, S the largest |a| + |c|:
   // rounded coordinates move it by 2 u S^2, |c|^2 and |a|^2 by 3 u S^2, the
   // four sums by 4 u S^2 (8 if products are rounded apart); 32 u S^2 is more
-  // than twice that.  A box so large that the band is not small takes the FP64
+  // than twice that.  A box so large that the band is not small, or an rc so
+  // near 0.01 that nothing lies clear of both thresholds, takes the FP64
   // predicate throughout.
   const float cutf = (float)cut2;
   const float span = 2.0f * sqrtf(ra2) + sqrtf(cutf);
   const float band = 0x1p-19f * (span * span);
-  const bool narrow = band < 0.05f * cutf;
   const float cut_m = (float)(cut2 - 0.0001);
+  const bool narrow = band < 0.05f * cutf && cut_m - band > 1e-4f + 2.0f * band;
   const unsigned in_lo = __float_as_uint(1e-4f + 2.0f * band);
   const unsigned in_w = __float_as_uint(cut_m - band) - in_lo;
   const float out_f = cut_m + band;
