@@ -1104,6 +1104,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   v.lj_only = p->force_field == RBMD_FF_LJ_CUT;
   v.rbl = p->neighbor_type == RBMD_NEIGHBOR_RBL;
   v.erfc_table = p->erfc_mode == RBMD_ERFC_TABLE;
+  v.erfc_direct = v.sqrt_alpha * v.cut > kCoulReach;
   v.mixed = p->precision == RBMD_PREC_MIXED ? 1 : 0;
   // accepted pairs have |r| < rc, so the minimum image is a no-op unless an edge is below 2 rc
   v.use_min_image = (v.box[0] < 2 * v.cut || v.box[1] < 2 * v.cut || v.box[2] < 2 * v.cut) ? 1 : 0;

@@ -23,6 +23,10 @@ constexpr int kCoulM = 32;      // Coulomb table intervals over [0, rc]
 constexpr int kCoulD = 9;       // polynomial degree per interval
 constexpr int kCoulPairs = (kCoulD + 1) / 2;           // coefficient pairs per interval
 constexpr int kCoulTab = 2 * kCoulPairs * kCoulM;      // double2 entries (P and Q)
+// Largest sqrt(alpha) rc at which the table's absolute error is that of erfc
+// and exp themselves (P 1.9e-16 against 2.4e-16, Q 1.5e-16 against 1.1e-16):
+// at 5 it is 3.9e-16, at 6.4 3.7e-15, at 10 2.4e-13
+constexpr double kCoulReach = 4.0;
 constexpr int kCoulD32 = 5;     // degree of the FP32 table of the mixed-precision path
 constexpr int kCoulPairs32 = (kCoulD32 + 1) / 2;
 constexpr int kCoulTab32 = 2 * kCoulPairs32 * kCoulM;  // float2 entries
@@ -60,6 +64,7 @@ struct SysView {
   int lj_only;      // LJ/CUT force field
   int rbl;          // random-batch list
   int erfc_table;   // step-table erfc (alpha = 0.1)
+  int erfc_direct;  // random-batch lists: sqrt(alpha) rc beyond kCoulReach, erfc without the radial table
   int rs_num, pice_num;
   int nslab;        // real-space partials per atom in fn*, vir_near, e_lj, e_coul (fused path 3, else 1)
   int use_min_image;  // some box edge < 2 rc: the pair vector may need the minimum image

@@ -229,12 +229,17 @@ void launch_nbr_build_rbl(const SysView& s, hipStream_t st) {
 // Gathers bound it; 16 lanes an atom and the table instead of one thread an
 // atom with erfc and divisions: 72 -> 8 us at 4096 salt atoms, 181 -> 43 us at
 // 30,000 water atoms.
-template <bool WEIGHTED, bool TABLE, bool VIR>
+//
+// ERFC: the analytic erfc by the Coulomb radial table or, where sqrt(alpha) rc
+// is too large for its 32 intervals (SysView::erfc_direct), by the functions
+// themselves; or the step table.
+enum { kErfcPoly = 0, kErfcStep = 1, kErfcDirect = 2 };
+template <bool WEIGHTED, int ERFC, bool VIR>
 __global__ __launch_bounds__(kBlock) void k_pair_rbl(SysView s, double* rows) {
 #pragma clang fp contract(off)  // the pair vector and d2 rounded as the list build and the oracle round them
   constexpr int L = kMaxLanes;
   __shared__ double teps[kMaxTypes * kMaxTypes], tsig[kMaxTypes * kMaxTypes];
-  __shared__ double2 ctab[TABLE ? 1 : kCoulTab / 2];
+  __shared__ double2 ctab[ERFC == kErfcPoly ? kCoulTab / 2 : 1];
   const int nt = s.ntypes;
   const bool ltab = nt <= kMaxTypes;
   if (ltab)
@@ -242,7 +247,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_rbl(SysView s, double* rows) {
       teps[k] = s.eps_ij[k];
       tsig[k] = s.sig6_ij[k];
     }
-  if (!TABLE)
+  if (ERFC == kErfcPoly)
     for (int k = threadIdx.x; k < kCoulTab / 2; k += kBlock) ctab[k] = s.ctab[k];
   __syncthreads();
   const int t = (int)(blockIdx.x * kBlock + threadIdx.x);
@@ -309,8 +314,10 @@ __global__ __launch_bounds__(kBlock) void k_pair_rbl(SysView s, double* rows) {
           const double sd6 = sig6 * (rinv2 * rinv2 * rinv2);
           const double ljs = w * (-24.0 * eps * (fma(2.0, sd6, -1.0) * sd6) * rinv2);
           double cs;
-          if (TABLE) {
+          if (ERFC == kErfcStep) {
             cs = -qq * gnear_table(sqrt(d2)) * rinv;
+          } else if (ERFC == kErfcDirect) {
+            cs = -qq * gnear(s.alpha, s.sqrt_alpha, sqrt(d2)) * rinv;
           } else {
             const double fk = (d2 * rinv) * s.ctab_inv_h;
             int kk = (int)fk;
@@ -400,16 +407,17 @@ int rbl_pair_blocks(const SysView& s) { return (int)(((size_t)s.n * kMaxLanes + 
 
 void launch_pair_rbl(const SysView& s, hipStream_t st, int virial) {
   const int grid = rbl_pair_blocks(s);
-#define RBL_PAIR(W_, T_, V_) hipLaunchKernelGGL((k_pair_rbl<W_, T_, V_>), dim3(grid), dim3(kBlock), 0, st, s, s.rbl_rows)
-#define RBL_PAIR_V(W_, T_)                                \
+#define RBL_PAIR(W_, E_, V_) hipLaunchKernelGGL((k_pair_rbl<W_, E_, V_>), dim3(grid), dim3(kBlock), 0, st, s, s.rbl_rows)
+#define RBL_PAIR_V(W_, E_)                                \
   do {                                                    \
-    if (virial) RBL_PAIR(W_, T_, true); else RBL_PAIR(W_, T_, false); \
+    if (virial) RBL_PAIR(W_, E_, true); else RBL_PAIR(W_, E_, false); \
   } while (0)
-  if (s.weighted) {
-    if (s.erfc_table) RBL_PAIR_V(true, true); else RBL_PAIR_V(true, false);
-  } else {
-    if (s.erfc_table) RBL_PAIR_V(false, true); else RBL_PAIR_V(false, false);
-  }
+#define RBL_PAIR_E(W_)                        \
+  do {                                        \
+    if (s.erfc_table) RBL_PAIR_V(W_, kErfcStep); else if (s.erfc_direct) RBL_PAIR_V(W_, kErfcDirect); else RBL_PAIR_V(W_, kErfcPoly); \
+  } while (0)
+  if (s.weighted) RBL_PAIR_E(true); else RBL_PAIR_E(false);
+#undef RBL_PAIR_E
 #undef RBL_PAIR_V
 #undef RBL_PAIR
   const dim3 blocks((s.n + kMeanThreads - 1) / kMeanThreads);
@@ -427,8 +435,8 @@ void launch_pair_rbl(const SysView& s, hipStream_t st, int virial) {
 // minimum-image vector gives
 //   e_lj   += w * 4 eps (s6/d6 - 1) s6/d6 / 2            (ComputePotentialEn_fix)
 //   e_coul += qqr2e (q q erfc(sqrt(alpha) r) / 2r - (1 - w) q q / 2r)
-// with the analytic erfc at the configured alpha (the Coulomb radial table),
-// not the step table.  No list is stored.  Runs on the steps that form thermo
+// with the analytic erfc at the configured alpha (the Coulomb radial table, or
+// erfc itself as in the force pass), not the step table.  No list is stored.  Runs on the steps that form thermo
 // sums; its rows also carry the mean-removed RBL virial of each atom.
 //
 // A wavefront queues the accepted (atom, candidate) pairs of its atoms in LDS
@@ -437,13 +445,13 @@ void launch_pair_rbl(const SysView& s, hipStream_t st, int virial) {
 // lanes off, where no other lane's register may be read.  PERATOM evaluates
 // each atom's pairs of a batch apart, for its sums.
 constexpr int kRblQueue = 2 * kWave;
-template <bool WEIGHTED, bool PERATOM>
+template <bool WEIGHTED, bool PERATOM, bool DIRECT>
 __global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) {
 #pragma clang fp contract(off)
   __shared__ RblTable tabs[kRblWaves];
   __shared__ RblStage stage;
   __shared__ int shared_int[2];
-  __shared__ double2 qtab[kCoulTab / 2];
+  __shared__ double2 qtab[DIRECT ? 1 : kCoulTab / 2];
   __shared__ int2 queue[kRblWaves][kRblQueue];  // atom, entry
   __shared__ double4 atom[kRblWaves][kRblAtoms];
   __shared__ int type[kRblWaves][kRblAtoms];
@@ -454,7 +462,8 @@ __global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) 
   double vals[kRowPair] = {0, 0, 0, 0, 0, 0, 0, 0};
   int c, first, nmine;
   if (rbl_atoms(s, (int)blockIdx.x, c, first, nmine)) {  // workgroup-uniform
-    for (int k = threadIdx.x; k < kCoulTab / 2; k += kBlock) qtab[k] = s.ctab[kCoulTab / 2 + k];
+    if (!DIRECT)
+      for (int k = threadIdx.x; k < kCoulTab / 2; k += kBlock) qtab[k] = s.ctab[kCoulTab / 2 + k];
     int mf_l = 0;
     if (lane < nmine) {
       atom[w][lane] = s.spos[first + lane];
@@ -497,10 +506,14 @@ __global__ __launch_bounds__(kBlock) void k_rbl_energy(SysView s, double* rows) 
         const double sd6 = s6 * (rinv2 * rinv2 * rinv2);
         el = 0.5 * (4.0 * eps * (sd6 - 1.0) * sd6);
         const double half = 0.5 * (pa.w * p.w) * rinv;
-        const double fk = (d2 * rinv) * s.ctab_inv_h;
-        int kk = (int)fk;
-        kk = kk < kCoulM - 1 ? kk : kCoulM - 1;
-        eco = half * coul_poly<false>(qtab, kk, fk - (double)kk - 0.5);  // qtab: the table's Q half
+        if (DIRECT) {
+          eco = half * erfc(s.sqrt_alpha * sqrt(d2));
+        } else {
+          const double fk = (d2 * rinv) * s.ctab_inv_h;
+          int kk = (int)fk;
+          kk = kk < kCoulM - 1 ? kk : kCoulM - 1;
+          eco = half * coul_poly<false>(qtab, kk, fk - (double)kk - 0.5);  // qtab: the table's Q half
+        }
         if (WEIGHTED) {
           double wt = 1.0;
           for (int u = 0; u < spmax; ++u)
@@ -564,17 +577,18 @@ int rbl_energy_blocks(const SysView& s) { return rbl_item_blocks(s); }
 void launch_rbl_energy(const SysView& s, hipStream_t st, int peratom, double* rows, int* nblocks) {
   const int grid = rbl_energy_blocks(s);
   if (nblocks) *nblocks = grid;
+#define RBL_ENERGY(W_, P_, D_) hipLaunchKernelGGL((k_rbl_energy<W_, P_, D_>), dim3(grid), dim3(kBlock), 0, st, s, rows)
+#define RBL_ENERGY_D(W_, P_)                                               \
+  do {                                                                     \
+    if (s.erfc_direct) RBL_ENERGY(W_, P_, true); else RBL_ENERGY(W_, P_, false); \
+  } while (0)
   if (s.weighted) {
-    if (peratom)
-      hipLaunchKernelGGL((k_rbl_energy<true, true>), dim3(grid), dim3(kBlock), 0, st, s, rows);
-    else
-      hipLaunchKernelGGL((k_rbl_energy<true, false>), dim3(grid), dim3(kBlock), 0, st, s, rows);
+    if (peratom) RBL_ENERGY_D(true, true); else RBL_ENERGY_D(true, false);
   } else {
-    if (peratom)
-      hipLaunchKernelGGL((k_rbl_energy<false, true>), dim3(grid), dim3(kBlock), 0, st, s, rows);
-    else
-      hipLaunchKernelGGL((k_rbl_energy<false, false>), dim3(grid), dim3(kBlock), 0, st, s, rows);
+    if (peratom) RBL_ENERGY_D(false, true); else RBL_ENERGY_D(false, false);
   }
+#undef RBL_ENERGY_D
+#undef RBL_ENERGY
 }
 
 __global__ __launch_bounds__(kBlock) void k_static_table(const double* dis, double* g, int n) {
