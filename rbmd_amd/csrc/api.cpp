@@ -865,20 +865,32 @@ rbmd_status ewald_ws(rbmd_sys* s, int64_t bytes, void** out) {
 constexpr int64_t kEwTables = int64_t(512) << 20, kEwPartials = int64_t(256) << 20;
 constexpr int64_t kEwTablesSmall = int64_t(14) << 20, kEwPartialsSmall = int64_t(10) << 20;
 
+// A sum with its rounding kept apart (Neumaier), as the terms of a grid run
+// over many orders of magnitude
+struct ExactSum {
+  double sum = 0, low = 0;
+  void add(double v) {
+    const double t = sum + v;
+    low += std::fabs(sum) >= std::fabs(v) ? (sum - t) + v : (v - t) + sum;
+    sum = t;
+  }
+  double value() const { return sum + low; }
+};
+
 // the grid sum from the energy rows of the weight pass
 rbmd_status ewald_grid_sum(rbmd_sys* s, const EwView& v, double* sum) {
   const size_t rows = ewald_energy_rows(v), most = s->pin_bytes / sizeof(double);
   const int h = s->pin_next;
   s->pin_next ^= 1;
-  double t = 0;
+  ExactSum t;
   for (size_t r = 0; r < rows; r += most) {
     const size_t len = std::min(most, rows - r);
     HIP_TRY(hipMemcpyAsync(s->pin[h], v.erow + r, len * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream));
     HIP_TRY(hipStreamSynchronize(s->ctx->stream));
     const double* e = (const double*)s->pin[h];
-    for (size_t k = 0; k < len; ++k) t += e[k];
+    for (size_t k = 0; k < len; ++k) t.add(e[k]);
   }
-  *sum = t;
+  *sum = t.value();
   return RBMD_OK;
 }
 
