@@ -894,47 +894,93 @@ rbmd_status ewald_grid_sum(rbmd_sys* s, const EwView& v, double* sum) {
   return RBMD_OK;
 }
 
+// Bytes of the direct form over K k vectors, in slices on 256-byte boundaries:
+// the k vectors, the structure factors of every atom block and their sums
+int64_t direct_bytes(const rbmd_sys* s, int64_t K, int* atoms) {
+  const int64_t kper = (int64_t)kWave * s->v.rho_kb;
+  *atoms = rho_atoms_per_block(s->n, (int)std::min<int64_t>((K + kper - 1) / kper, 1 << 30));
+  const int nblk = (s->n + *atoms - 1) / *atoms;
+  auto up = [](int64_t b) { return (b + 255) & ~int64_t(255); };
+  return up(3 * K * 8) + up((int64_t)nblk * 2 * K * 8) + up(2 * K * 8);
+}
+
+// the grid sum by one sine and cosine per (atom, k), in the buffer `base` of direct_bytes
+rbmd_status direct_grid_sum(rbmd_sys* s, const int kmax[3], int atoms, void* base, double* sum) {
+  std::vector<double> kg;
+  for (int i = -kmax[0]; i <= kmax[0]; ++i)
+    for (int j = -kmax[1]; j <= kmax[1]; ++j)
+      for (int k = -kmax[2]; k <= kmax[2]; ++k)
+        if (i || j || k) {
+          kg.push_back(2 * kPi * i / s->v.box[0]);
+          kg.push_back(2 * kPi * j / s->v.box[1]);
+          kg.push_back(2 * kPi * k / s->v.box[2]);
+        }
+  const int K = (int)(kg.size() / 3);
+  const int nblk = (s->n + atoms - 1) / atoms;
+  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+  double* const kdev = static_cast<double*>(base);
+  double* const part = reinterpret_cast<double*>(static_cast<char*>(base) + up(kg.size() * 8));
+  double* const rho_dev = reinterpret_cast<double*>(reinterpret_cast<char*>(part) + up((size_t)nblk * 2 * K * 8));
+  std::vector<double> rho((size_t)2 * K);
+  hipStream_t st = s->ctx->stream;
+  HIP_TRY(hipMemcpyAsync(kdev, kg.data(), kg.size() * 8, hipMemcpyHostToDevice, st));
+  KView k{};
+  k.P = K;
+  k.S_over_P = 1.0;
+  k.kvec = kdev;
+  k.rho_part = part;
+  k.rho = rho_dev;
+  k.nblk_rho = nblk;
+  k.rho_atoms = atoms;  // no records: the energy alone
+  launch_rho_partial(s->v, k, st);
+  launch_rho_reduce(s->v, k, st);
+  HIP_TRY(hipMemcpyAsync(rho.data(), rho_dev, rho.size() * 8, hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  ExactSum t;
+  for (int l = 0; l < K; ++l) {
+    const double kx = kg[3 * l], ky = kg[3 * l + 1], kz = kg[3 * l + 2];
+    const double k2 = kx * kx + ky * ky + kz * kz;
+    t.add(std::exp(-k2 / (4 * s->p.alpha)) * (rho[2 * l] * rho[2 * l] + rho[2 * l + 1] * rho[2 * l + 1]) / k2);
+  }
+  *sum = t.value();
+  return RBMD_OK;
+}
+
 // e_long = qqr2e (2 pi / V) sum_grid e^{-k^2/4a}|rho|^2/k^2 / N + self / N
 // (ComputeEwaldEnergy + ComputeSelfEnergy, ExecutionMD.cpp:405-443, 508-558).
 // The phase tables and the structure-factor partials live in the system's
 // workspace, or, with `scratch` (the no-alloc entry point), in that buffer of
 // scratch_bytes, which every launch overwrites in full before reading it (no
-// clearing needed).  Grids that the scratch takes run the same plan, to the
-// same bits, in both.
+// clearing needed).  The scratch takes the grids that the direct form fits it
+// with; these run the same plan, to the same bits, in both: the separable form
+// in small tables or, for the few long flat grids whose tables and partials
+// need more (100 x 100 x 0 with 30,000 atoms), the direct form.
 rbmd_status long_energy(rbmd_sys* s, const int kmax[3], double* e_avg, double* grid_sum_out,
                         void* scratch = nullptr, size_t scratch_bytes = 0) {
   int64_t K = 1;
   for (int d = 0; d < 3; ++d) K *= kmax[d] < 0 ? 0 : 2 * (int64_t)kmax[d] + 1;
   K = K > 0 ? K - 1 : 0;
   if (K == 0) return fail(RBMD_ERR_HIP, "Ewald energy: the kmax grid holds no k vector");
-  // the scratch takes the grids whose k vectors, reduced and partial structure
-  // factors per atom block fit it, in slices on 256-byte boundaries
-  const int64_t kper = (int64_t)kWave * s->v.rho_kb;
-  const int atoms = rho_atoms_per_block(s->n, (int)std::min<int64_t>((K + kper - 1) / kper, 1 << 30));
-  const int nblk = (s->n + atoms - 1) / atoms;
-  auto up = [](int64_t b) { return (b + 255) & ~int64_t(255); };
-  const int64_t need = up(3 * K * 8) + up((int64_t)nblk * 2 * K * 8) + up(2 * K * 8);
+  int atoms = 0;
+  const int64_t need = direct_bytes(s, K, &atoms);
   const bool small = need <= (int64_t)kScratchBytes;
   if (scratch && need > (int64_t)scratch_bytes)
-    return fail(RBMD_ERR_ARG,
-                "the kmax grid (%lld k vectors over %d atom blocks) needs %lld bytes of scratch; the no-alloc "
-                "scratch holds %zu",
-                (long long)K, nblk, (long long)need, scratch_bytes);
+    return fail(RBMD_ERR_ARG, "the kmax grid (%lld k vectors) needs %lld bytes of scratch; the no-alloc scratch holds %zu",
+                (long long)K, (long long)need, scratch_bytes);
   EwView v;
   ewald_plan(s->n, kmax, small ? kEwTablesSmall : kEwTables, small ? kEwPartialsSmall : kEwPartials, &v);
   const int64_t bytes = ewald_bytes(v, false);
+  const bool direct = small && bytes > (int64_t)kScratchBytes;
   void* base = scratch;
-  if (scratch) {
-    if (bytes > (int64_t)scratch_bytes)
-      return fail(RBMD_ERR_ARG, "the kmax grid needs %lld bytes of scratch; the no-alloc scratch holds %zu",
-                  (long long)bytes, scratch_bytes);
-  } else {
-    RC_TRY(ewald_ws(s, bytes, &base));
-  }
-  ewald_buffers(&v, base, false);
-  launch_ewald_rho(s->v, v, s->ctx->stream);
+  if (!scratch) RC_TRY(ewald_ws(s, direct ? need : bytes, &base));
   double sum = 0;
-  RC_TRY(ewald_grid_sum(s, v, &sum));
+  if (direct) {
+    RC_TRY(direct_grid_sum(s, kmax, atoms, base, &sum));
+  } else {
+    ewald_buffers(&v, base, false);
+    launch_ewald_rho(s->v, v, s->ctx->stream);
+    RC_TRY(ewald_grid_sum(s, v, &sum));
+  }
   const double self = -std::sqrt(s->p.alpha / kPi) * s->q2;
   if (grid_sum_out) *grid_sum_out = sum;
   *e_avg = s->u.qqr2e * sum * (2 * kPi / s->v.volume) / s->n + s->u.qqr2e * self / s->n;
