@@ -710,6 +710,30 @@ rbmd_status ensure_rho(rbmd_sys* s, int P) {
   return RBMD_OK;
 }
 
+// k vectors 2 pi m / L of the whole kmax grid in the reference's order
+std::vector<double> grid_list(const rbmd_sys* s, const int kmax[3]) {
+  std::vector<double> kg;
+  for (int i = -kmax[0]; i <= kmax[0]; ++i)
+    for (int j = -kmax[1]; j <= kmax[1]; ++j)
+      for (int k = -kmax[2]; k <= kmax[2]; ++k)
+        if (i || j || k) {
+          kg.push_back(2 * kPi * i / s->v.box[0]);
+          kg.push_back(2 * kPi * j / s->v.box[1]);
+          kg.push_back(2 * kPi * k / s->v.box[2]);
+        }
+  return kg;
+}
+
+// Grid Ewald systems: the k vectors and the direct form's buffers for
+// rbmd_rbe_structure_factor, at its first call (the steps do without)
+rbmd_status grid_kvectors(rbmd_sys* s) {
+  if (s->kcur) return RBMD_OK;
+  const std::vector<double> kg = grid_list(s, s->p.kmax);
+  s->P = (int)(kg.size() / 3);
+  RC_TRY(ensure_rho(s, s->P));
+  return s->upload(&s->kcur, kg.data(), kg.size());
+}
+
 // Full force evaluation on the current locator (ExecutionNVT::ComputeAllForce,
 // ExecutionNVT.cpp:195-235).  kvec: device pointer to this step's k vectors.
 // k-space and bonded forces on stream st (they read the unsorted positions
@@ -720,7 +744,6 @@ static KView step_kview(const rbmd_sys* s, const double* kvec) {
   k.kvec = kvec;
   k.S_over_P = s->p.coulomb_type == RBMD_COULOMB_RBE ? s->S / (double)s->P : 1.0;
   k.f32 = s->v.mixed;
-  k.ewald = s->p.coulomb_type == RBMD_COULOMB_EWALD;
   return k;
 }
 
@@ -906,15 +929,7 @@ int64_t direct_bytes(const rbmd_sys* s, int64_t K, int* atoms) {
 
 // the grid sum by one sine and cosine per (atom, k), in the buffer `base` of direct_bytes
 rbmd_status direct_grid_sum(rbmd_sys* s, const int kmax[3], int atoms, void* base, double* sum) {
-  std::vector<double> kg;
-  for (int i = -kmax[0]; i <= kmax[0]; ++i)
-    for (int j = -kmax[1]; j <= kmax[1]; ++j)
-      for (int k = -kmax[2]; k <= kmax[2]; ++k)
-        if (i || j || k) {
-          kg.push_back(2 * kPi * i / s->v.box[0]);
-          kg.push_back(2 * kPi * j / s->v.box[1]);
-          kg.push_back(2 * kPi * k / s->v.box[2]);
-        }
+  const std::vector<double> kg = grid_list(s, kmax);
   const int K = (int)(kg.size() / 3);
   const int nblk = (s->n + atoms - 1) / atoms;
   auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
@@ -1497,19 +1512,9 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
       }
       A(ensure_rho(s, s->P));
     } else {
-      // Ewald force over the kmax grid in the reference's k order
-      std::vector<double> kg;
-      for (int i = -p->kmax[0]; i <= p->kmax[0]; ++i)
-        for (int j = -p->kmax[1]; j <= p->kmax[1]; ++j)
-          for (int k = -p->kmax[2]; k <= p->kmax[2]; ++k)
-            if (i || j || k) {
-              kg.push_back(2 * kPi * i / v.box[0]);
-              kg.push_back(2 * kPi * j / v.box[1]);
-              kg.push_back(2 * kPi * k / v.box[2]);
-            }
-      s->P = (int)(kg.size() / 3);
-      A(s->upload(&s->kcur, kg.data(), kg.size()));
-      A(ensure_rho(s, s->P));
+      int64_t K = 1;
+      for (int d = 0; d < 3; ++d) K *= std::max(2 * (int64_t)p->kmax[d] + 1, int64_t(0));
+      s->P = (int)std::max(K - 1, int64_t(0));
       // one batch (packs take a system's tables whole)
       if (rc == RBMD_OK && ewald_plan(n, p->kmax, INT64_MAX, kEwPartials, &s->ew)) {
         char* base = nullptr;
@@ -1518,6 +1523,8 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
           ewald_buffers(&s->ew, base, true);
           s->ew_on = true;
         }
+      } else {
+        A(grid_kvectors(s));
       }
     }
   }
@@ -1829,6 +1836,7 @@ rbmd_status rbmd_rbe_sample(rbmd_sys* s, uint64_t seed, uint64_t stream, double*
 
 rbmd_status rbmd_rbe_structure_factor(rbmd_sys* s, double* rho_out) {
   if (!s || !rho_out) return fail(RBMD_ERR_ARG, "bad arguments");
+  if (has_k(s) && s->p.coulomb_type == RBMD_COULOMB_EWALD) RC_TRY(grid_kvectors(s));
   if (!has_k(s) || !s->kcur) return fail(RBMD_ERR_STATE, "no k vectors");
   KView k = s->kv;
   k.P = s->P;
@@ -2445,7 +2453,6 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
   p->sig.pair_sp = sp_of(s0);
   p->sig.f32 = s0->v.mixed;
   p->sig.has_k = p->has_k;
-  p->sig.ewald = s0->p.coulomb_type == RBMD_COULOMB_EWALD;
   p->sig.has_b = p->has_b;
   p->sig.k_lanes_lg = k_lanes_lg_of(s0->p);  // compact systems have their own tiles
   p->sig.rho_kb = rho_kb_of(s0->p);
@@ -2476,7 +2483,6 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
     e.kv.kvec = p->ring ? s->kgraph : s->kcur;
     e.kv.S_over_P = s->p.coulomb_type == RBMD_COULOMB_RBE ? s->S / (double)s->P : 1.0;
     e.kv.f32 = s->v.mixed;
-    e.kv.ewald = s->p.coulomb_type == RBMD_COULOMB_EWALD;
     e.ew = s->ew;
     e.nhc = s->nhc;
     e.np = s->np;

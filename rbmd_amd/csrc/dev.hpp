@@ -236,8 +236,8 @@ int force_cells_blocks(const SysView& s);
 
 // ---------------------------------------------------------------- k space
 // One k vector as the force pass reads it (written by the rho reduction):
-// k, the prefactor 1/(V k^2) (Ewald: times e^{-k^2/4 alpha}), m = k L / 2 pi
-// and rho(k); in mixed precision rr and ri hold pre Re rho and pre Im rho.
+// k, the prefactor 1/(V k^2), m = k L / 2 pi and rho(k); in mixed precision rr
+// and ri hold pre Re rho and pre Im rho.
 // 80 bytes, read with scalar loads.
 struct KRec {
   double kx, ky, kz, pre, mx, my, mz, rr, ri, pad;
@@ -252,7 +252,6 @@ struct KView {
   int nblk_rho;
   int f32;              // phases' sin/cos and the force coefficient in FP32 (sums in FP64)
   KRec* krec;           // [P] records for the force pass (null: the reduction writes none)
-  int ewald;            // prefactor with the Ewald Gaussian
   int rho_atoms;        // atoms per structure-factor workgroup (= n / nblk_rho rounded up to it)
 };
 // atoms per structure-factor workgroup for n atoms and kblocks k-vector
@@ -435,7 +434,7 @@ enum PackKernel {
 int pack_blocks(const SysView& s, const IntView& iv, int P, int kernel);
 
 struct PackSig {  // launch-wide choices, equal for every system of a pack
-  int pair_mode, pair_sp, f32, has_k, ewald, has_b, k_lanes_lg, rho_kb;
+  int pair_mode, pair_sp, f32, has_k, has_b, k_lanes_lg, rho_kb;
   int thermo;  // this step computes the virial and energy sums (else forces and KE only)
 };
 

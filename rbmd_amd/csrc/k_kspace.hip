@@ -9,8 +9,7 @@
 // F_i = (S/P) sum_l -(4 pi q_i / (V k_l^2)) (cos(k.r) Im rho - sin(k.r) Re rho) k_l, x qqr2e
 //   ComputeNewRBEForceWorklet (RunWorklet.cpp:2086-2141), ComputeRBEForceSum_fix
 //   (ExecForceFunction.h:748-762), ComputeKspaceVirial (:397-410), UnitRescale
-//   (ExecutionNVT.cpp:718).  With an Ewald prefactor e^{-k^2/4 alpha} and scale 1
-//   the same kernel is ComputeNewFarElectrostaticsWorklet (RunWorklet.cpp:2492-2540).
+//   (ExecutionNVT.cpp:718).  (The Ewald sum over a kmax grid: k_ewald.hip.)
 #include "dev.hpp"
 #include "pack.hpp"
 #include "reduce.hpp"
@@ -87,7 +86,7 @@ __device__ __forceinline__ void rho_reduce_body(const SysView& s, const KView& k
       const int l = t >> 1;
       const double kx = kv.kvec[3 * l], ky = kv.kvec[3 * l + 1], kz = kv.kvec[3 * l + 2];
       const double k2 = kx * kx + ky * ky + kz * kz;
-      const double pre = kv.ewald ? exp(-k2 / (4 * s.alpha)) / (s.volume * k2) : 1.0 / (s.volume * k2);
+      const double pre = 1.0 / (s.volume * k2);
       rec.kx = kx;
       rec.ky = ky;
       rec.kz = kz;
