@@ -140,8 +140,10 @@ typedef struct rbmd_params {
    * of the k-space force kernel (2, 4, 8; default 4), k vectors per lane of
    * the structure-factor kernel (1, 2, 4; default 1).  rbmd_amd/tune.py
    * measures them per kind, precision and size and rbmd_amd/tiles.json holds
-   * the result.  Systems of up to a few thousand atoms whose steps compute the
-   * pair forces from the cells keep 16 lanes and 16 wavefronts. */
+   * the result.  Dense systems of up to a few thousand atoms compute the pair
+   * forces from the cells (rbmd_md_path COMPACT) by 16 lanes and the k-space
+   * force by 16 wavefronts; with pair_lanes 4 or 8 they run over lists, and
+   * kforce_lanes applies. */
   int32_t pair_lanes;
   int32_t kforce_lanes;
   int32_t rho_kblock;

@@ -1241,11 +1241,12 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
   // 8 and 16: salt 20,000 23, 19 and 18 us, 99,000 57, 57 and 62, 300,000 144,
   // 138 and 167; water (mixed) 300,000 457, 381 and 359
   v.lanes_lg = n <= 60000 ? 4 : 3;
-  v.compact = p->coulomb_type != RBMD_COULOMB_EWALD && !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes && stencil_pays(v) ? 1 : 0;
+  // (the stencil kernel sums by 16 lanes: 4 or 8 asked for are the lists')
+  v.compact = p->coulomb_type != RBMD_COULOMB_EWALD && !v.rbl && !s->fused && !s->skin && d->n_types <= kMaxTypes &&
+              (p->pair_lanes == 0 || p->pair_lanes == 16) && stencil_pays(v) ? 1 : 0;
   if (v.accept_d2 - v.test_band <= 1e-4 + 2.0 * v.test_band) v.compact = 0;  // an FP32 test has no room at such an rc
   v.st_cfg = stencil_choice(v);
   if (p->pair_lanes) v.lanes_lg = p->pair_lanes == 4 ? 2 : (p->pair_lanes == 8 ? 3 : 4);
-  if (v.compact) v.lanes_lg = 4;  // as the stencil kernel sums
   v.k_lanes_lg = k_lanes_lg_of(*p);
   v.rho_kb = rho_kb_of(*p);
   if (v.compact) v.k_lanes_lg = 4;  // the latency counts: 16 wavefronts over the k range

@@ -14,7 +14,9 @@ HIP events on the library's stream, every option of
 
 (option i of all three in run i: the kernels are timed separately, in the
 library's kernel-profiling mode, on one stream).  The pair lanes are chosen
-per size (a per-system runtime value) by the pair kernel's time.
+per size (a per-system runtime value) by the pair kernel's time, or, where 16
+lanes take the steps off the lists (rbmd_md_path COMPACT), by the time of
+whole steps.
 
 The two k-space choices are made per kind and precision (the kernels of a
 pack take them as template parameters, so all systems of a pack share them)
@@ -52,6 +54,7 @@ def measure(ctx, kind, precision, atoms, steps, step_steps, log):
     for i in range(3):
         run = type(r)(**{**r.__dict__, **{key: OPTIONS[key][i] for key in OPTIONS}})
         g = GpuSystem(ctx, s, run)
+        compact = g.md_path() == "compact"
         g.md_init()
         g.md_step(3)
         ctx.synchronize()
@@ -66,7 +69,8 @@ def measure(ctx, kind, precision, atoms, steps, step_steps, log):
             out[key].append(1e3 * ms / max(n, 1))
         log(f"[tune] {kind} {precision} n={s.n_atoms} option {i}: " +
             ", ".join(f"{KERNEL[k]} {out[k][-1]:.1f} us" for k in OPTIONS))
-    for key in K_TILES:
+    # compact: the last option's, 16 lanes
+    for key in (("pair_lanes",) if compact else ()) + K_TILES:
         out["step_" + key] = []
         for i in range(3):
             run = type(r)(**{**r.__dict__, "tiles": "default", "pair_lanes": 0, "kforce_lanes": 0, "rho_kblock": 0,
@@ -94,7 +98,8 @@ def choose(per_size):
         entry[key] = OPTIONS[key][min(range(3), key=lambda i: score[i])]
     lanes = []
     for k, (n, t) in enumerate(per_size):
-        best = OPTIONS["pair_lanes"][min(range(3), key=lambda i: t["pair_lanes"][i])]
+        times = t.get("step_pair_lanes", t["pair_lanes"])
+        best = OPTIONS["pair_lanes"][min(range(3), key=lambda i: times[i])]
         # bucket edge: geometric midpoint to the next measured size
         edge = int(math.sqrt(n * per_size[k + 1][0])) if k + 1 < len(per_size) else 2 ** 31 - 1
         lanes.append([edge, best])

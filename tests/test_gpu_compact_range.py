@@ -58,3 +58,25 @@ def test_atoms_boxes_away(ctx, n, density, cut, away):
         g.close()
     for u, v in zip(*out):
         assert np.array_equal(u, v)
+
+
+@pytest.mark.parametrize("lanes,path", [(0, "compact"), (4, "lists"), (8, "lists"), (16, "compact")])
+def test_pair_lanes_asked_for(ctx, lanes, path):
+    """4 and 8 lanes are the lists'; the forces differ by the order of at most 140
+    terms, 140 x 1.1e-16 of the largest sum of magnitudes, which stays below ten
+    times the largest force: 2e-13"""
+    s = make_salt(n_ions=2000, seed=2)
+    ref = GpuSystem(ctx, s, salt_config(tiles="default"))
+    g = GpuSystem(ctx, s, salt_config(tiles="default", pair_lanes=lanes))
+    assert ref.md_path() == "compact" and g.md_path() == path
+    for k in (ref, g):
+        k.md_init()
+    a, b = ref.state()[2], g.state()[2]
+    assert np.abs(a - b).max() <= 2e-13 * np.abs(a).max()
+    assert np.array_equal(a, b) == (path == "compact")  # lanes of another number sum in another order
+    for k in (ref, g):
+        k.md_step(3)
+    a, b = ref.state()[0], g.state()[0]
+    assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
+    ref.close()
+    g.close()
