@@ -489,13 +489,14 @@ rbmd_status read_status(rbmd_sys* s, int* st) {
   return RBMD_OK;
 }
 
-// Staging for n atoms: all arrays of a call for small systems (12 words an
-// atom), parts of 1 MiB for large ones.  Coherent memory, and events that
+// Staging for n atoms and P k vectors: all arrays of a call for small systems
+// (12 words an atom), parts of 1 MiB for large ones.  Coherent memory, and events that
 // release to the system: what the kernels wrote is the host's to read once the
 // event is reached.
 constexpr size_t kPinMost = size_t(1) << 20;
 rbmd_status pin_create(rbmd_sys* s) {
-  s->pin_bytes = std::min(kPinMost, std::max<size_t>(4096, (size_t)s->n * 12 * sizeof(double)));
+  const size_t kvec = s->p.coulomb_type == RBMD_COULOMB_RBE ? (size_t)s->P * 3 * sizeof(double) : 0;
+  s->pin_bytes = std::min(kPinMost, std::max<size_t>({4096, (size_t)s->n * 12 * sizeof(double), kvec}));
   for (int h = 0; h < 2; ++h) {
     if (hipHostMalloc((void**)&s->pin[h], s->pin_bytes, hipHostMallocCoherent) != hipSuccess) return fail(RBMD_ERR_OOM, "hipHostMalloc staging");
     if (hipEventCreateWithFlags(&s->pin_ev[h], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess)
@@ -573,13 +574,14 @@ struct Transfer {
 // The caller's arrays to the device.  Returns with the last parts' kernels in
 // the stream (the caller's memory has been read).
 rbmd_status transfer_in(rbmd_sys* s, Transfer& t) {
-  if (t.d.width == 0 || s->n <= 0) return RBMD_OK;
+  const int n = t.d.n;
+  if (t.d.width == 0 || n <= 0) return RBMD_OK;
   const int per = (int)(s->pin_bytes / (8 * (size_t)t.d.width));
-  for (int a0 = 0; a0 < s->n; a0 += per) {
+  for (int a0 = 0; a0 < n; a0 += per) {
     const int h = s->pin_next;
     s->pin_next ^= 1;
     t.d.a0 = a0;
-    t.d.atoms = std::min(per, s->n - a0);
+    t.d.atoms = std::min(per, n - a0);
     t.d.host = (double*)s->pin[h];
     HIP_TRY(hipEventSynchronize(s->pin_ev[h]));
     t.host_copy(s->pin[h], a0, t.d.atoms, false);
@@ -1813,15 +1815,10 @@ rbmd_status rbmd_rbe_set_kvectors(rbmd_sys* s, int32_t p, const double* m) {
   std::vector<double> k(3 * (size_t)p);
   for (int l = 0; l < p; ++l)
     for (int d = 0; d < 3; ++d) k[3 * l + d] = 2 * kPi * m[3 * l + d] / s->v.box[d];
-  for (size_t k0 = 0; k0 < k.size(); k0 += s->pin_bytes / 8) {
-    const int h = s->pin_next;
-    const size_t len = std::min(k.size() - k0, s->pin_bytes / 8);
-    s->pin_next ^= 1;
-    HIP_TRY(hipEventSynchronize(s->pin_ev[h]));
-    std::memcpy(s->pin[h], k.data() + k0, len * 8);
-    HIP_TRY(hipMemcpyAsync(s->kcur + k0, s->pin[h], len * 8, hipMemcpyHostToDevice, s->ctx->stream));
-    HIP_TRY(hipEventRecord(s->pin_ev[h], s->ctx->stream));
-  }
+  Transfer t(s);
+  t.d.n = p;  // a record per k vector
+  t.records(k.data(), s->kcur, 3);
+  RC_TRY(transfer_in(s, t));
   s->injected = true;
   return RBMD_OK;
 }
