@@ -2523,25 +2523,30 @@ rbmd_status rbmd_pack_create(rbmd_ctx* ctx, rbmd_sys* const* systems, int32_t n,
     p->nblk[q] = (int)tot;
     moff[q + 1] = moff[q] + (size_t)tot;
   }
-  std::vector<int> map(std::max<size_t>(moff[PK_COUNT], 1));
+  // one buffer: the systems, the first blocks, the block maps, the status words
+  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+  const size_t at_first = up(sizeof(PackSys) * n), at_map = at_first + up(sizeof(int) * first.size());
+  const size_t at_status = at_map + up(sizeof(int) * std::max<size_t>(moff[PK_COUNT], 1));
+  std::vector<char> host(at_status);
+  std::memcpy(host.data(), tab.data(), sizeof(PackSys) * n);
+  std::memcpy(host.data() + at_first, first.data(), sizeof(int) * first.size());
+  int* const map = reinterpret_cast<int*>(host.data() + at_map);
   for (int q = 0; q < PK_COUNT; ++q)
-    for (int k = 0; k < n; ++k)
-      for (int b = 0; b < blocks[q][k]; ++b) map[moff[q] + first[(size_t)q * (n + 1) + k] + b] = k;
-  rbmd_status rc = RBMD_OK;
-  if (rc == RBMD_OK) rc = dalloc((void**)&p->dsys, sizeof(PackSys) * n);
-  if (rc == RBMD_OK) rc = dalloc((void**)&p->dmap, sizeof(int) * map.size());
-  if (rc == RBMD_OK) rc = dalloc((void**)&p->dfirst, sizeof(int) * first.size());
-  if (rc == RBMD_OK) rc = dalloc((void**)&p->dstatus, sizeof(int) * n);
+    for (int k = 0; k < n; ++k) std::fill_n(map + moff[q] + first[(size_t)q * (n + 1) + k], blocks[q][k], k);
+  char* dev = nullptr;
+  const rbmd_status rc = dalloc((void**)&dev, at_status + sizeof(int) * n);
   if (rc != RBMD_OK) return pack_fail_free(p, rc);
+  p->dsys = reinterpret_cast<PackSys*>(dev);
+  p->dfirst = reinterpret_cast<int*>(dev + at_first);
+  p->dmap = reinterpret_cast<int*>(dev + at_map);
+  p->dstatus = reinterpret_cast<int*>(dev + at_status);
   if (hipHostMalloc((void**)&p->hstatus, sizeof(int) * n) != hipSuccess)
     return pack_fail_free(p, fail(RBMD_ERR_OOM, "pinned status array"));
   if (hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming) != hipSuccess)
     return pack_fail_free(p, fail(RBMD_ERR_HIP, "hipEventCreate"));
   hipStream_t st = ctx->stream;
-  if (hipMemcpyAsync(p->dsys, tab.data(), sizeof(PackSys) * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-      hipMemcpyAsync(p->dmap, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
-      hipMemcpyAsync(p->dfirst, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
+  if (hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return pack_fail_free(p, fail(RBMD_ERR_HIP, "pack table upload"));
   for (int q = 0; q < PK_COUNT; ++q) p->L[q] = PackLaunch{p->dsys, p->dmap + moff[q], p->dfirst + (size_t)q * (n + 1)};
