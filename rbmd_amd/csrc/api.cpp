@@ -2577,8 +2577,12 @@ static rbmd_status pack_lists(rbmd_pack* p) {
     v.cap = now.cap;
   }
   if (!moved) return RBMD_OK;
-  HIP_TRY(hipMemcpyAsync(p->dsys, p->tab.data(), sizeof(PackSys) * p->tab.size(), hipMemcpyHostToDevice, p->ctx->stream));
-  HIP_TRY(hipStreamSynchronize(p->ctx->stream));
+  hipError_t e = hipMemcpyAsync(p->dsys, p->tab.data(), sizeof(PackSys) * p->tab.size(), hipMemcpyHostToDevice, p->ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(p->ctx->stream);
+  if (e != hipSuccess) {
+    p->tab[0].v.nbr = nullptr;  // tried again by the next call
+    return fail(RBMD_ERR_HIP, "pack table upload: %s", hipGetErrorString(e));
+  }
   return RBMD_OK;
 }
 
