@@ -892,7 +892,7 @@ constexpr int64_t kEwTablesSmall = int64_t(14) << 20, kEwPartialsSmall = int64_t
 
 // A sum with its rounding kept apart (Neumaier), as the terms of a grid run
 // over many orders of magnitude
-struct ExactSum {
+struct CompensatedSum {
   double sum = 0, low = 0;
   void add(double v) {
     const double t = sum + v;
@@ -907,7 +907,7 @@ rbmd_status ewald_grid_sum(rbmd_sys* s, const EwView& v, double* sum) {
   const size_t rows = ewald_energy_rows(v), most = s->pin_bytes / sizeof(double);
   const int h = s->pin_next;
   s->pin_next ^= 1;
-  ExactSum t;
+  CompensatedSum t;
   for (size_t r = 0; r < rows; r += most) {
     const size_t len = std::min(most, rows - r);
     HIP_TRY(hipMemcpyAsync(s->pin[h], v.erow + r, len * sizeof(double), hipMemcpyDeviceToHost, s->ctx->stream));
@@ -953,7 +953,7 @@ rbmd_status direct_grid_sum(rbmd_sys* s, const int kmax[3], int atoms, void* bas
   launch_rho_reduce(s->v, k, st);
   HIP_TRY(hipMemcpyAsync(rho.data(), rho_dev, rho.size() * 8, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  ExactSum t;
+  CompensatedSum t;
   for (int l = 0; l < K; ++l) {
     const double kx = kg[3 * l], ky = kg[3 * l + 1], kz = kg[3 * l + 2];
     const double k2 = kx * kx + ky * ky + kz * kz;
