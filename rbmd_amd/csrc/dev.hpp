@@ -113,7 +113,7 @@ struct SysView {
   double4* spos;    // [n] x,y,z,q in sorted order
   float4* spos32;   // [n] x - lo, y - lo, z - lo in FP32 and the type's bits, in sorted order (stencil pair kernel)
   int* stype;       // [n]
-  // neighbour lists, column-major [cap][n] of packed (j_sorted << 9 | shift code)
+  // neighbour lists, [n][cap], of packed (j_sorted << 9 | shift code)
   int* nbr;         // layout nbr_index(slot, i, cap): one row per atom
   int lds_bins;     // binning kernels aggregate counts in LDS (ncell small enough)
   int* nbr_num;     // VERLET [n]; RBL [2n] (core, shell kept)

@@ -14,10 +14,11 @@
 // leaves the vector unit the range test and the append.  Accepted lanes store
 // their entries side by side at the row's count plus the ballot prefix.
 //
-// Bound by instruction issue: 15 slots per atom and 64 candidates (four of the
+// Bound by instruction issue at 300,000 atoms (vector ALUs 77 % busy, the matrix
+// instructions beside them): 15 slots per atom and 64 candidates (four of the
 // matrix instructions per group of four atoms, 3 for the range and band tests,
-// 7 to append), and by the latency of the chain from the cell to the first
-// test where few wavefronts are in flight.  A lane per atom over LDS-staged
+// 7 to append).  At 30,000 they are 38 % busy: the latency of the chain from
+// the cell to the first test, with few wavefronts in flight.  A lane per atom over LDS-staged
 // candidates, 9 stencil columns apart, took 48 us at 12,000 water atoms, 60 at
 // 30,000, 355 at 300,000 and 79 at 99,000 ions; this one 40, 55, 268 and 64,
 // and one row per atom instead of nine segments takes the pair kernel from 63

@@ -5,9 +5,10 @@
 // from the sorted double4 array (resident in L2) and keeps its partial sums in
 // registers; the L partials are combined with a fixed xor-shuffle tree.
 // Forces are gathered, never scattered: no atomics, deterministic sums.
-// The gathers bound it (54 us at 30,000 water atoms, 355 at 300,000 mixed): a
-// loop of 15 % fewer instructions with one position less in flight ran at 52.5
-// and 414 us.
+// At 300,000 mixed water atoms (355 us) vector issue bounds it, the ALUs 88 %
+// busy; at 30,000 in FP64 (54 us) they are 58 % busy and the gathers' latency
+// counts as much: a loop of 15 % fewer instructions with one position less in
+// flight ran at 414 and 52.5 us.
 //
 // Formulas (FP64; the mixed-precision variant evaluates the pair scalar in FP32):
 //   VERLET plain    ComputeNearForceVerletVirialWorklet, RunWorklet.cpp:2890-2985

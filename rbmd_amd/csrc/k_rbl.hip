@@ -17,13 +17,15 @@
 // atoms.  An atom whose current cell is not its binned one (moved by SHAKE
 // after the binning) takes a stream of its own over its own stencil.
 //
-// Bound by the issue of the FP64 distance tests (1000 to 2000 candidates an
-// atom, of which one in four is kept): sharing the staged candidates among up
-// to 32 atoms, equal shares (a cell's 17 atoms as 5 + 4 + 4 + 4) and one
-// ballot per test hold the rest down.  One wavefront over 64 atoms of a cell,
+// Bound by the chain behind each distance test (1000 to 2000 candidates an
+// atom, of which one in four is kept): the ballots, counts and branches are
+// scalar work in series, and the vector ALUs are busy 29 % of the time (28 % in
+// the energies).  Sharing the staged candidates among up to 32 atoms, equal
+// shares (a cell's 17 atoms as 5 + 4 + 4 + 4) and one ballot per test hold it
+// down.  One wavefront over 64 atoms of a cell,
 // a candidate at a time, took 276 us (4096 salt atoms) and 593 us (30,000
 // water atoms) for the lists, 162 and 1202 us for the energies; this one takes
-// 22 and 149 us, 28 and 275 us.  A stream per wavefront, without the shared
+// 22 and 139 us, 28 and 275 us.  A stream per wavefront, without the shared
 // stage, took 50 and 381 us for the lists.
 #include "cells.hpp"
 #include "dev.hpp"

@@ -476,7 +476,8 @@ static int64_t stencil_blocks_of(const SysView& s, int cfg) {
 // 29.9; water 600 atoms 118 / 46, 1,800 70 / 51, 3,000 57 / 54, 6,000 mixed
 // 77 / 104.
 //
-// Three lines: on the number of candidates; on the atoms, as the list build
+// Three lines: on the number of candidates (or, where cells are crowded, of the
+// atoms: 3,000 of water are a tie, 57 / 54); on the atoms, as the list build
 // has the chip full from about 8,000 on whatever the candidates (steps with
 // lists and with this kernel, us: 8,000 ions 70 / 61 at 1,000 candidates, 75 /
 // 75 at 216; 14,000 81 / 88 at 519, 84 / 106 at 172; 20,000 89 / 124 at 246);
