@@ -1537,6 +1537,7 @@ rbmd_status rbmd_sys_create(rbmd_ctx* ctx, const rbmd_sys_desc* d, const rbmd_pa
     return rc;
   }
   hipStream_t st = ctx->stream;
+  launch_fill_int(v.nbr_num, 0, (v.rbl ? 2 : 1) * n, st);  // a cell beyond its 256 work items leaves atoms unlisted
   launch_fill_int(v.cell_count, 0, ncell_max, st);
   launch_fill_int(v.cursor, 0, ncell_max, st);  // the one-launch scan + scatter counts from zero
   launch_fill_int(v.status, 0, 1, st);

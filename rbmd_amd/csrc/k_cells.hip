@@ -303,19 +303,19 @@ __device__ __forceinline__ void cell_sort_body(const SysView& s, const int bid) 
     s.cursor[c] = 0;
     if (c == 0 && s.list_builds) atomicAdd(s.list_builds, 1);
   }
-  if (cnt > kSortCap) {
-    if (threadIdx.x == 0) atomicOr(s.status, 4);
-    return;
-  }
-  const int nq = (cnt + 3) / 4;
+  // A cell of more is refused by the status flag, but its atoms keep valid
+  // copies, in the scatter's order: later kernels index by rank and type.
+  const bool sorts = cnt <= kSortCap;
+  if (!sorts && threadIdx.x == 0) atomicOr(s.status, 4);
+  const int nq = sorts ? (cnt + 3) / 4 : 0;
   for (int t = threadIdx.x; t < 4 * nq; t += blockDim.x) ids[t] = t < cnt ? s.point_ids[start + t] : 0x7fffffff;
   __syncthreads();
   const int a = c % s.dims[0];
   const int b = (c / s.dims[0]) % s.dims[1];
   const int e = c / (s.dims[0] * s.dims[1]);
   for (int t = threadIdx.x; t < cnt; t += blockDim.x) {
-    const int me = ids[t];
-    int r = 0;  // four ids a read: one a read took 29 us for a cell of 600, this 17
+    const int me = sorts ? ids[t] : s.point_ids[start + t];
+    int r = sorts ? 0 : t;  // four ids a read: one a read took 29 us for a cell of 600, this 17
 #pragma unroll 8
     for (int k = 0; k < nq; ++k) {
       const int4 v = quads[k];
